@@ -298,8 +298,9 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
  *                      recent reads serve the rest from cache.  Every
  *                      variant gives bitwise the same product.  0 .. 7, or
  *                      -1 (default): 7 for a single problem of 2^17 nodes
- *                      or more, 2 for a batch of 2^17 nodes or more, else
- *                      0. */
+ *                      or more, 2 for a batch of 2^17 nodes or more, 3
+ *                      from 98,304 nodes, else 0 (there, untuned, several
+ *                      waves share a row's blocks). */
 /* TG_TUNE_AMG_DEGREE   multigrid: Chebyshev degree of each pre- and
  *                      post-smoothing pass, 2 (default) .. 4. */
 /* TG_TUNE_AMG_WEIGHT   multigrid: weight of the coarse-grid correction in
@@ -307,11 +308,12 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
  *                      aggregation under-corrects; any weight in (0, 2)
  *                      keeps the V-cycle symmetric positive definite). */
 /* TG_TUNE_PCG_FUSED    1: the direction update is formed inside the SpMV
- *                      (four kernels per PCG iteration instead of five, no
- *                      separate direction pass) for the Jacobi and
- *                      multigrid preconditioners, in any SpMV variant;
- *                      0: the five-kernel iteration; -1 (default): 0 for a
- *                      problem or batch of 2^17 nodes or more, else 1. */
+ *                      (one kernel less per PCG iteration, no separate
+ *                      direction pass), in any SpMV variant (block Jacobi:
+ *                      only while no segment has more than 4,096 slices of
+ *                      64 nodes); 0: the direction in its own pass; -1
+ *                      (default): 0 for a problem or batch of more than
+ *                      98,304 nodes, else 1. */
 /* TG_TUNE_STIFF_GATHER 0 (default): the total-Lagrangian stiffness is
  *                      added into the MSR element by element (colour-
  *                      ordered read-modify-write through the slot map);

@@ -27,10 +27,37 @@ namespace tg {
 constexpr int PB = 256;  // threads (= nodes) per block, 4 slices
 constexpr int FB = 1024; // threads of the per-segment finalize blocks
 
+// v of the lane that DPP control CTRL names, for a double
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, true));
+}
+
+// Sum over the wave, the same bits in every lane: lanes 1 and 2 apart by
+// quad permutes, 4 and 8 apart by mirroring 8 and 16 lanes (whose halves
+// each hold one value by then), the rows of 16 and the halves by row swaps.
+// All in the vector registers; a butterfly of __shfl_xor goes through LDS
+// twelve times, about 0.4 us that every kernel of a short iteration pays.
+// All 64 lanes must be active.
 __device__ __forceinline__ double wsum(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    v += dpp<0xB1>(v);    // quad_perm 1,0,3,2
+    v += dpp<0x4E>(v);    // quad_perm 2,3,0,1
+    v += dpp<0x141>(v);   // row_half_mirror
+    v += dpp<0x140>(v);   // row_mirror
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+    {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+        v = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
     return v;
 }
 
@@ -56,44 +83,158 @@ __device__ __forceinline__ void precondition(const double* __restrict__ m, long 
     }
 }
 
-// ---- per-slice partials -> per-segment totals ------------------------------
+// ---- partials -> per-segment totals -----------------------------------------
+//
+// A segment's slices are taken in groups of GS = 4; a group's sum is
+// ((s0 + s1) + s2) + s3 (missing slices 0), lane l of a wave adds groups l,
+// l + 64, ... in order, and the lanes are summed by wsum.  A kernel whose
+// workgroups own a group each writes one partial per group, a kernel with a
+// workgroup per slice one per slice (GROUPED = false: the reader adds four).
+// The order depends only on the segment's own slice count, never on other
+// segments.
+constexpr int GS = 4;
 
-// Sum of part[k][sb..se) by one block of FB threads: thread i adds slices
-// sb+i, sb+i+FB, ... in order, then a fixed tree (waves by butterfly, then
-// the FB/64 wave sums in order).  The order depends only on the segment's
-// own slice count, never on other segments.  The result is in thread 0.
-template <int NV>
-__device__ __forceinline__ void seg_total(const double* part, long nslices, int sb, int se, double (&tot)[NV])
+// lane sums over n partials (groups, or slices) from part[k * stride]; this
+// wave takes every wstep-th run of 64 groups, from run w0
+template <int NV, bool GROUPED>
+__device__ __forceinline__ void lane_sums(const double* part, long stride, int n, int w0, int wstep, double (&x)[NV])
 {
-    __shared__ double red[NV][FB / 64];
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int k = 0; k < NV; k++) x[k] = 0.0;
+    const int per = GROUPED ? 1 : GS;
+#pragma unroll 4
+    for (int base = 64 * per * w0; base < n; base += 64 * per * wstep) {
+        const int s = base + per * l;
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const double* q = part + k * stride + s;
+            if (GROUPED) {
+                x[k] += s < n ? q[0] : 0.0;
+            } else {
+                const double a0 = s < n ? q[0] : 0.0, a1 = s + 1 < n ? q[1] : 0.0;
+                const double a2 = s + 2 < n ? q[2] : 0.0, a3 = s + 3 < n ? q[3] : 0.0;
+                x[k] += ((a0 + a1) + a2) + a3;
+            }
+        }
+    }
+}
+
+// Sum of the partials of a segment of at most FOLD_SLICES slices by one
+// wave, the same in every lane.  Any kernel that needs a total forms it by
+// itself, so an iteration needs no kernel that does only that: at 16^3
+// elements (77 slices) such a kernel took 4 us of a 28 us iteration, twice.
+constexpr int FOLD_SLICES = PCG_FOLD_SLICES;
+template <int NV, bool GROUPED>
+__device__ __forceinline__ void wave_total(const double* part, long stride, int n, double (&tot)[NV])
+{
+    lane_sums<NV, GROUPED>(part, stride, n, 0, 1, tot);
+#pragma unroll
+    for (int k = 0; k < NV; k++) tot[k] = wsum(tot[k]);
+}
+
+// The same total by one block of FB threads: a segment of at most
+// FOLD_SLICES slices exactly as wave_total sums it (by wave 0); a larger one
+// with wave w taking every (FB / 64)-th run and the wave sums added in
+// order.  The result is in thread 0.
+template <int NV, bool GROUPED>
+__device__ __forceinline__ void seg_total(const double* part, long stride, int n, int nsl, double (&tot)[NV])
+{
     const int t = threadIdx.x;
+    if (nsl <= FOLD_SLICES) {
+        if (t < 64) wave_total<NV, GROUPED>(part, stride, n, tot);
+        return;
+    }
+    __shared__ double red[NV][FB / 64];
+    double x[NV];
+    lane_sums<NV, GROUPED>(part, stride, n, t >> 6, FB / 64, x);
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        double x = 0.0;
-        for (int s = sb + t; s < se; s += FB) x += part[k * nslices + s];
-        x = wsum(x);
-        if ((t & 63) == 0) red[k][t >> 6] = x;
+        const double y = wsum(x[k]);
+        if ((t & 63) == 0) red[k][t >> 6] = y;
     }
     __syncthreads();
     if (t == 0)
 #pragma unroll
         for (int k = 0; k < NV; k++) {
-            double x = 0.0;
-            for (int w = 0; w < FB / 64; w++) x += red[k][w];
-            tot[k] = x;
+            double y = 0.0;
+            for (int w = 0; w < FB / 64; w++) y += red[k][w];
+            tot[k] = y;
         }
 }
 
-// x = 0, r = b, p = M^-1 b; per segment rz = b.M^-1 b, bb = b.b
-template <int PC>
-__global__ void __launch_bounds__(PB) k_seg_init(int nnd, const double* __restrict__ b,
-                                                 const double* __restrict__ m, double* __restrict__ x,
-                                                 double* __restrict__ r, double* __restrict__ p,
-                                                 double* __restrict__ part, long nslices)
+// Segment tables as the kernels take them.  grp[i] = (first slice, slices,
+// segment, -) of group i; seg g owns slices [seg_slice[g], seg_slice[g + 1])
+// and groups [seg_grp[g], seg_grp[g + 1]).
+struct SegTab {
+    const int* slice_seg;
+    const int* seg_slice;
+    const int* seg_grp;
+    const int4* grp;
+    int nseg;
+    long nslices;
+    __device__ __forceinline__ int slices(int g) const { return seg_slice[g + 1] - seg_slice[g]; }
+    __device__ __forceinline__ int groups(int g) const { return seg_grp[g + 1] - seg_grp[g]; }
+};
+
+// The group's partials of this workgroup's up to GS waves (PB threads, wave
+// w = slice w of the group), from per-lane values already summed by wsum:
+// thread 0 writes part[k * stride + group].
+template <int NV>
+__device__ __forceinline__ void group_partials(const double (&v)[NV], double* part, long stride, const bool (&on)[NV])
 {
-    const int a = blockIdx.x * PB + threadIdx.x;
-    double v0 = 0.0, v1 = 0.0;
-    if (a < nnd) {
+    __shared__ double red[NV][GS];
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+        if ((t & 63) == 0) red[k][t >> 6] = v[k];
+    __syncthreads();
+    if (t == 0)
+#pragma unroll
+        for (int k = 0; k < NV; k++)
+            if (on[k]) part[k * stride + blockIdx.x] = ((red[k][0] + red[k][1]) + red[k][2]) + red[k][3];
+}
+
+// slots of r.z and the iteration count before (o) and after the iteration
+__device__ __forceinline__ double* slot_rz(double* sc, int o, int nseg, int g) { return sf(sc, o ? S_RZ1 : S_RZ, nseg, g); }
+__device__ __forceinline__ double* slot_it(double* sc, int o, int nseg, int g) { return sf(sc, o ? S_IT1 : S_IT0, nseg, g); }
+
+// End of an iteration of segment g with tot = (r.z, r.r): beta = rz'/rz,
+// stop on ||r||^2 <= rtol^2 ||b||^2 or the iteration cap.  Several waves may
+// form the same decision in one kernel, so the values of the iteration
+// before (slot o) are kept and the new ones go to slot o ^ 1; the owner (one
+// lane per segment) writes.  Returns whether the segment is done.
+__device__ __forceinline__ bool seg_advance(const double (&tot)[2], double* sc, int nseg, int g, int o, bool owner,
+                                            int* ndone, double& beta)
+{
+    const double it = *slot_it(sc, o, nseg, g) + 1.0;
+    beta = tot[0] / *slot_rz(sc, o, nseg, g);
+    const bool done = tot[1] <= *sf(sc, S_THRESH, nseg, g) || it >= *sf(sc, S_MAXIT, nseg, g);
+    if (owner) {
+        *slot_rz(sc, o ^ 1, nseg, g) = tot[0];
+        *slot_it(sc, o ^ 1, nseg, g) = it;
+        *sf(sc, S_ITER, nseg, g) = it;
+        *sf(sc, S_BETA, nseg, g) = beta;
+        *sf(sc, S_RR, nseg, g) = tot[1];
+        if (done) {
+            *sf(sc, S_DONE, nseg, g) = 1.0;
+            atomicAdd(ndone, 1);
+        }
+    }
+    return done;
+}
+
+// x = 0, r = b, z = p = M^-1 b; per segment rz = b.M^-1 b, bb = b.b.  b and z
+// may be one array.
+template <int PC>
+__global__ void __launch_bounds__(PB) k_seg_init(SegTab T, int nnd, const double* b, const double* __restrict__ m,
+                                                 double* __restrict__ x, double* __restrict__ r,
+                                                 double* __restrict__ p, double* z, double* __restrict__ part)
+{
+    const int4 gr = T.grp[blockIdx.x];
+    const int a = 64 * gr.x + threadIdx.x;
+    double v[2] = {0.0, 0.0};
+    if ((int)(threadIdx.x >> 6) < gr.y && a < nnd) {
         double bi[3], zi[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) bi[i] = b[3L * a + i];
@@ -104,34 +245,29 @@ __global__ void __launch_bounds__(PB) k_seg_init(int nnd, const double* __restri
             x[k] = 0.0;
             r[k] = bi[i];
             p[k] = zi[i];
-            v0 += bi[i] * zi[i];
-            v1 += bi[i] * bi[i];
+            if (PC != 2 && z) z[k] = zi[i];
+            v[0] += bi[i] * zi[i];
+            v[1] += bi[i] * bi[i];
         }
     }
-    v0 = wsum(v0);
-    v1 = wsum(v1);
-    if ((threadIdx.x & 63) == 0) {
-        const long s = a >> 6;
-        if (s < nslices) {
-            part[s] = v0;
-            part[nslices + s] = v1;
-        }
-    }
+    v[0] = wsum(v[0]);
+    v[1] = wsum(v[1]);
+    group_partials<2>(v, part, T.nslices, {true, true});
 }
 
-__global__ void __launch_bounds__(FB) k_seg_fin_init(const double* __restrict__ part, long nslices,
-                                                     const int* __restrict__ seg_slice, const int* __restrict__ active,
-                                                     int nseg, double* __restrict__ sc, double rtol, int maxit,
-                                                     int* __restrict__ ndone)
+__global__ void __launch_bounds__(FB) k_seg_fin_init(SegTab T, const double* __restrict__ part,
+                                                     const int* __restrict__ active, double* __restrict__ sc,
+                                                     double rtol, int maxit, int* __restrict__ ndone)
 {
-    const int g = blockIdx.x;
+    const int g = blockIdx.x, nseg = T.nseg;
     double tot[2];
-    seg_total<2>(part, nslices, seg_slice[g], seg_slice[g + 1], tot);
+    seg_total<2, true>(part + T.seg_grp[g], T.nslices, T.groups(g), T.slices(g), tot);
     if (threadIdx.x == 0) {
         *sf(sc, S_RZ, nseg, g) = tot[0];
         *sf(sc, S_BB, nseg, g) = tot[1];
         *sf(sc, S_RR, nseg, g) = tot[1];
         *sf(sc, S_ITER, nseg, g) = 0.0;
+        *sf(sc, S_IT0, nseg, g) = 0.0;
         *sf(sc, S_BETA, nseg, g) = 0.0;  // the fused iteration forms p_0 = z_0 + 0 p
         *sf(sc, S_THRESH, nseg, g) = rtol * rtol * tot[1];
         *sf(sc, S_MAXIT, nseg, g) = (double)maxit;
@@ -182,164 +318,213 @@ __device__ __forceinline__ void block_values(const MT* __restrict__ bval, const 
     v[7] = tr ? u[5] : u[7];
 }
 
+// A row's sum over its blocks k = 0 .. w-1 is formed in groups of RG
+// consecutive slots: each group from zero in slot order, the groups added in
+// order.  So one lane can sum a whole row, or the waves of a workgroup can
+// take a group each, with the same rounding.  Nine groups of three are the
+// 27 blocks of an interior node of a hexahedral mesh.
+constexpr int RG = 3;
+
+// y += A_blk x for one slot of a row
+__device__ __forceinline__ void block_mac(const double (&v)[9], double x0, double x1, double x2, double (&y)[3])
+{
+    y[0] += v[0] * x0 + v[1] * x1 + v[2] * x2;
+    y[1] += v[3] * x0 + v[4] * x1 + v[5] * x2;
+    y[2] += v[6] * x0 + v[7] * x1 + v[8] * x2;
+}
+
+// One lane's row sum: x(c, x0, x1, x2) gives the vector at node c.  UNR:
+// padding slots (column -1) hold zero values: they multiply the row's own x,
+// which keeps the loop branch-free so its loads can be issued ahead; adding
+// the zero products leaves the sums unchanged.
+template <class MT, bool UNR, bool SYM, class X>
+__device__ __forceinline__ void row_sum(const int* __restrict__ bcol, const MT* __restrict__ bval,
+                                        const int* __restrict__ tpos, long b0, int w, int l, int a, X x,
+                                        double (&y)[3])
+{
+    y[0] = y[1] = y[2] = 0.0;
+    int k = 0;
+    for (; k + RG <= w; k += RG) {
+        double g[3] = {0.0, 0.0, 0.0};
+#pragma unroll(UNR ? RG : 1)
+        for (int i = 0; i < RG; i++) {
+            const long blk = b0 + k + i;
+            const int cr = bcol[blk * 64 + l];
+            if (!UNR && cr < 0) continue;
+            const int c = cr < 0 ? a : cr;
+            double x0, x1, x2, v[9];
+            x(c, x0, x1, x2);
+            block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
+            block_mac(v, x0, x1, x2, g);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) y[i] += g[i];
+    }
+    if (k < w) {
+        double g[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+        for (; k < w; k++) {
+            const long blk = b0 + k;
+            const int cr = bcol[blk * 64 + l];
+            if (!UNR && cr < 0) continue;
+            const int c = cr < 0 ? a : cr;
+            double x0, x1, x2, v[9];
+            x(c, x0, x1, x2);
+            block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
+            block_mac(v, x0, x1, x2, g);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) y[i] += g[i];
+    }
+}
+
 // q = A p on the block operator, with per-slice partials of p.q.  MT is the
 // storage type of the operator values (double, or float in mixed
 // precision); products and sums are FP64.
 template <class MT, bool XCD, bool UNR, bool SYM>
-__global__ void __launch_bounds__(PB) k_seg_spmv(int nnd, const int* __restrict__ slice_seg,
+__global__ void __launch_bounds__(PB) k_seg_spmv(SegTab T, int nnd,
                                                  const int* __restrict__ sbase, const int* __restrict__ swidth,
                                                  const int* __restrict__ bcol, const MT* __restrict__ bval,
                                                  const int* __restrict__ tpos, const double* __restrict__ x,
-                                                 double* __restrict__ y,
-                                                 double* __restrict__ part, long nslices, int nseg,
+                                                 double* __restrict__ y, double* __restrict__ ppq,
                                                  const double* __restrict__ sc)
 {
     const int a = row_block<XCD>() * PB + threadIdx.x;
-    const int s = a >> 6, l = a & 63;
-    if (a >= 64L * nslices) return;
-    const int g = slice_seg[s];  // wave-uniform
-    if (*sf((double*)sc, S_DONE, nseg, g) != 0.0) return;
+    const int s = __builtin_amdgcn_readfirstlane(a >> 6), l = a & 63;
+    if (s >= T.nslices) return;
+    const int g = T.slice_seg[s];
+    if (*sf((double*)sc, S_DONE, T.nseg, g) != 0.0) return;
     double dv = 0.0;
     if (a < nnd) {
-        const long b0 = sbase[s];
-        const int w = swidth[s];
-        double y0 = 0, y1 = 0, y2 = 0;
-        if (UNR) {
-            // padding slots (column -1) hold zero values: they multiply the
-            // row's own x, which keeps the loop branch-free so its loads can
-            // be issued ahead; adding the zero products leaves the sums
-            // unchanged
-#pragma unroll 3
-            for (int k = 0; k < w; k++) {
-                const long blk = b0 + k;
-                const int cr = bcol[blk * 64 + l];
-                const int c = cr < 0 ? a : cr;
-                const double x0 = x[3L * c], x1 = x[3L * c + 1], x2 = x[3L * c + 2];
-                double v[9];
-                block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
-                y0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-                y1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-                y2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
-            }
-        } else {
-            for (int k = 0; k < w; k++) {
-                const long blk = b0 + k;
-                const int c = bcol[blk * 64 + l];
-                if (c < 0) continue;
-                const double x0 = x[3L * c], x1 = x[3L * c + 1], x2 = x[3L * c + 2];
-                double v[9];
-                block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
-                y0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-                y1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-                y2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
-            }
-        }
-        y[3L * a] = y0;
-        y[3L * a + 1] = y1;
-        y[3L * a + 2] = y2;
-        dv = y0 * x[3L * a] + y1 * x[3L * a + 1] + y2 * x[3L * a + 2];
+        double yi[3];
+        row_sum<MT, UNR, SYM>(bcol, bval, tpos, sbase[s], swidth[s], l, a, [&](int c, double& x0, double& x1, double& x2) {
+            x0 = x[3L * c];
+            x1 = x[3L * c + 1];
+            x2 = x[3L * c + 2];
+        }, yi);
+        y[3L * a] = yi[0];
+        y[3L * a + 1] = yi[1];
+        y[3L * a + 2] = yi[2];
+        dv = yi[0] * x[3L * a] + yi[1] * x[3L * a + 1] + yi[2] * x[3L * a + 2];
     }
     dv = wsum(dv);
-    if (l == 0) part[s] = dv;
+    if (l == 0) ppq[s] = dv;
 }
 
-__global__ void __launch_bounds__(FB) k_seg_fin_alpha(const double* __restrict__ part, long nslices,
-                                                      const int* __restrict__ seg_slice, int nseg,
+__global__ void __launch_bounds__(FB) k_seg_fin_alpha(SegTab T, const double* __restrict__ ppq, int o,
                                                       double* __restrict__ sc)
 {
     const int g = blockIdx.x;
-    if (*sf(sc, S_DONE, nseg, g) != 0.0) return;
+    if (*sf(sc, S_DONE, T.nseg, g) != 0.0) return;
     double tot[1];
-    seg_total<1>(part, nslices, seg_slice[g], seg_slice[g + 1], tot);
-    if (threadIdx.x == 0) {
-        *sf(sc, S_PQ, nseg, g) = tot[0];
-        *sf(sc, S_ALPHA, nseg, g) = *sf(sc, S_RZ, nseg, g) / tot[0];
-    }
+    seg_total<1, false>(ppq + T.seg_slice[g], 0, T.slices(g), T.slices(g), tot);
+    if (threadIdx.x == 0) *sf(sc, S_ALPHA, T.nseg, g) = *slot_rz(sc, o, T.nseg, g) / tot[0];
 }
 
-// x += alpha p, r -= alpha q; per-slice partials of r.M^-1 r and r.r (with
-// the multigrid, r.r only: r.z follows the V-cycle)
-template <int PC>
-__global__ void __launch_bounds__(PB) k_seg_update(int nnd, const int* __restrict__ slice_seg,
-                                                   const double* __restrict__ p, const double* __restrict__ q,
-                                                   const double* __restrict__ m, double* __restrict__ x,
-                                                   double* __restrict__ r, double* __restrict__ part, long nslices,
-                                                   int nseg, const double* __restrict__ sc)
+// x += alpha p, r -= alpha q; partials of r.M^-1 r and r.r (with the
+// multigrid, r.r only: r.z follows the V-cycle).  One workgroup per group.
+// FOLD: alpha = r.z / p.q from the slice partials of p.q, else from its
+// scalar slot.  With z given, M^-1 r is kept for the direction.
+template <int PC, bool FOLD>
+__global__ void __launch_bounds__(PB) k_seg_update(SegTab T, int nnd, const double* __restrict__ p,
+                                                   const double* __restrict__ q, const double* __restrict__ m,
+                                                   double* __restrict__ x, double* __restrict__ r,
+                                                   double* __restrict__ z, const double* __restrict__ ppq,
+                                                   double* __restrict__ part, int o, double* sc)
 {
-    const int a = blockIdx.x * PB + threadIdx.x;
-    const int s = a >> 6;
-    if (a >= 64L * nslices) return;
-    const int g = slice_seg[s];
-    if (*sf((double*)sc, S_DONE, nseg, g) != 0.0) return;
-    const double alpha = *sf((double*)sc, S_ALPHA, nseg, g);
-    double v0 = 0.0, v1 = 0.0;
-    if (a < nnd) {
-        double ri[3], zi[3];
+    const int4 gr = T.grp[blockIdx.x];
+    const int g = gr.z, nseg = T.nseg;
+    if (*sf(sc, S_DONE, nseg, g) != 0.0) return;
+    // the vectors first: their loads are in flight while the total is formed
+    const int a = 64 * gr.x + threadIdx.x;
+    const bool own = (int)(threadIdx.x >> 6) < gr.y && a < nnd;
+    double xi[3], ri[3], pi[3], qi[3], mi[PC == 1 ? 9 : 3];
+    const long k0 = own ? 3L * a : 0;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        pi[i] = p[k0 + i];
+        qi[i] = q[k0 + i];
+        ri[i] = r[k0 + i];
+        xi[i] = x[k0 + i];
+    }
+    if (PC != 2)
+#pragma unroll
+        for (int i = 0; i < (PC == 1 ? 9 : 3); i++) mi[i] = m[(PC == 1 ? 3 : 1) * k0 + i];
+    double alpha;
+    if (FOLD) {
+        double tot[1];
+        wave_total<1, false>(ppq + T.seg_slice[g], 0, T.slices(g), tot);
+        alpha = *slot_rz(sc, o, nseg, g) / tot[0];
+    } else {
+        alpha = *sf(sc, S_ALPHA, nseg, g);
+    }
+    double v[2] = {0.0, 0.0};
+    if (own) {
+        double zi[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            const long k = 3L * a + i;
-            x[k] += alpha * p[k];
-            ri[i] = r[k] - alpha * q[k];
-            r[k] = ri[i];
+            x[k0 + i] = xi[i] + alpha * pi[i];
+            ri[i] = ri[i] - alpha * qi[i];
+            r[k0 + i] = ri[i];
         }
-        if (PC != 2) precondition<PC>(m, a, ri, zi);
+        if (PC != 2) precondition<PC>(mi, 0, ri, zi);
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            if (PC != 2) v0 += ri[i] * zi[i];
-            v1 += ri[i] * ri[i];
+            if (PC != 2) v[0] += ri[i] * zi[i];
+            v[1] += ri[i] * ri[i];
         }
+        if (PC != 2 && z)
+#pragma unroll
+            for (int i = 0; i < 3; i++) z[k0 + i] = zi[i];
     }
-    v0 = wsum(v0);
-    v1 = wsum(v1);
-    if ((a & 63) == 0) {
-        if (PC != 2) part[s] = v0;
-        part[nslices + s] = v1;
-    }
+    if (PC != 2) v[0] = wsum(v[0]);
+    v[1] = wsum(v[1]);
+    group_partials<2>(v, part, T.nslices, {PC != 2, true});
 }
 
-// beta = rz'/rz; stop on ||r||^2 <= rtol^2 ||b||^2 or the iteration cap
-__global__ void __launch_bounds__(FB) k_seg_fin_beta(const double* __restrict__ part, long nslices,
-                                                     const int* __restrict__ seg_slice, int nseg,
+// the end of an iteration, one workgroup per segment
+__global__ void __launch_bounds__(FB) k_seg_fin_beta(SegTab T, const double* __restrict__ part, int o,
                                                      double* __restrict__ sc, int* __restrict__ ndone)
 {
     const int g = blockIdx.x;
-    if (*sf(sc, S_DONE, nseg, g) != 0.0) return;
-    double tot[2];
-    seg_total<2>(part, nslices, seg_slice[g], seg_slice[g + 1], tot);
-    if (threadIdx.x == 0) {
-        const double it = *sf(sc, S_ITER, nseg, g) + 1.0;
-        *sf(sc, S_ITER, nseg, g) = it;
-        *sf(sc, S_BETA, nseg, g) = tot[0] / *sf(sc, S_RZ, nseg, g);
-        *sf(sc, S_RZ, nseg, g) = tot[0];
-        *sf(sc, S_RR, nseg, g) = tot[1];
-        if (tot[1] <= *sf(sc, S_THRESH, nseg, g) || it >= *sf(sc, S_MAXIT, nseg, g)) {
-            *sf(sc, S_DONE, nseg, g) = 1.0;
-            atomicAdd(ndone, 1);
-        }
-    }
+    if (*sf(sc, S_DONE, T.nseg, g) != 0.0) return;
+    double tot[2], beta;
+    seg_total<2, true>(part + T.seg_grp[g], T.nslices, T.groups(g), T.slices(g), tot);
+    if (threadIdx.x == 0) seg_advance(tot, sc, T.nseg, g, o, true, ndone, beta);
 }
 
-// p = M^-1 r + beta p
-template <int PC>
-__global__ void __launch_bounds__(PB) k_seg_direction(int nnd, const int* __restrict__ slice_seg,
-                                                      const double* __restrict__ r, const double* __restrict__ m,
-                                                      double* __restrict__ p, long nslices, int nseg,
-                                                      const double* __restrict__ sc)
+// p = M^-1 r + beta p.  FOLD: the end of the iteration (beta, the stopping
+// test) from the partials, else beta from its scalar slot.  PC = 2: m holds
+// M^-1 r itself.
+template <int PC, bool FOLD>
+__global__ void __launch_bounds__(PB) k_seg_direction(SegTab T, int nnd, const double* __restrict__ r,
+                                                      const double* __restrict__ m, double* __restrict__ p,
+                                                      const double* __restrict__ part, int o, double* sc, int* ndone)
 {
-    const int a = blockIdx.x * PB + threadIdx.x;
-    if (a >= nnd) return;
-    const int g = slice_seg[a >> 6];
-    if (*sf((double*)sc, S_DONE, nseg, g) != 0.0) return;
-    const double beta = *sf((double*)sc, S_BETA, nseg, g);
-    double ri[3], zi[3];
-#pragma unroll
-    for (int i = 0; i < 3; i++) ri[i] = r[3L * a + i];
-    precondition<PC>(m, a, ri, zi);
+    const int4 gr = T.grp[blockIdx.x];
+    const int g = gr.z, nseg = T.nseg;
+    if (*sf(sc, S_DONE, nseg, g) != 0.0) return;
+    const int a = 64 * gr.x + threadIdx.x;
+    const bool own = (int)(threadIdx.x >> 6) < gr.y && a < nnd;
+    const long k0 = own ? 3L * a : 0;
+    double ri[3], pi[3], zi[3];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const long k = 3L * a + i;
-        p[k] = zi[i] + beta * p[k];
+        ri[i] = PC == 2 ? 0.0 : r[k0 + i];
+        pi[i] = p[k0 + i];
     }
+    precondition<PC>(m, k0 / 3, ri, zi);
+    double beta;
+    if (FOLD) {
+        double tot[2];
+        wave_total<2, true>(part + T.seg_grp[g], T.nslices, T.groups(g), tot);
+        if (seg_advance(tot, sc, nseg, g, o, gr.x == T.seg_slice[g] && threadIdx.x == 0, ndone, beta)) return;
+    } else {
+        beta = *sf(sc, S_BETA, nseg, g);
+    }
+    if (!own) return;
+#pragma unroll
+    for (int i = 0; i < 3; i++) p[k0 + i] = zi[i] + beta * pi[i];
 }
 
 // ---- persistent iteration: one workgroup per small segment ----------------
@@ -348,43 +533,31 @@ __global__ void __launch_bounds__(PB) k_seg_direction(int nnd, const int* __rest
 // whole CG loop inside one workgroup of PW threads, thread t owning node
 // 64 sb + t: its x and r stay in registers, the direction p in LDS
 // (the SpMV gathers neighbours from there), the per-slice partials and the
-// segment scalars in LDS and in thread 0's registers; only the operator is
-// read from memory (L2) each iteration, and no kernel is launched per
-// iteration.  The arithmetic is the five-kernel iteration's, in the same
-// order: the row sums of k_seg_spmv (its unrolled form, padding slots
-// multiplying zeros), the updates of k_seg_update and k_seg_direction, and
-// each per-segment total summed as seg_total sums it with FB threads (here
-// FB = PW: thread t holds slice sb + t's partial).  So the iterates are
+// segment scalars in registers; only the operator is read from memory (L2)
+// each iteration, and no kernel is launched per iteration.  The arithmetic
+// is the kernel-per-step iteration's, in the same order: the row sums of
+// row_sum, the updates of k_seg_update and k_seg_direction, and each
+// per-segment total summed as wave_total sums it, by every wave for itself
+// from the partials in LDS (one barrier per total).  So the iterates are
 // bitwise those of the kernel-per-step iteration.  The loop ends on the
-// segment's own stopping test or iteration cap, as k_seg_fin_beta decides;
-// the final x, r, p and scalars are written back as that iteration leaves
-// them.
+// segment's own stopping test or iteration cap, as seg_advance decides; the
+// final x, r, p and scalars are written back as that iteration leaves them.
 constexpr int PW = FB;
 constexpr int PERSIST_MAX = PW / 64;
 static_assert(PERSIST_MAX == PCG_PERSIST_MAX, "the host's threshold cap is the kernel's slice capacity");
 
-// per-segment totals of NV partials held by threads 0..nsl-1 in lp[k][t],
-// summed in seg_total's order
+// per-segment totals of the NV x nsl partials lp, in every lane, in
+// wave_total's order (nsl <= 16: lanes 0..3 hold four each)
 template <int NV>
-__device__ __forceinline__ void seg_total_lds(const double (&lp)[2][PERSIST_MAX], int nsl, double (&red)[2][PW / 64],
-                                              double (&tot)[NV])
+__device__ __forceinline__ void wave_total_lds(const double (&lp)[2][PERSIST_MAX], int nsl, double (&tot)[NV])
 {
-    const int t = threadIdx.x;
+    const int s = 4 * (threadIdx.x & 63);
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        double x = 0.0;
-        if (t < nsl) x += lp[k][t];
-        x = wsum(x);
-        if ((t & 63) == 0) red[k][t >> 6] = x;
+        const double a0 = s < nsl ? lp[k][s] : 0.0, a1 = s + 1 < nsl ? lp[k][s + 1] : 0.0;
+        const double a2 = s + 2 < nsl ? lp[k][s + 2] : 0.0, a3 = s + 3 < nsl ? lp[k][s + 3] : 0.0;
+        tot[k] = wsum(0.0 + (((a0 + a1) + a2) + a3));
     }
-    __syncthreads();
-    if (t == 0)
-#pragma unroll
-        for (int k = 0; k < NV; k++) {
-            double x = 0.0;
-            for (int w = 0; w < PW / 64; w++) x += red[k][w];
-            tot[k] = x;
-        }
 }
 
 template <class MT, int PC>
@@ -397,10 +570,7 @@ __global__ void __launch_bounds__(PW) k_pcg_persistent(const int* __restrict__ s
                                                        double* __restrict__ sc, int* __restrict__ ndone)
 {
     __shared__ double sp[PW][3];
-    __shared__ double lp[2][PERSIST_MAX];
-    __shared__ double red[2][PW / 64];
-    __shared__ double bc[2];
-    __shared__ int bdone;
+    __shared__ double lpq[2][PERSIST_MAX], lrz[2][PERSIST_MAX];
     const int g = segs[blockIdx.x];
     const int sb = seg_slice[g], nsl = seg_slice[g + 1] - sb;
     const int t = threadIdx.x, l = t & 63;
@@ -408,16 +578,9 @@ __global__ void __launch_bounds__(PW) k_pcg_persistent(const int* __restrict__ s
     const int base = 64 * sb;             // first node of the segment
     const int a = base + t;               // this thread's node
     const bool own = (t >> 6) < nsl && a < nnd;
-    // thread 0: the segment's scalars
-    double rz = 0.0, thresh = 0.0, maxit = 0.0, iter = 0.0, beta = 0.0, pq = 0.0, alpha = 0.0, rr = 0.0;
-    if (t == 0) {
-        bdone = *sf(sc, S_DONE, nseg, g) != 0.0;
-        rz = *sf(sc, S_RZ, nseg, g);
-        thresh = *sf(sc, S_THRESH, nseg, g);
-        maxit = *sf(sc, S_MAXIT, nseg, g);
-        iter = *sf(sc, S_ITER, nseg, g);
-        rr = *sf(sc, S_RR, nseg, g);
-    }
+    if (*sf(sc, S_DONE, nseg, g) != 0.0) return;
+    double rz = *sf(sc, S_RZ, nseg, g), rr = 0.0, iter = 0.0;
+    const double thresh = *sf(sc, S_THRESH, nseg, g), maxit = *sf(sc, S_MAXIT, nseg, g);
     double xi[3] = {0, 0, 0}, ri[3] = {0, 0, 0}, zi[3] = {0, 0, 0}, pi[3] = {0, 0, 0};
 #pragma unroll
     for (int i = 0; i < 3; i++) {
@@ -429,48 +592,27 @@ __global__ void __launch_bounds__(PW) k_pcg_persistent(const int* __restrict__ s
         sp[t][i] = pi[i];
     }
     __syncthreads();
-    if (bdone) return;
     for (;;) {
-        // q = A p and the slice partial of p.q (k_seg_spmv, unrolled form)
+        // q = A p and the slice partial of p.q
         double qi[3] = {0, 0, 0};
         {
             double dv = 0.0;
             if (own) {
-                const long b0 = sbase[s];
-                const int wd = swidth[s];
-                double y0 = 0, y1 = 0, y2 = 0;
-#pragma unroll 3
-                for (int k = 0; k < wd; k++) {
-                    const long blk = b0 + k;
-                    const int cr = bcol[blk * 64 + l];
-                    const int c = (cr < 0 ? a : cr) - base;
-                    const double x0 = sp[c][0], x1 = sp[c][1], x2 = sp[c][2];
-                    double v[9];
-                    block_values<MT, false>(bval, nullptr, blk, l, false, v);
-                    y0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-                    y1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-                    y2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
-                }
-                qi[0] = y0;
-                qi[1] = y1;
-                qi[2] = y2;
-                dv = y0 * pi[0] + y1 * pi[1] + y2 * pi[2];
+                row_sum<MT, true, false>(bcol, bval, nullptr, sbase[s], swidth[s], l, a,
+                                         [&](int c, double& x0, double& x1, double& x2) {
+                                             x0 = sp[c - base][0];
+                                             x1 = sp[c - base][1];
+                                             x2 = sp[c - base][2];
+                                         }, qi);
+                dv = qi[0] * pi[0] + qi[1] * pi[1] + qi[2] * pi[2];
             }
             dv = wsum(dv);
-            if (l == 0 && (t >> 6) < nsl) lp[0][t >> 6] = dv;
+            if (l == 0 && (t >> 6) < nsl) lpq[0][t >> 6] = dv;
         }
         __syncthreads();
-        {
-            double tot[1];
-            seg_total_lds<1>(lp, nsl, red, tot);
-            if (t == 0) {
-                pq = tot[0];
-                alpha = rz / tot[0];  // k_seg_fin_alpha
-                bc[0] = alpha;
-            }
-        }
-        __syncthreads();
-        const double al = bc[0];
+        double pq[1];
+        wave_total_lds<1>(lpq, nsl, pq);
+        const double al = rz / pq[0];
         // x += alpha p, r -= alpha q, z = M^-1 r; slice partials of r.z, r.r (k_seg_update)
         {
             double v0 = 0.0, v1 = 0.0;
@@ -490,38 +632,27 @@ __global__ void __launch_bounds__(PW) k_pcg_persistent(const int* __restrict__ s
             v0 = wsum(v0);
             v1 = wsum(v1);
             if (l == 0 && (t >> 6) < nsl) {
-                lp[0][t >> 6] = v0;
-                lp[1][t >> 6] = v1;
+                lrz[0][t >> 6] = v0;
+                lrz[1][t >> 6] = v1;
             }
         }
         __syncthreads();
-        {
-            double tot[2];
-            seg_total_lds<2>(lp, nsl, red, tot);
-            if (t == 0) {
-                // k_seg_fin_beta
-                iter = iter + 1.0;
-                beta = tot[0] / rz;
-                rz = tot[0];
-                rr = tot[1];
-                bc[1] = beta;
-                bdone = tot[1] <= thresh || iter >= maxit;
-            }
-        }
-        __syncthreads();
-        if (bdone) break;
-        const double be = bc[1];
-        // p = M^-1 r + beta p, with z formed again here as k_seg_direction
-        // forms it (the same expression, so the same contraction into FMAs)
-        if (own) {
-            double zd[3];
-            precondition<PC>(m, a, ri, zd);
+        // the end of the iteration (seg_advance), the same in every lane
+        double tot[2];
+        wave_total_lds<2>(lrz, nsl, tot);
+        iter = iter + 1.0;
+        const double be = tot[0] / rz;
+        rz = tot[0];
+        rr = tot[1];
+        if (tot[1] <= thresh || iter >= maxit) break;
+        // p = M^-1 r + beta p (every wave is past this iteration's reads of
+        // sp: they came before the first barrier)
+        if (own)
 #pragma unroll
             for (int i = 0; i < 3; i++) {
-                pi[i] = zd[i] + be * pi[i];
+                pi[i] = zi[i] + be * pi[i];
                 sp[t][i] = pi[i];
             }
-        }
         __syncthreads();
     }
     if (own)
@@ -533,9 +664,6 @@ __global__ void __launch_bounds__(PW) k_pcg_persistent(const int* __restrict__ s
         }
     if (t == 0) {
         *sf(sc, S_ITER, nseg, g) = iter;
-        *sf(sc, S_PQ, nseg, g) = pq;
-        *sf(sc, S_ALPHA, nseg, g) = alpha;
-        *sf(sc, S_BETA, nseg, g) = beta;
         *sf(sc, S_RZ, nseg, g) = rz;
         *sf(sc, S_RR, nseg, g) = rr;
         *sf(sc, S_DONE, nseg, g) = 1.0;
@@ -543,96 +671,207 @@ __global__ void __launch_bounds__(PW) k_pcg_persistent(const int* __restrict__ s
     }
 }
 
-// ---- fused iteration: four kernels per PCG iteration -----------------------
+// ---- fused iteration: the direction formed inside the SpMV ------------------
 //
 // The direction update p = z + beta p_old is formed inside the SpMV -- for
 // the SpMV's own rows, which it stores, and for every neighbour it gathers --
 // so the separate direction pass (and its reads of r, z and p) disappears;
 // p is double-buffered (the SpMV reads p_old of its neighbours while it
-// writes p of its own rows).  The per-segment reductions stay in their own
-// finalize kernels: a kernel boundary publishes every workgroup's partials
-// at no cost, where a device-scope fence per wave would write back and
-// invalidate the XCD's L2 each time.
+// writes p of its own rows).  With the totals folded into the kernels that
+// need them, an iteration is two kernels: this one, which first closes the
+// iteration before (beta, the stopping test: seg_advance) from the update's
+// partials, and the update, which forms alpha from this one's.  A device-
+// scope fence per wave instead (one kernel per iteration) would write back
+// and invalidate the XCD's L2 each time.
 
-// z at dof k: Jacobi (m = 1/diag) or multigrid (m = z)
+// z at dof k: Jacobi (m = 1/diag) or kept by the update / the multigrid (m = z)
 template <int PC>
 __device__ __forceinline__ double zval(const double* __restrict__ m, const double* __restrict__ r, long k)
 {
     return PC == 2 ? m[k] : m[k] * r[k];
 }
 
+// beta of segment g for the SpMV of slice s, closing the iteration before
+// when `close`; returns whether the segment is done
+__device__ __forceinline__ bool direction_beta(const SegTab& T, const double* part, int g, int s, bool owner_lane,
+                                               bool close, int o, double* sc, int* ndone, double& beta)
+{
+    if (!close) {
+        beta = *sf(sc, S_BETA, T.nseg, g);
+        return false;
+    }
+    double tot[2];
+    wave_total<2, true>(part + T.seg_grp[g], T.nslices, T.groups(g), tot);
+    return seg_advance(tot, sc, T.nseg, g, o, s == T.seg_slice[g] && owner_lane, ndone, beta);
+}
+
 template <class MT, int PC, bool XCD, bool UNR, bool SYM>
-__global__ void __launch_bounds__(PB) k_fused_spmv(int nnd, const int* __restrict__ slice_seg,
+__global__ void __launch_bounds__(PB) k_fused_spmv(SegTab T, int nnd,
                                                    const int* __restrict__ sbase, const int* __restrict__ swidth,
                                                    const int* __restrict__ bcol, const MT* __restrict__ bval,
                                                    const int* __restrict__ tpos,
                                                    const double* __restrict__ m, const double* __restrict__ r,
                                                    const double* __restrict__ pold, double* __restrict__ pnew,
-                                                   double* __restrict__ y, double* __restrict__ part, long nslices,
-                                                   int nseg, const double* __restrict__ sc)
+                                                   double* __restrict__ y, const double* __restrict__ part,
+                                                   double* __restrict__ ppq, int close, int o, double* sc, int* ndone)
 {
     const int a = row_block<XCD>() * PB + threadIdx.x;
-    const int s = a >> 6, l = a & 63;
-    if (a >= 64L * nslices) return;
-    const int g = slice_seg[s];  // wave-uniform
-    if (*sf((double*)sc, S_DONE, nseg, g) != 0.0) return;
-    const double beta = *sf((double*)sc, S_BETA, nseg, g);
+    const int s = __builtin_amdgcn_readfirstlane(a >> 6), l = a & 63;
+    if (s >= T.nslices) return;
+    const int g = T.slice_seg[s];
+    if (*sf(sc, S_DONE, T.nseg, g) != 0.0) return;
+    double beta;
+    if (direction_beta(T, part, g, s, l == 0, close, o, sc, ndone, beta)) return;
     double dv = 0.0;
     if (a < nnd) {
-        const long b0 = sbase[s];
-        const int w = swidth[s];
-        double y0 = 0, y1 = 0, y2 = 0;
-        // UNR: padding slots (column -1, zero values) multiply the row's own
-        // direction, as in k_seg_spmv
-#pragma unroll(UNR ? 3 : 1)
-        for (int k = 0; k < w; k++) {
-            const long blk = b0 + k;
-            const int cr = bcol[blk * 64 + l];
-            if (!UNR && cr < 0) continue;
-            const int c = cr < 0 ? a : cr;
-            const double x0 = zval<PC>(m, r, 3L * c) + beta * pold[3L * c];
-            const double x1 = zval<PC>(m, r, 3L * c + 1) + beta * pold[3L * c + 1];
-            const double x2 = zval<PC>(m, r, 3L * c + 2) + beta * pold[3L * c + 2];
-            double v[9];
-            block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
-            y0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-            y1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-            y2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
-        }
-        double p3[3];
+        double yi[3], p3[3];
+        row_sum<MT, UNR, SYM>(bcol, bval, tpos, sbase[s], swidth[s], l, a, [&](int c, double& x0, double& x1, double& x2) {
+            x0 = zval<PC>(m, r, 3L * c) + beta * pold[3L * c];
+            x1 = zval<PC>(m, r, 3L * c + 1) + beta * pold[3L * c + 1];
+            x2 = zval<PC>(m, r, 3L * c + 2) + beta * pold[3L * c + 2];
+        }, yi);
 #pragma unroll
         for (int i = 0; i < 3; i++) {
             p3[i] = zval<PC>(m, r, 3L * a + i) + beta * pold[3L * a + i];
             pnew[3L * a + i] = p3[i];
+            y[3L * a + i] = yi[i];
         }
-        y[3L * a] = y0;
-        y[3L * a + 1] = y1;
-        y[3L * a + 2] = y2;
-        dv = y0 * p3[0] + y1 * p3[1] + y2 * p3[2];
+        dv = yi[0] * p3[0] + yi[1] * p3[1] + yi[2] * p3[2];
     }
     dv = wsum(dv);
-    if (l == 0) part[s] = dv;
+    if (l == 0) ppq[s] = dv;
 }
 
-// per-segment dot product a.b into out[seg]
-__global__ void __launch_bounds__(PB) k_seg_dot(int nnd, const double* __restrict__ x, const double* __restrict__ y,
-                                                double* __restrict__ part, long nslices)
+// The fused SpMV with a row's groups of slots dealt to the NW waves of a
+// workgroup, one workgroup per slice: at a few hundred slices a lane that
+// walks 27 blocks by itself is a chain of dependent loads on a nearly idle
+// chip (FP64, 77 slices: 17.2 us a launch with a lane per row, 6.3 with nine
+// waves; 363 slices: 23.1 and 12.5 with five, where the 48 MB operator comes
+// from the last-level cache at 3.8 TB/s).  z holds M^-1 r.  Wave 0 closes the iteration before while the other
+// waves' first loads are in flight; the group sums meet in LDS and wave 0
+// adds them in order, so the product is bitwise k_fused_spmv's.  Each XCD
+// takes a contiguous range of slices (row_block), so the gathered vectors
+// stay in its L2 (1,077 slices, FP32: 27.7 us per iteration in launch order,
+// 25.4 so).
+// PRE: the gathers, too, are issued before beta is known (more registers).
+template <class MT, int NW, bool PRE>
+__global__ void __launch_bounds__(64 * NW) k_split_spmv(SegTab T, int nnd,
+                                                        const int* __restrict__ sbase, const int* __restrict__ swidth,
+                                                        const int* __restrict__ bcol, const MT* __restrict__ bval,
+                                                        const double* __restrict__ z, const double* __restrict__ pold,
+                                                        double* __restrict__ pnew, double* __restrict__ y,
+                                                        const double* __restrict__ part, double* __restrict__ ppq,
+                                                        int close, int o, double* sc, int* ndone)
 {
-    const int a = blockIdx.x * PB + threadIdx.x;
-    double v = 0.0;
-    if (a < nnd)
+    __shared__ double red[NW][3][64];
+    __shared__ double sbeta;
+    __shared__ int sdone;
+    const int s = row_block<true>(), l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (s >= T.nslices) return;
+    const int a = 64 * s + l;
+    const int g = T.slice_seg[s];
+    const long b0 = sbase[s];
+    const int w = swidth[s];
+    // the owner may set the flag while this kernel runs: a wave that sees it
+    // skips its loads, and wave 0 comes to the same decision for them all
+    const bool was_done = *sf(sc, S_DONE, T.nseg, g) != 0.0;
+    const bool own = a < nnd;
+    int c[RG];
+    MT v[RG][9];
+    double zc[PRE ? RG : 1][3], pc[PRE ? RG : 1][3];
+    // slots k0 .. k0 + RG - 1, k0 < w; past the row's last slot that slot
+    // again (not used), so no branch stands around a load
+    auto load_group = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < 3; i++) v += x[3L * a + i] * y[3L * a + i];
-    v = wsum(v);
-    if ((threadIdx.x & 63) == 0 && (a >> 6) < nslices) part[a >> 6] = v;
+        for (int i = 0; i < RG; i++) {
+            const long blk = b0 + min(k0 + i, w - 1);
+            const int cr = bcol[blk * 64 + l];
+            c[i] = own && cr >= 0 ? cr : (own ? a : 0);
+#pragma unroll
+            for (int m = 0; m < 9; m++) v[i][m] = bval[(blk * 9 + m) * 64 + l];
+        }
+        if (PRE)
+#pragma unroll
+            for (int i = 0; i < RG; i++)
+#pragma unroll
+                for (int m = 0; m < 3; m++) {
+                    zc[PRE ? i : 0][m] = z[3L * c[i] + m];
+                    pc[PRE ? i : 0][m] = pold[3L * c[i] + m];
+                }
+    };
+    if (!was_done && RG * wv < w) load_group(RG * wv);
+    if (wv == 0) {
+        double b = 0.0;
+        const bool d = was_done || direction_beta(T, part, g, s, l == 0, close, o, sc, ndone, b);
+        if (l == 0) {
+            sbeta = b;
+            sdone = d;
+        }
+    }
+    __syncthreads();
+    if (sdone) return;
+    const double beta = sbeta;
+    double yi[3] = {0.0, 0.0, 0.0};
+    for (int r0 = 0; r0 < w; r0 += RG * NW) {
+        const int k0 = r0 + RG * wv;
+        if (k0 < w) {
+            if (r0 > 0) load_group(k0);
+            double gs[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int i = 0; i < RG; i++) {
+                double xv[3], vd[9];
+#pragma unroll
+                for (int m = 0; m < 3; m++)
+                    xv[m] = PRE ? zc[PRE ? i : 0][m] + beta * pc[PRE ? i : 0][m] : z[3L * c[i] + m] + beta * pold[3L * c[i] + m];
+#pragma unroll
+                for (int m = 0; m < 9; m++) vd[m] = (double)v[i][m];
+                if (k0 + i < w) block_mac(vd, xv[0], xv[1], xv[2], gs);
+            }
+#pragma unroll
+            for (int i = 0; i < 3; i++) red[wv][i][l] = gs[i];
+        }
+        __syncthreads();
+        if (wv == 0)
+            for (int j = 0; j < NW && r0 + RG * j < w; j++)
+#pragma unroll
+                for (int i = 0; i < 3; i++) yi[i] += red[j][i][l];
+        if (r0 + RG * NW < w) __syncthreads();
+    }
+    if (wv > 0) return;
+    double dv = 0.0;
+    if (own) {
+        double p3[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            p3[i] = z[3L * a + i] + beta * pold[3L * a + i];
+            pnew[3L * a + i] = p3[i];
+            y[3L * a + i] = yi[i];
+        }
+        dv = yi[0] * p3[0] + yi[1] * p3[1] + yi[2] * p3[2];
+    }
+    dv = wsum(dv);
+    if (l == 0) ppq[s] = dv;
 }
 
-__global__ void __launch_bounds__(FB) k_seg_fin_dot(const double* __restrict__ part, long nslices,
-                                                    const int* __restrict__ seg_slice, double* __restrict__ out)
+// per-segment dot product a.b into out[seg]: partials per group, then totals
+__global__ void __launch_bounds__(PB) k_seg_dot(SegTab T, int nnd, const double* __restrict__ x,
+                                                const double* __restrict__ y, double* __restrict__ part)
+{
+    const int4 gr = T.grp[blockIdx.x];
+    const int a = 64 * gr.x + threadIdx.x;
+    double v[1] = {0.0};
+    if ((int)(threadIdx.x >> 6) < gr.y && a < nnd)
+#pragma unroll
+        for (int i = 0; i < 3; i++) v[0] += x[3L * a + i] * y[3L * a + i];
+    v[0] = wsum(v[0]);
+    group_partials<1>(v, part, 0, {true});
+}
+
+__global__ void __launch_bounds__(FB) k_seg_fin_dot(SegTab T, const double* __restrict__ part, double* __restrict__ out)
 {
     const int g = blockIdx.x;
     double tot[1];
-    seg_total<1>(part, nslices, seg_slice[g], seg_slice[g + 1], tot);
+    seg_total<1, true>(part + T.seg_grp[g], 0, T.groups(g), T.slices(g), tot);
     if (threadIdx.x == 0) out[g] = tot[0];
 }
 
@@ -641,6 +880,12 @@ __global__ void __launch_bounds__(FB) k_seg_fin_dot(const double* __restrict__ p
 // ---------------------------------------------------------------------------
 
 static unsigned node_blocks(const tg_ctx* c) { return (unsigned)((c->nnd + PB - 1) / PB); }
+
+static SegTab seg_tab(const tg_ctx* c)
+{
+    const Segments& S = c->seg;
+    return SegTab{S.d_slice_seg.p, S.d_seg_slice.p, S.d_seg_grp.p, S.d_grp.p, S.nseg, S.nslices};
+}
 
 // f(std::integral_constant<int, v>) for the SpMV variant v = 0..7 (bit 0
 // XCD row ranges, bit 1 unrolled loop, bit 2 symmetric read), so every
@@ -662,12 +907,12 @@ static void spmv_dispatch(int v, F f)
 
 void segment_dots(tg_ctx* c, const double* a, const double* b, double* host_out)
 {
-    const long ns = c->seg.nslices;
     {
         TimedRegion tr(c, T_VECTOR);
-        hipLaunchKernelGGL(k_seg_dot, dim3(node_blocks(c)), dim3(PB), 0, c->stream, c->nnd, a, b, c->seg.d_part.p, ns);
-        hipLaunchKernelGGL(k_seg_fin_dot, dim3(c->seg.nseg), dim3(FB), 0, c->stream, c->seg.d_part.p, ns,
-                           c->seg.d_seg_slice.p, c->seg.d_out.p);
+        const SegTab T = seg_tab(c);
+        hipLaunchKernelGGL(k_seg_dot, dim3((unsigned)c->seg.ngroups), dim3(PB), 0, c->stream, T, c->nnd, a, b,
+                           c->seg.d_part.p);
+        hipLaunchKernelGGL(k_seg_fin_dot, dim3(c->seg.nseg), dim3(FB), 0, c->stream, T, c->seg.d_part.p, c->seg.d_out.p);
         TG_HIP(hipGetLastError());
     }
     TG_HIP(hipMemcpyAsync(host_out, c->seg.d_out.p, sizeof(double) * c->seg.nseg, hipMemcpyDeviceToHost, c->stream));
@@ -690,9 +935,9 @@ void pcg_run(tg_ctx* c, const MT* val, const double* dinv, const double* b, doub
     } else {
         // the context's own reductions, scalars and done count; the second
         // direction buffer of the fused iteration is allocated on first use
-        if (pcg_fused(c) && c->precond != TG_PC_BLOCK_JACOBI && c->vp2.n != 3 * (size_t)c->nnd)
-            c->vp2.alloc(3 * (size_t)c->nnd);
-        W = PcgWork{c->seg.d_part.p, c->seg.d_scal.p, c->seg.d_ndone.p, c->vp2.p, true};
+        if (pcg_fused(c) && c->vp2.n != 3 * (size_t)c->nnd) c->vp2.alloc(3 * (size_t)c->nnd);
+        W = PcgWork{c->seg.d_part.p, c->seg.d_part.p + 2 * c->seg.nslices, c->seg.d_scal.p, c->seg.d_ndone.p, c->vp2.p,
+                    c->vz.p, true};
     }
     if (c->precond == TG_PC_BLOCK_JACOBI)
         pcg_loop<MT, 1>(c, val, c->vbinv.p, b, x, r, p, q, rtol, maxit, d_active, W, st);
@@ -709,7 +954,8 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
     Segments& S = c->seg;
     const long ns = S.nslices;
     const int nseg = S.nseg;
-    const unsigned nb = node_blocks(c);
+    const unsigned nb = node_blocks(c), ng = (unsigned)S.ngroups;
+    const SegTab T = seg_tab(c);
     TG_HIP(hipMemsetAsync(W.ndone, 0, sizeof(int), c->stream));
     // multigrid: dinv is the z vector; *done of the single segment gates the V-cycle
     const double* done = W.scal + S_DONE * nseg;
@@ -717,11 +963,23 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
         TimedRegion tr(c, T_PRECOND);
         amg_vcycle(c, b, (double*)dinv, nullptr);
     }
+    // The totals are formed inside the kernels that need them (FOLD) when no
+    // segment has more than FOLD_SLICES slices and the work space has room
+    // for the partials of p.q beside those of r.z and r.r; the multigrid
+    // needs r.r before its cycle and r.z after it, and keeps its finalize
+    // kernels.
+    const bool fold = PC != 2 && W.ppq && S.max_slices <= FOLD_SLICES;
+    const bool fused = pcg_fused(c) && (PC != 1 || fold);
+    // M^-1 r kept by the update: for the folded fused iteration, whose SpMV
+    // gathers it, and for block Jacobi, whose direction would form it again
+    // from the 3x3 blocks
+    const bool keep_z = PC != 2 && W.z && (fold ? fused || PC == 1 : false);
+    double* z = keep_z ? W.z : nullptr;
     {
         TimedRegion tr(c, T_VECTOR);
-        hipLaunchKernelGGL(k_seg_init<PC>, dim3(nb), dim3(PB), 0, c->stream, c->nnd, b, dinv, x, r, p, W.part, ns);
-        hipLaunchKernelGGL(k_seg_fin_init, dim3(nseg), dim3(FB), 0, c->stream, W.part, ns, S.d_seg_slice.p,
-                           d_active, nseg, W.scal, rtol, maxit, W.ndone);
+        hipLaunchKernelGGL(k_seg_init<PC>, dim3(ng), dim3(PB), 0, c->stream, T, c->nnd, b, dinv, x, r, p, z, W.part);
+        hipLaunchKernelGGL(k_seg_fin_init, dim3(nseg), dim3(FB), 0, c->stream, T, W.part, d_active, W.scal, rtol, maxit,
+                           W.ndone);
     }
     // small segments: the whole iteration in one persistent workgroup each
     // (the list is built at set-up and when the threshold changes)
@@ -734,44 +992,87 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
         TG_HIP(hipGetLastError());
     }
     if (npers < nseg) {
-    const int CHUNK = PC == 2 ? 8 : 16;  // even: the fused iteration alternates its two direction buffers
-    const bool fused = pcg_fused(c) && PC != 1;
+    const int CHUNK = PC == 2 ? 8 : 16;  // even: direction buffers and scalar slots alternate
     double* pbuf[2] = {p, nullptr};
     if (fused) {
         if (!W.p2) fail(TG_GENERAL_FAIL, "fused PCG iteration without its second direction buffer");
         pbuf[1] = W.p2;
     }
     const int variant = spmv_variant(c);
+    double* ppq = fold ? W.ppq : W.part;
+    // rows split over the waves of a workgroup
+    const int split = fold && fused ? pcg_split(c) : 0;
+    auto update = [&](const double* pk, int o) {
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(ng), dim3(PB), 0, c->stream, T, c->nnd, pk, q, dinv, x, r, z, ppq, W.part, o,
+                               W.scal);
+        };
+        if (fold)
+            go(k_seg_update<PC, true>);
+        else
+            go(k_seg_update<PC, false>);
+    };
+    auto fin_alpha = [&](int o) {
+        hipLaunchKernelGGL(k_seg_fin_alpha, dim3(nseg), dim3(FB), 0, c->stream, T, ppq, o, W.scal);
+    };
+    auto fin_beta = [&](int o) {
+        hipLaunchKernelGGL(k_seg_fin_beta, dim3(nseg), dim3(FB), 0, c->stream, T, W.part, o, W.scal, W.ndone);
+    };
+    auto precond_pass = [&]() {
+        TimedRegion tr(c, T_PRECOND);
+        amg_vcycle(c, r, (double*)dinv, done);
+        hipLaunchKernelGGL(k_seg_dot, dim3(ng), dim3(PB), 0, c->stream, T, c->nnd, r, dinv, W.part);
+    };
+    // the fused SpMV of iteration k; folded, it closes iteration k - 1 itself
+    // (slot o = (k - 1) & 1), except in the first iteration of a chunk, which
+    // finds beta in its scalar slot
+    auto spmv_fused = [&](int k) {
+        TimedRegion tr(c, T_SPMV);
+        const double* pold = pbuf[k & 1];
+        double* pnew = pbuf[(k + 1) & 1];
+        const int close = fold && k > 0, o = (k + 1) & 1;
+        auto go_split = [&](auto kernel, int nw) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(ns + 7) / 8 * 8), dim3(64 * nw), 0, c->stream, T, c->nnd, c->op.d_slice_base.p,
+                               c->op.d_slice_width.p, c->op.d_col.p, val, z, pold, pnew, q, W.part, ppq, close, o,
+                               W.scal, W.ndone);
+        };
+        if (split == 9) {
+            go_split(k_split_spmv<MT, 9, true>, 9);
+            return;
+        }
+        if (split == 5) {
+            go_split(k_split_spmv<MT, 5, false>, 5);
+            return;
+        }
+        if (split == 3) {
+            go_split(k_split_spmv<MT, 3, false>, 3);
+            return;
+        }
+        spmv_dispatch(variant, [&](auto V) {
+            constexpr int v = decltype(V)::value;
+            auto go = [&](auto kernel, const double* m) {
+                hipLaunchKernelGGL(kernel, dim3((v & 1) ? (nb + 7) / 8 * 8 : nb), dim3(PB), 0, c->stream, T, c->nnd,
+                                   c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val, c->op.d_tpos.p, m,
+                                   r, pold, pnew, q, W.part, ppq, close, o, W.scal, W.ndone);
+            };
+            if (PC == 2 || z)
+                go(k_fused_spmv<MT, 2, (v & 1) != 0, (v & 2) != 0, (v & 4) != 0>, z ? z : dinv);
+            else if constexpr (PC == 0)
+                go(k_fused_spmv<MT, 0, (v & 1) != 0, (v & 2) != 0, (v & 4) != 0>, dinv);
+        });
+    };
     auto issue_fused = [&]() {
         for (int k = 0; k < CHUNK; k++) {
-            double* pold = pbuf[k & 1];
-            double* pnew = pbuf[(k + 1) & 1];
-            {
-                TimedRegion tr(c, T_SPMV);
-spmv_dispatch(variant, [&](auto V) {
-                    constexpr int v = decltype(V)::value;
-                    hipLaunchKernelGGL((k_fused_spmv<MT, PC, (v & 1) != 0, (v & 2) != 0, (v & 4) != 0>),
-                                       dim3((v & 1) ? (nb + 7) / 8 * 8 : nb), dim3(PB), 0, c->stream, c->nnd,
-                                       S.d_slice_seg.p, c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val,
-                                       c->op.d_tpos.p, dinv, r, pold, pnew, q, W.part, ns, nseg, W.scal);
-                });
-            }
+            spmv_fused(k);
             {
                 TimedRegion tr(c, T_VECTOR);
-                hipLaunchKernelGGL(k_seg_fin_alpha, dim3(nseg), dim3(FB), 0, c->stream, W.part, ns,
-                                   S.d_seg_slice.p, nseg, W.scal);
-                hipLaunchKernelGGL(k_seg_update<PC>, dim3(nb), dim3(PB), 0, c->stream, c->nnd, S.d_slice_seg.p, pnew,
-                                   q, dinv, x, r, W.part, ns, nseg, W.scal);
+                if (!fold) fin_alpha(k & 1);
+                update(pbuf[(k + 1) & 1], k & 1);
             }
-            if (PC == 2) {
-                TimedRegion tr(c, T_PRECOND);
-                amg_vcycle(c, r, (double*)dinv, done);
-                hipLaunchKernelGGL(k_seg_dot, dim3(nb), dim3(PB), 0, c->stream, c->nnd, r, dinv, W.part, ns);
-            }
-            {
+            if (PC == 2) precond_pass();
+            if (!fold || k == CHUNK - 1) {
                 TimedRegion tr(c, T_VECTOR);
-                hipLaunchKernelGGL(k_seg_fin_beta, dim3(nseg), dim3(FB), 0, c->stream, W.part, ns,
-                                   S.d_seg_slice.p, nseg, W.scal, W.ndone);
+                fin_beta(k & 1);
             }
         }
     };
@@ -783,32 +1084,33 @@ spmv_dispatch(variant, [&](auto V) {
         for (int k = 0; k < CHUNK; k++) {
             {
                 TimedRegion tr(c, T_SPMV);
-spmv_dispatch(variant, [&](auto V) {
+                spmv_dispatch(variant, [&](auto V) {
                     constexpr int v = decltype(V)::value;
                     hipLaunchKernelGGL((k_seg_spmv<MT, (v & 1) != 0, (v & 2) != 0, (v & 4) != 0>),
-                                       dim3((v & 1) ? (nb + 7) / 8 * 8 : nb), dim3(PB), 0, c->stream, c->nnd,
-                                       S.d_slice_seg.p, c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val,
-                                       c->op.d_tpos.p, p, q, W.part, ns, nseg, W.scal);
+                                       dim3((v & 1) ? (nb + 7) / 8 * 8 : nb), dim3(PB), 0, c->stream, T, c->nnd,
+                                       c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val,
+                                       c->op.d_tpos.p, p, q, ppq, W.scal);
                 });
             }
             {
                 TimedRegion tr(c, T_VECTOR);
-                hipLaunchKernelGGL(k_seg_fin_alpha, dim3(nseg), dim3(FB), 0, c->stream, W.part, ns,
-                                   S.d_seg_slice.p, nseg, W.scal);
-                hipLaunchKernelGGL(k_seg_update<PC>, dim3(nb), dim3(PB), 0, c->stream, c->nnd, S.d_slice_seg.p, p, q,
-                                   dinv, x, r, W.part, ns, nseg, W.scal);
+                if (!fold) fin_alpha(k & 1);
+                update(p, k & 1);
             }
-            if (PC == 2) {
-                TimedRegion tr(c, T_PRECOND);
-                amg_vcycle(c, r, (double*)dinv, done);
-                hipLaunchKernelGGL(k_seg_dot, dim3(nb), dim3(PB), 0, c->stream, c->nnd, r, dinv, W.part, ns);
-            }
+            if (PC == 2) precond_pass();
             {
                 TimedRegion tr(c, T_VECTOR);
-                hipLaunchKernelGGL(k_seg_fin_beta, dim3(nseg), dim3(FB), 0, c->stream, W.part, ns,
-                                   S.d_seg_slice.p, nseg, W.scal, W.ndone);
-                hipLaunchKernelGGL(k_seg_direction<PC>, dim3(nb), dim3(PB), 0, c->stream, c->nnd, S.d_slice_seg.p, r,
-                                   dinv, p, ns, nseg, W.scal);
+                if (!fold) fin_beta(k & 1);
+                auto go = [&](auto kernel, const double* m) {
+                    hipLaunchKernelGGL(kernel, dim3(ng), dim3(PB), 0, c->stream, T, c->nnd, r, m, p, W.part, k & 1,
+                                       W.scal, W.ndone);
+                };
+                if (!fold)
+                    go(k_seg_direction<PC, false>, dinv);
+                else if (z)
+                    go(k_seg_direction<2, true>, z);
+                else
+                    go(k_seg_direction<PC, true>, dinv);
             }
         }
     };
@@ -821,10 +1123,10 @@ spmv_dispatch(variant, [&](auto V) {
         // every address and size the chunk's launches take (tg_initialize
         // also drops the graph, as buffers may come back at old addresses)
         const void* key[24] = {val, dinv, x, r, p, q, W.part, W.scal, W.ndone,
-                               (const void*)(long)(PC + 4L * (variant + 8L * ((int)fused + 2L * c->amg.gen))),
+                               (const void*)(long)(PC + 4L * (variant + 8L * ((int)fused + 2L * (split + 16L * c->amg.gen)))),
                                (const void*)(long)sizeof(MT), (const void*)(long)c->nnd, (const void*)(long)nseg,
-                               (const void*)ns, S.d_seg_slice.p, S.d_slice_seg.p, c->op.d_slice_base.p,
-                               c->op.d_slice_width.p, c->op.d_col.p, pbuf[1], c->vbinv.p,
+                               (const void*)ns, S.d_grp.p, S.d_slice_seg.p, c->op.d_slice_base.p,
+                               c->op.d_slice_width.p, c->op.d_col.p, pbuf[1], z,
                                c->amg.lv.empty() ? nullptr : (const void*)c->amg.lv[0], c->op.d_tpos.p};
         if (!c->pg.exec || std::memcmp(key, c->pg.key, sizeof key) != 0) {
             drop_pcg_graph(c);

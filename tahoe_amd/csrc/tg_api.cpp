@@ -158,7 +158,20 @@ static void setup_segments(tg_ctx* c)
     S.d_active.alloc((size_t)S.nseg);
     S.d_elem_seg.alloc((size_t)c->nel);
     S.d_scal.alloc((size_t)S_NSCAL * S.nseg);
-    S.d_part.alloc(2 * (size_t)S.nslices);
+    S.max_slices = 0;
+    for (int g = 0; g < S.nseg; g++) S.max_slices = std::max(S.max_slices, (long)(seg_slice[g + 1] - seg_slice[g]));
+    std::vector<int> seg_grp((size_t)S.nseg + 1, 0);
+    std::vector<int4> grp;
+    grp.reserve((size_t)S.nslices / 4 + S.nseg);
+    for (int g = 0; g < S.nseg; g++) {
+        for (int s = seg_slice[g]; s < seg_slice[g + 1]; s += 4)
+            grp.push_back(make_int4(s, std::min(4, seg_slice[g + 1] - s), g, 0));
+        seg_grp[g + 1] = (int)grp.size();
+    }
+    S.ngroups = (long)grp.size();
+    S.d_seg_grp.alloc(seg_grp.size());
+    S.d_grp.alloc(grp.size());
+    S.d_part.alloc(3 * (size_t)S.nslices);
     S.d_out.alloc((size_t)S.nseg);
     S.d_ndone.alloc(1);
     S.d_segstat.alloc((size_t)S.nseg);
@@ -170,6 +183,8 @@ static void setup_segments(tg_ctx* c)
     };
     up(S.d_slice_seg.p, slice_seg);
     up(S.d_seg_slice.p, seg_slice);
+    up(S.d_seg_grp.p, seg_grp);
+    TG_HIP(hipMemcpyAsync(S.d_grp.p, grp.data(), sizeof(int4) * grp.size(), hipMemcpyHostToDevice, c->stream));
     up(S.d_active.p, ones);
     up(S.d_elem_seg.p, S.elem_seg);
     TG_HIP(hipMemsetAsync(S.d_scal.p, 0, sizeof(double) * S_NSCAL * S.nseg, c->stream));
@@ -900,8 +915,9 @@ int tg_solve_noalloc(tg_ctx* c, const double* b_dev, double* x_dev, double rtol,
         if (c->linear_solver != TG_LIN_PCG) fail(TG_BAD_INPUT, "tg_solve_noalloc: PCG only");
         double* base = (double*)scratch_of(c->device);
         if (!base) fail(TG_GENERAL_FAIL, "tg_solve_noalloc: scratch not resolved for this device");
-        // layout (doubles): b, x, r, p, q, p2 [3 nnd each], part [2 nslices],
-        // scal [S_NSCAL nseg], then the done count (int)
+        // layout (doubles): b (then z), x, r, p, q, p2 [3 nnd each], part
+        // [2 nslices], scal [S_NSCAL nseg], the done count (int), and where it
+        // still fits the partials of p.q [nslices]
         const size_t n3 = 3 * (size_t)c->nnd;
         const size_t ns = (size_t)c->seg.nslices, nseg = (size_t)c->seg.nseg;
         const size_t ndoubles = 6 * n3 + 2 * ns + (size_t)S_NSCAL * nseg;
@@ -932,7 +948,9 @@ int tg_solve_noalloc(tg_ctx* c, const double* b_dev, double* x_dev, double rtol,
         // every buffer the run reads before writing is set by the run itself
         // (x, r, p, partials and scalars by the init kernels, the done count
         // by a clear), so what an earlier call left does not matter
-        const PcgWork W{part, scal, ndone, vp2, false};
+        double* ppq = scal + (size_t)S_NSCAL * nseg + 1;  // past the done count
+        if (need + sizeof(int) + ns * sizeof(double) > (size_t)TG_NOALLOC_SCRATCH_BYTES) ppq = nullptr;
+        const PcgWork W{part, ppq, scal, ndone, vp2, vb, false};
         if (mixed_operator(c))
             pcg_run<float>(c, c->op.d_val32.p, c->vdinv.p, vb, vx, vr, vp, vq, rtol, maxit, c->seg.d_active.p,
                            c->seg.nseg, st, &W);

@@ -244,7 +244,10 @@ struct Gmres {
 };
 
 // device scalar slots of an iteration (per segment for the PCG)
-enum { S_RZ = 0, S_PQ, S_ALPHA, S_RZNEW, S_RR, S_BETA, S_BB, S_DONE, S_ITER, S_THRESH, S_MAXIT, S_DOT, S_NSCAL };
+// (S_RZ / S_RZ1 and S_IT0 / S_IT1: r.z and the iteration count, alternating
+// from one PCG iteration to the next; S_DOT is a slot of the context's own
+// scalars, not of a segment's)
+enum { S_RZ = 0, S_IT0, S_ALPHA, S_RZ1, S_RR, S_BETA, S_BB, S_DONE, S_ITER, S_THRESH, S_MAXIT, S_DOT, S_IT1 = S_DOT, S_NSCAL };
 
 // Independent problems packed in one context: segment g owns nodes
 // [node_begin[g], node_begin[g+1]), each starting at a multiple of 64, so a
@@ -252,14 +255,18 @@ enum { S_RZ = 0, S_PQ, S_ALPHA, S_RZNEW, S_RR, S_BETA, S_BB, S_DONE, S_ITER, S_T
 struct Segments {
     int nseg = 1;
     long nslices = 0;
+    long max_slices = 0;                  // slices of the largest segment
+    long ngroups = 0;                     // groups of up to 4 slices of one segment
     std::vector<int> node_begin;          // [nseg+1]
     std::vector<int> elem_seg;            // [nel] segment of each element (host)
     DBuf<int> d_slice_seg;                // [nslices]
     DBuf<int> d_seg_slice;                // [nseg+1] first slice of each segment
+    DBuf<int> d_seg_grp;                  // [nseg+1] first group of each segment
+    DBuf<int4> d_grp;                     // [ngroups] (first slice, slices, segment, 0)
     DBuf<int> d_active;                   // [nseg] 1 = solve this segment
     DBuf<int> d_elem_seg;                 // [nel]
     DBuf<double> d_scal;                  // [S_NSCAL][nseg]
-    DBuf<double> d_part;                  // [2][nslices]
+    DBuf<double> d_part;                  // [3][nslices]: r.z, r.r, p.q
     DBuf<double> d_out;                   // [nseg]
     DBuf<int> d_ndone;
     DBuf<int> d_segstat;                  // [nseg] 7 when an element of the segment inverted in a residual pass
@@ -381,24 +388,38 @@ inline bool mixed_stiffness(const tg_ctx* c) { return c->precision == TG_MIXED &
 inline bool mixed_operator(const tg_ctx* c) { return c->precision == TG_MIXED; }
 // the stiffness shape in effect (the measured fastest untuned choice at 128^3)
 inline int stiffness_shape(const tg_ctx* c) { return c->stiff_variant >= 0 ? c->stiff_variant : (mixed_stiffness(c) ? 17 : 9); }
-// PCG variants in effect.  Untuned: a single problem of 2^17 nodes or more
-// reads lower blocks through their partners (XCD row ranges, unrolled loop)
-// and forms the direction in its own pass, the fastest pair at 128^3 in
-// FP64 and mixed precision.  A batch of 2^17 nodes or more reads the full
-// operator in index order with the unrolled loop, direction in its own pass
-// (the fastest pair on 2 M-element batches of RVE cubes of edge 4-24: the
-// symmetric read is slower on small cubes, whose rows are mostly boundary
-// rows, and the fused direction's extra gathers cost more than the launch
-// it saves).  Smaller problems and batches, which are launch-bound, read in
-// hardware order with the direction formed inside the SpMV.  Every choice
-// gives bitwise the same iterates.
+// PCG variants in effect, untuned, by the size that decides what bounds the
+// SpMV (us per iteration on cubes, FP32 / FP64 operator; every choice gives
+// bitwise the same iterates):
+//  - up to 98,304 nodes (1,536 slices) the direction is formed inside the
+//    SpMV, whose workgroups share a slice's rows (pcg_split): one lane per
+//    row leaves the chip waiting on its 27 dependent blocks.  25^3 nodes:
+//    23.2 / 33.1 with a lane per row, 9.5 / 11.8 split; 46^3: 37 / 47 and
+//    30 / 40;
+//  - above, the operator's bytes bound it and the fused direction's second
+//    gathered vector costs more than the direction pass: 124 k nodes, mixed:
+//    38.6 fused and split, 35.4 with the unrolled row loop (variant 3);
+//  - a single problem of 2^17 nodes or more reads lower blocks through their
+//    partners (7), a batch of that size the full operator in index order (2;
+//    its rows are mostly boundary rows, where the symmetric read diverges).
 inline bool large_single(const tg_ctx* c) { return c->seg.nseg <= 1 && c->nnd >= (1 << 17); }
 inline bool large_total(const tg_ctx* c) { return c->nnd >= (1 << 17); }
+inline bool pcg_small(const tg_ctx* c) { return c->nnd <= 64 * 1536; }
 inline int spmv_variant(const tg_ctx* c)
 {
-    return c->spmv_xcd >= 0 ? c->spmv_xcd : (large_single(c) ? 7 : large_total(c) ? 2 : 0);
+    return c->spmv_xcd >= 0 ? c->spmv_xcd : (large_single(c) ? 7 : large_total(c) ? 2 : pcg_small(c) ? 0 : 3);
 }
-inline bool pcg_fused(const tg_ctx* c) { return c->pcg_fused >= 0 ? c->pcg_fused != 0 : !large_total(c); }
+inline bool pcg_fused(const tg_ctx* c) { return c->pcg_fused >= 0 ? c->pcg_fused != 0 : pcg_small(c); }
+// waves that share a slice's rows in the fused SpMV (untuned SpMV variant
+// only; 0: a lane per row).  More waves per row shorten its chain but fill
+// the chip sooner: 245 slices 9.3 / 10.4 / 11.2 us per iteration with 9, 5
+// and 3 waves (FP32), 562 slices 20.8 / 17.8 / 18.1, 1,077 slices 31.0 /
+// 28.2 / 25.4.
+inline int pcg_split(const tg_ctx* c)
+{
+    if (c->spmv_xcd >= 0 || !pcg_small(c)) return 0;
+    return c->nnd <= 64 * 256 ? 9 : c->nnd <= 64 * 640 ? 5 : 3;
+}
 // segments of at most this many slices run their whole PCG in one
 // persistent workgroup of 1024 threads, one node each (0: none).  Default
 // 12 slices (768 nodes, an 8^3-element cube): there it halves a PCG
@@ -406,6 +427,9 @@ inline bool pcg_fused(const tg_ctx* c) { return c->pcg_fused >= 0 ? c->pcg_fused
 // faster with a kernel per step.
 constexpr int PCG_PERSIST_MAX = 16;
 constexpr int PCG_PERSIST_DEFAULT = 12;
+// a segment of at most this many slices has its reductions formed inside the
+// kernels that need them (k_pcg.hip: wave_total)
+constexpr int PCG_FOLD_SLICES = 4096;
 inline int pcg_persist(const tg_ctx* c) { return c->pcg_persist >= 0 ? c->pcg_persist : PCG_PERSIST_DEFAULT; }
 
 // TG_SETUP_TRACE=1 prints host-side set-up phases to stderr, each timed
@@ -451,14 +475,19 @@ void pcg_solve_mixed(tg_ctx* c, const double* b_node, double* x_node, double rto
 double device_dot(tg_ctx* c, const double* a, const double* b, long n);
 void pcg_solve(tg_ctx* c, const double* b_node, double* x_node, double rtol, int maxit, tg_lin_stats* st);
 // Device work space of one PCG run besides its vectors: per-slice reduction
-// partials [2][nslices], per-segment scalar slots [S_NSCAL][nseg], the done
-// count [1] and the second direction buffer of the fused iteration [3 nnd];
+// partials of r.z and r.r [2][nslices] and of p.q [nslices] (nullptr: p.q
+// shares the first, and the totals keep their own kernels), per-segment
+// scalar slots [S_NSCAL][nseg], the done count [1], the second direction
+// buffer of the fused iteration [3 nnd] and a vector for M^-1 r [3 nnd]
+// (the right-hand side's array will do: it is read before z is written);
 // graph = false issues every launch directly (no capture, no instantiation).
 struct PcgWork {
     double* part = nullptr;
+    double* ppq = nullptr;
     double* scal = nullptr;
     int* ndone = nullptr;
     double* p2 = nullptr;
+    double* z = nullptr;
     bool graph = true;
 };
 // work = nullptr: the context's own buffers
