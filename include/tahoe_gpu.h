@@ -341,9 +341,20 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
  *                      start a new solve (the next tangent sets the coarse
  *                      levels up again).  0: a new set-up for every
  *                      tangent; default 6. */
+/* TG_TUNE_STIFF_ROWS   1 (default): the element kernels write their 3x3
+ *                      blocks to a buffer (all elements in one launch), and
+ *                      one gather by matrix rows sums them in element order
+ *                      and writes the MSR values, the solver's operator and
+ *                      1/diag once; 0: the colour-ordered assembly of the
+ *                      knobs above.  Setting TG_TUNE_STIFF_CHUNK,
+ *                      TG_TUNE_STIFF_SHAPE, TG_TUNE_NEWTON_ASSEMBLY or
+ *                      TG_TUNE_STIFF_GATHER also selects the colour-ordered
+ *                      assembly; setting this one to 1 afterwards takes it
+ *                      back.  Reads 0 too on a mesh whose rows have more
+ *                      than 27 upper blocks (the gather's LDS). */
 enum { TG_TUNE_STIFF_CHUNK = 1, TG_TUNE_STIFF_SHAPE = 2, TG_TUNE_NEWTON_ASSEMBLY = 3, TG_TUNE_PCG_GRAPH = 4,
        TG_TUNE_SPMV_XCD = 5, TG_TUNE_AMG_DEGREE = 6, TG_TUNE_AMG_WEIGHT = 7, TG_TUNE_PCG_FUSED = 8,
-       TG_TUNE_STIFF_GATHER = 9, TG_TUNE_PCG_PERSIST = 10, TG_TUNE_AMG_REUSE = 11 };
+       TG_TUNE_STIFF_GATHER = 9, TG_TUNE_PCG_PERSIST = 10, TG_TUNE_AMG_REUSE = 11, TG_TUNE_STIFF_ROWS = 12 };
 int tg_set_tuning(tg_ctx* ctx, int knob, long value);
 int tg_get_tuning(tg_ctx* ctx, int knob, long* value);
 

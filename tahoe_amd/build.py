@@ -20,7 +20,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 HOST_SOURCES = ["TotalLagrangianHIPT.cpp", "HIPMSRMatrixT.cpp", "NLSolverHIP.cpp", "InputDeck.cpp",
                 "FEManagerHIP.cpp"]
 
-SOURCES = ["tg_setup.cpp", "tg_amg.cpp", "tg_api.cpp", "k_element.hip", "k_q1p0.hip", "k_gather.hip", "k_solver.hip",
+SOURCES = ["tg_setup.cpp", "tg_amg.cpp", "tg_api.cpp", "k_element.hip", "k_q1p0.hip", "k_rows.hip", "k_gather.hip", "k_solver.hip",
            "k_pcg.hip", "k_amg.hip", "k_gmres.hip", "k_graph.hip"]
 HEADERS = ["tg_internal.h", "tg_kinematics.h", "tg_element.h", "../../include/tahoe_gpu.h"]
 # per-source extra flags.  The PCG kernels are built without FMA

@@ -18,26 +18,27 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 
 
-// R -= f_int for the elements of one colour.  Per integration point
-// (TotalLagrangianT::FormKd, TotalLagrangianT.cpp:107-143, called with
-// constK = -1 from SolidElementT::ElementRHSDriver, SolidElementT.cpp:1240):
+// -f_int of every element into the force buffer [element][rank][3] (k_rows.hip
+// sums it by nodes).  Per integration point (TotalLagrangianT::FormKd,
+// TotalLagrangianT.cpp:107-143, called with constK = -1 from
+// SolidElementT::ElementRHSDriver, SolidElementT.cpp:1240):
 //   R_a,i += -J w det0 sum_k (sigma F^-T)_ik dN_a/dX_k
+// Bound by FP64 issue; one launch over all elements in mesh order, where the
+// passes colour by colour paid eight launches and read and wrote R each time.
 template <int MAT>
-__global__ void __launch_bounds__(256) k_residual_tl(const int* __restrict__ elems, int count,
-                                                     const int* __restrict__ conn, const int* __restrict__ emat,
+__global__ void __launch_bounds__(256) k_residual_tl(int nel, const int* __restrict__ conn,
+                                                     const unsigned* __restrict__ perm, const int* __restrict__ emat,
                                                      const double2* __restrict__ props,
                                                      const double* __restrict__ X, const double* __restrict__ U,
-                                                     const int* __restrict__ eqn, double* __restrict__ R,
-                                                     int* __restrict__ status, const int* __restrict__ elem_seg,
-                                                     int* __restrict__ segstat)
+                                                     double* __restrict__ fe, int* __restrict__ status,
+                                                     const int* __restrict__ slice_seg, int* __restrict__ segstat)
 {
     __shared__ double sxu[32][8][6];
     const int t = threadIdx.x, le = t >> 3, q = t & 7;
-    const long slot = (long)blockIdx.x * 32 + le;
-    const bool valid = slot < count;
-    int e = 0, node = 0;
+    const int e = blockIdx.x * 32 + le;
+    const bool valid = e < nel;
+    int node = 0;
     if (valid) {
-        e = elems[slot];
         node = conn[8L * e + q];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -87,62 +88,38 @@ __global__ void __launch_bounds__(256) k_residual_tl(const int* __restrict__ ele
     double v[3];
     reduce_scatter8(r, q, v);
     if (valid) {
+        double* f = fe + 3 * (8L * e + rank_of(perm[e], q));
 #pragma unroll
-        for (int i = 0; i < 3; i++)
-            if (eqn[3L * node + i] >= 0) R[3L * node + i] += v[i];
+        for (int i = 0; i < 3; i++) f[i] = v[i];
     }
     if (bad) {
         // the context's flag, and the flag of the element's problem in a batch
         atomicOr(status, 7);
-        atomicOr(&segstat[elem_seg[e]], 7);
+        atomicOr(&segstat[slice_seg[node >> 6]], 7);
     }
 }
 
-void launch_q1p0(tg_ctx* c, const double* u, double* R_node, bool stiff);
+void launch_q1p0_forces(tg_ctx* c, const double* u);
+void launch_q1p0_blocks(tg_ctx* c, const double* u);
 
-// R += applied nodal forces at active dofs (FieldT::FormRHS, FieldT.cpp:390-401)
-__global__ void __launch_bounds__(256) k_add_forces(long n3, const int* __restrict__ eqn,
-                                                    const double* __restrict__ f, double* __restrict__ R)
-{
-    const long k = (long)blockIdx.x * 256 + threadIdx.x;
-    if (k < n3 && eqn[k] >= 0) R[k] += f[k];
-}
-
-static void element_residual(tg_ctx* c, const double* u, double* R_node);
-
-void launch_residual(tg_ctx* c, const double* u, double* R_node)
+void launch_residual(tg_ctx* c, const double* u, double* R_node, double* R_eq)
 {
     TimedRegion tr(c, T_RESIDUAL);
-    TG_HIP(hipMemsetAsync(R_node, 0, sizeof(double) * 3 * (size_t)c->nnd, c->stream));
-    element_residual(c, u, R_node);
-    if (c->dfext.p) {
-        const long n3 = 3L * c->nnd;
-        hipLaunchKernelGGL(k_add_forces, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, c->stream, n3, c->deqn.p,
-                           c->dfext.p, R_node);
+    if (c->formulation == TG_Q1P0) {
+        launch_q1p0_forces(c, u);
+    } else {
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((c->nel + 31) / 32), dim3(256), 0, c->stream, c->nel, c->dconn.p,
+                               c->r_perm.p, c->dmat.p, c->dmatprops.p, c->dX.p, u, c->r_force.p, c->dstatus.p,
+                               c->seg.d_slice_seg.p, c->seg.d_segstat.p);
+        };
+        if (c->material_model == TG_MAT_STVENANT)
+            go(k_residual_tl<MAT_STVENANT>);
+        else
+            go(k_residual_tl<MAT_SIMO>);
         TG_HIP(hipGetLastError());
     }
-}
-
-static void element_residual(tg_ctx* c, const double* u, double* R_node)
-{
-    if (c->formulation == TG_Q1P0) {
-        launch_q1p0(c, u, R_node, false);
-        return;
-    }
-    for (int col = 0; col < c->ncolors; col++) {
-        const int first = c->color_ptr[col], count = c->color_ptr[col + 1] - first;
-        if (count == 0) continue;
-        const int blocks = (count + 31) / 32;
-        if (c->material_model == TG_MAT_STVENANT)
-            hipLaunchKernelGGL(k_residual_tl<MAT_STVENANT>, dim3(blocks), dim3(256), 0, c->stream,
-                               c->dcolor_elems.p + first, count, c->dconn.p, c->dmat.p, c->dmatprops.p, c->dX.p, u,
-                               c->deqn.p, R_node, c->dstatus.p, c->seg.d_elem_seg.p, c->seg.d_segstat.p);
-        else
-            hipLaunchKernelGGL(k_residual_tl<MAT_SIMO>, dim3(blocks), dim3(256), 0, c->stream,
-                               c->dcolor_elems.p + first, count, c->dconn.p, c->dmat.p, c->dmatprops.p, c->dX.p, u,
-                               c->deqn.p, R_node, c->dstatus.p, c->seg.d_elem_seg.p, c->seg.d_segstat.p);
-    }
-    TG_HIP(hipGetLastError());
+    launch_node_residual(c, R_node, R_eq);
 }
 
 // ---------------------------------------------------------------------------
@@ -326,7 +303,9 @@ __device__ __forceinline__ void upper_block(int p, int& a, int& b)
 // before the block products, so the read half of the read-modify-write is in
 // flight during the arithmetic (no other element of the launch touches those
 // entries); 2 memory-side atomic adds with no return value; 5 (MSR path) the
-// element buffer of the gather assembly instead of the MSR.
+// element buffer of the gather assembly instead of the MSR; 6 the block
+// buffer of the assembly by rows (k_rows.hip; all elements in mesh order,
+// elems = nullptr, slot = the elements' ranks).
 template <class VT, int EPB, bool TO_OP, bool PM, int SC, int MAT = MAT_SIMO>
 __global__ void __launch_bounds__(36 * EPB) k_stiffness_tl(const int* __restrict__ elems, int count,
                                                              const int* __restrict__ conn,
@@ -347,11 +326,12 @@ __global__ void __launch_bounds__(36 * EPB) k_stiffness_tl(const int* __restrict
     auto ti = [](int le, int q, int k) { return PM ? (q * 6 + k) * EPB + le : (le * 8 + q) * 6 + k; };
     const int t = threadIdx.x;
     const long base = (long)blockIdx.x * EPB;
+    auto el = [&](int i) { return SC == 6 ? (int)(base + i) : elems[base + i]; };
     bool bad = false;
     if (t < 8 * EPB) {
         const int le = t >> 3, q = t & 7;
         if (base + le < count) {
-            const int node = conn[8L * elems[base + le] + q];
+            const int node = conn[8L * el(le) + q];
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 sxu[le][q][c] = X[3L * node + c];
@@ -364,7 +344,7 @@ __global__ void __launch_bounds__(36 * EPB) k_stiffness_tl(const int* __restrict
     if (t < 8 * EPB) {
         const int le = t >> 3, q = t & 7;
         const bool valid = base + le < count;
-        const double2 mk = valid ? props[emat[elems[base + le]]] : make_double2(0.0, 0.0);
+        const double2 mk = valid ? props[emat[el(le)]] : make_double2(0.0, 0.0);
         double g[3][8], D[21], T[6];
         bad |= !stiffness_ip<MAT>(q, valid, mk, [&](int a, int c) { return sxu[le][a][c]; }, g, D, T);
 #pragma unroll
@@ -386,7 +366,7 @@ __global__ void __launch_bounds__(36 * EPB) k_stiffness_tl(const int* __restrict
         int sidx[PRE ? 9 : 1];
         VT old[PRE ? 9 : 1];
         if (PRE) {
-            const int* es = slot + 300L * elems[base + le];
+            const int* es = slot + 300L * el(le);
 #pragma unroll
             for (int i = 0; i < 3; i++)
 #pragma unroll
@@ -447,6 +427,15 @@ __global__ void __launch_bounds__(36 * EPB) k_stiffness_tl(const int* __restrict
                     const int k = PRE ? 3 * i + j : 0;
                     if (sidx[k] >= 0) val[sidx[k]] = old[k] + K[i][j];
                 }
+        } else if (SC == 6) {
+            const unsigned pm = (unsigned)slot[base + le];
+            const int ra = rank_of(pm, a), rb = rank_of(pm, b);
+            VT* eb = val + 324L * (base + le) + 9 * pair_index(min(ra, rb), max(ra, rb));
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+#pragma unroll
+                for (int j = 0; j < 3; j++)
+                    if (a != b || j >= i) eb[ra <= rb ? 3 * i + j : 3 * j + i] = K[i][j];
         } else if (SC == 5) {
             // element buffer: val = the row of the launch's first element
             VT* eb = val + 300L * (base + le);
@@ -458,7 +447,7 @@ __global__ void __launch_bounds__(36 * EPB) k_stiffness_tl(const int* __restrict
                     if (n >= m) eb[upper_index(m, n)] = K[i][j];
                 }
         } else {
-            scatter_block<VT, TO_OP, SC == 2>(elems[base + le], a, b, p, K, conn, slot, eqn, val);
+            scatter_block<VT, TO_OP, SC == 2>(el(le), a, b, p, K, conn, slot, eqn, val);
         }
     }
     if (bad) atomicOr(status, 7);
@@ -513,8 +502,9 @@ static const std::vector<std::pair<int, int>>& stiffness_launches(tg_ctx* c)
     std::vector<long> rank((size_t)nseg, 0);
     std::vector<int> key((size_t)c->nel);
     int nkeys = 1;
+    const std::vector<int> seg_of = slice_segments(c);
     for (int e = 0; e < c->nel; e++) {
-        const int g = c->seg.elem_seg.empty() ? 0 : c->seg.elem_seg[e];
+        const int g = seg_of[(size_t)c->conn[8L * e] >> 6];
         key[e] = (int)(rank[g]++ / chunk);
         nkeys = std::max(nkeys, key[e] + 1);
     }
@@ -712,7 +702,9 @@ __device__ __forceinline__ int node_major(int p) { return 3 * (p & 7) + (p >> 3)
 // MINW > 1 asks the compiler for registers that fit MINW waves per SIMD.
 // GATHER: the entries go to the element buffer, val = its row of the
 // launch's first element (no slot map, no loads); else into the MSR.
-template <class VT, int EPW, int MAT = MAT_SIMO, int MINW = 1, bool GATHER = false>
+// ROWS (with GATHER): to the block buffer of the assembly by rows, all
+// elements in mesh order (elems = nullptr, slot = the elements' ranks).
+template <class VT, int EPW, int MAT = MAT_SIMO, int MINW = 1, bool GATHER = false, bool ROWS = false>
 __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restrict__ elems, int count,
                                                         const int* __restrict__ conn, const int* __restrict__ emat,
                                                         const double2* __restrict__ props,
@@ -728,11 +720,12 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
     const int l = threadIdx.x;
     const long base = (long)blockIdx.x * EPW;
     const int nel = (int)(count - base < EPW ? count - base : EPW);
+    auto el = [&](int i) { return ROWS ? (int)(base + i) : elems[base + i]; };
     bool bad = false;
     if (l < 8 * EPW) {
         const int le = l >> 3, q = l & 7;
         if (le < nel) {
-            const int node = conn[8L * elems[base + le] + q];
+            const int node = conn[8L * el(le) + q];
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 sxu[le][q][k] = X[3L * node + k];
@@ -744,7 +737,7 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
     if (l < 8 * EPW) {
         const int le = l >> 3, q = l & 7;
         if (le < nel) {
-            const double2 mk = props[emat[elems[base + le]]];
+            const double2 mk = props[emat[el(le)]];
             double g[3][8], D[21], T[6];
             bad |= !stiffness_ip<MAT>(q, true, mk, [&](int a, int k) { return sxu[le][a][k]; }, g, D, T);
 #pragma unroll
@@ -783,7 +776,7 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
     int nsidx[12];
     VT nold[12];
     if (!GATHER) {
-        const int* es = slot + 300L * elems[base];
+        const int* es = slot + 300L * el(0);
 #pragma unroll
         for (int k = 0; k < 12; k++) {
             const int x = es[ent[k] >= 0 ? ent[k] : 0];
@@ -796,7 +789,30 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
             nold[k] = nsidx[k] >= 0 ? x : VT(0);
         }
     }
+    // ROWS: places of the entries in the element's 36 x 9 block values, formed
+    // again only when the ranks change (structured meshes: never)
+    unsigned pm = 0;
+    int dst[ROWS ? 12 : 1];
+    auto place = [&](int p, int q) {
+        // dofs p and q of the dof-major order: nodes p & 7, q & 7, directions p >> 3, q >> 3
+        const int rp = rank_of(pm, p & 7), rq = rank_of(pm, q & 7), i = p >> 3, j = q >> 3;
+        const bool keep = rp < rq || (rp == rq && i <= j);
+        return 9 * pair_index(min(rp, rq), max(rp, rq)) + (keep ? 3 * i + j : 3 * j + i);
+    };
     for (int le = 0; le < nel; le++) {
+        if (ROWS) {
+            const unsigned x = __builtin_amdgcn_readfirstlane((unsigned)slot[base + le]);
+            if (x != pm) {
+                pm = x;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = Mfma<VT>::row(kq, r);
+                    dst[ROWS ? r : 0] = m <= c ? place(m, c) : -1;
+                    dst[ROWS ? 4 + r : 0] = lo8 ? place(m, 16 + na) : -1;
+                    dst[ROWS ? 8 + r : 0] = (lo8 && m < 8 && m <= c) ? place(16 + m, 16 + na) : -1;
+                }
+            }
+        }
         int sidx[12];
         VT old[12];
 #pragma unroll
@@ -806,7 +822,7 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
         }
         const bool more = !GATHER && le + 1 < nel;
         if (more) {
-            const int* es = slot + 300L * elems[base + le + 1];
+            const int* es = slot + 300L * el(le + 1);
 #pragma unroll
             for (int k = 0; k < 12; k++) {
                 const int x = es[ent[k] >= 0 ? ent[k] : 0];
@@ -873,6 +889,16 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
                 const VT x = val[nsidx[k] >= 0 ? nsidx[k] : 0];
                 nold[k] = nsidx[k] >= 0 ? x : VT(0);
             }
+        }
+        if (ROWS) {
+            VT* eb = val + 324L * (base + le);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (dst[ROWS ? r : 0] >= 0) eb[dst[ROWS ? r : 0]] = acc00[r];
+                if (dst[ROWS ? 4 + r : 0] >= 0) eb[dst[ROWS ? 4 + r : 0]] = acc01[r];
+                if (dst[ROWS ? 8 + r : 0] >= 0) eb[dst[ROWS ? 8 + r : 0]] = acc11[r];
+            }
+            continue;
         }
         if (GATHER) {
             VT* eb = val + 300L * (base + le);
@@ -997,9 +1023,49 @@ static bool gather_ready(tg_ctx* c)
     return true;
 }
 
+// Block buffer of the assembly by rows: the FP32 stiffness on the matrix
+// cores, FP64 in the 12-element block kernel (both the fastest untuned
+// shapes of their precision).
+static void launch_block_scatter(tg_ctx* c);
+
+template <class VT>
+static void launch_blocks(tg_ctx* c, const double* u, VT* eb)
+{
+    const int* ranks = reinterpret_cast<const int*>(c->r_perm.p);
+    const int n = c->nel;
+    auto go = [&](auto kernel, int epb, int threads) {
+        hipLaunchKernelGGL(kernel, dim3((n + epb - 1) / epb), dim3(threads), 0, c->stream, nullptr, n, c->dconn.p,
+                           c->dmat.p, c->dmatprops.p, c->dX.p, u, ranks, c->deqn.p, eb, c->dstatus.p);
+    };
+    if (c->material_model == TG_MAT_STVENANT)
+        go(k_stiffness_tl<VT, 12, false, false, 6, MAT_STVENANT>, 12, 36 * 12);
+    else if constexpr (sizeof(VT) == 4)
+        hipLaunchKernelGGL((k_stiffness_mfma<VT, 4, MAT_SIMO, 1, true, true>), dim3((n + 3) / 4), dim3(64), 0,
+                           c->stream, nullptr, n, c->dconn.p, c->dmat.p, c->dmatprops.p, c->dX.p, u, ranks, eb,
+                           c->dstatus.p);
+    else
+        go(k_stiffness_tl<VT, 12, false, false, 6, MAT_SIMO>, 12, 36 * 12);
+}
+
 void launch_stiffness(tg_ctx* c, const double* u)
 {
-    const bool gather = gather_ready(c);  // (setup on first use, outside the timed region)
+    c->op_fresh = false;
+    if (rows_assembly(c)) {
+        rows_buffers(c);
+        TimedRegion tr(c, T_STIFFNESS);
+        if (c->formulation == TG_Q1P0)
+            launch_q1p0_blocks(c, u);
+        else if (mixed_stiffness(c))
+            launch_blocks<float>(c, u, c->r_blocks32.p);
+        else
+            launch_blocks<double>(c, u, c->r_blocks.p);
+        TG_HIP(hipGetLastError());
+        launch_gather_rows(c);
+        c->op_fresh = true;
+        return;
+    }
+    colour_structure(c);                  // (set-up on first use, outside the timed region)
+    const bool gather = gather_ready(c);
     TimedRegion tr(c, T_STIFFNESS);
     const bool mixed = mixed_stiffness(c);
     const int v = std::min(std::max(stiffness_shape(c), 0), N_STIFF_SHAPES - 1);
@@ -1020,7 +1086,8 @@ void launch_stiffness(tg_ctx* c, const double* u)
     else
         TG_HIP(hipMemsetAsync(c->dval.p, 0, sizeof(double) * (size_t)c->msr_len, c->stream));
     if (c->formulation == TG_Q1P0) {
-        launch_q1p0(c, u, c->dR.p, true);
+        launch_q1p0_blocks(c, u);
+        launch_block_scatter(c);
         return;
     }
     for (const auto& fc : stiffness_launches(c)) {
@@ -1032,10 +1099,45 @@ void launch_stiffness(tg_ctx* c, const double* u)
     TG_HIP(hipGetLastError());
 }
 
+// The Q1P0 block buffer into the MSR through the slot map, colour by colour
+// (rows too wide for the gather by rows, or that assembly switched off): one
+// thread per upper entry, no two elements of a launch share one.
+__global__ void __launch_bounds__(256) k_block_scatter(const int* __restrict__ elems, int count,
+                                                       const unsigned* __restrict__ perm,
+                                                       const double* __restrict__ eb, const int* __restrict__ slot,
+                                                       double* __restrict__ val)
+{
+    const long t = (long)blockIdx.x * 256 + threadIdx.x;
+    if (t >= 324L * count) return;
+    const int e = elems[t / 324], x = (int)(t % 324);
+    const int p = x / 9, i = x % 9 / 3, j = x % 3;
+    int a, b;
+    upper_block(p, a, b);
+    const int m = 3 * a + i, n = 3 * b + j;
+    if (n < m) return;
+    const int s = slot_target(slot[300L * e + upper_index(m, n)]);
+    if (s < 0) return;
+    const int ra = rank_of(perm[e], a), rb = rank_of(perm[e], b);
+    val[s] += eb[324L * e + 9 * pair_index(min(ra, rb), max(ra, rb)) + (ra <= rb ? 3 * i + j : 3 * j + i)];
+}
+
+static void launch_block_scatter(tg_ctx* c)
+{
+    for (int col = 0; col < c->ncolors; col++) {
+        const int first = c->color_ptr[col], count = c->color_ptr[col + 1] - first;
+        if (count == 0) continue;
+        hipLaunchKernelGGL(k_block_scatter, dim3((unsigned)((324L * count + 255) / 256)), dim3(256), 0, c->stream,
+                           c->dcolor_elems.p + first, count, c->r_perm.p, c->r_blocks.p, c->dslot.p, c->dval.p);
+    }
+    TG_HIP(hipGetLastError());
+}
+
 // Newton's stiffness straight into the solver operator (total-Lagrangian
 // element): cleared values, the colour-ordered passes of TO_OP kernels.
 void launch_stiffness_operator(tg_ctx* c, const double* u)
 {
+    colour_structure(c);
+    c->op_fresh = false;
     TimedRegion tr(c, T_STIFFNESS);
     const bool mixed = c->precision == TG_MIXED;
     const size_t nv = (size_t)c->op.nblocks_padded * 9;
@@ -1143,6 +1245,26 @@ void launch_element_slots(tg_ctx* c)
                        c->dconn.p, c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, c->op.d_src.p,
                        c->dslot.p, c->op.d_oslot.n ? c->op.d_oslot.p : nullptr);
     TG_HIP(hipGetLastError());
+}
+
+// What the colour-ordered assembly needs: the colours and the slot maps,
+// built when it is first used on a mesh (the assembly by rows needs neither).
+void colour_structure(tg_ctx* c)
+{
+    if (c->colours_ready) return;
+    c->ncolors = color_elements(c->nnd, c->nel, c->conn.data(), c->color_ptr, c->color_elems);
+    c->dcolor_elems.alloc((size_t)c->nel);
+    TG_HIP(hipMemcpyAsync(c->dcolor_elems.p, c->color_elems.data(), sizeof(int) * c->nel, hipMemcpyHostToDevice,
+                          c->stream));
+    c->dslot.alloc(300 * (size_t)c->nel);
+    if (c->formulation == TG_TOTAL_LAGRANGIAN)
+        c->op.d_oslot.alloc(72 * (size_t)c->nel);
+    else
+        c->op.d_oslot.release();
+    launch_element_slots(c);
+    TG_HIP(hipStreamSynchronize(c->stream));
+    if (c->formulation == TG_Q1P0) rows_buffers(c);
+    c->colours_ready = true;
 }
 
 void launch_build_operator_diag(tg_ctx* c)

@@ -26,19 +26,26 @@ __global__ void k_ne_count(long n8, const int* __restrict__ conn, int* __restric
     if (k < n8) atomicAdd(&cnt[conn[k] + 1], 1);
 }
 
-// element of incidence k into its node's list (order within a list is
-// arbitrary; only sets are read from it)
+// incidence k into its node's list, as 8 element + the node's rank among the
+// element's nodes (order within a list is arbitrary here: only sets are read
+// from it until rows_structure sorts it)
 __global__ void k_ne_fill(long n8, const int* __restrict__ conn, int* __restrict__ fill, int* __restrict__ list)
 {
     const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n8) list[atomicAdd(&fill[conn[k]], 1)] = (int)(k >> 3);
+    if (k >= n8) return;
+    const int a = conn[k];
+    const int* c = conn + (k & ~7L);
+    int r = 0;
+#pragma unroll
+    for (int b = 0; b < 8; b++) r += c[b] < a;
+    list[atomicAdd(&fill[a], 1)] = (int)(k & ~7L) + r;
 }
 
 // candidate t of a node whose element list starts at p0: node t % 8 of the
 // (t / 8)-th element
 __device__ __forceinline__ int candidate(const int* conn, const int* list, int p0, int t)
 {
-    return conn[8L * list[p0 + (t >> 3)] + (t & 7)];
+    return conn[(long)(list[p0 + (t >> 3)] & ~7) + (t & 7)];
 }
 
 // FILL = false: deg[a] = the number of distinct candidates of node a (its

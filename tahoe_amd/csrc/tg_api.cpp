@@ -124,7 +124,17 @@ static void require_init(const tg_ctx* c)
 
 static void build_persist_list(tg_ctx* c);
 
-// Segment tables: slice -> segment, segment -> first slice, element -> segment.
+// segment of each slice
+std::vector<int> slice_segments(const tg_ctx* c)
+{
+    const Segments& S = c->seg;
+    std::vector<int> out((size_t)(c->nnd + 63) / 64, 0);
+    for (int g = 0; g < S.nseg; g++)
+        for (int s = S.node_begin[g] / 64; s < (S.node_begin[g + 1] + 63) / 64; s++) out[s] = g;
+    return out;
+}
+
+// Segment tables: slice -> segment, segment -> first slice and group.
 static void setup_segments(tg_ctx* c)
 {
     Segments& S = c->seg;
@@ -133,30 +143,25 @@ static void setup_segments(tg_ctx* c)
         S.node_begin = {0, c->nnd};
     }
     S.nslices = (c->nnd + 63) / 64;
-    std::vector<int> slice_seg((size_t)S.nslices), seg_slice((size_t)S.nseg + 1);
-    std::vector<int> node_seg((size_t)c->nnd);
-    for (int g = 0; g < S.nseg; g++) {
-        seg_slice[g] = S.node_begin[g] / 64;
-        for (int a = S.node_begin[g]; a < S.node_begin[g + 1]; a++) node_seg[a] = g;
-    }
+    std::vector<int> seg_slice((size_t)S.nseg + 1);
+    for (int g = 0; g < S.nseg; g++) seg_slice[g] = S.node_begin[g] / 64;
     seg_slice[S.nseg] = (int)S.nslices;
-    for (long s = 0; s < S.nslices; s++) slice_seg[s] = node_seg[64 * s];
-    S.elem_seg.resize((size_t)c->nel);
+    const std::vector<int> slice_seg = slice_segments(c);
+    // every element inside one segment
     int straddle = 0;
-    parallel_for(c->nel, [&](long b, long end) {
-        int bad = 0;
-        for (long e = b; e < end; e++) {
-            const int g = node_seg[c->conn[8 * e]];
-            for (int a = 1; a < 8; a++) bad |= node_seg[c->conn[8 * e + a]] != g;
-            S.elem_seg[e] = g;
-        }
-        if (bad) __atomic_store_n(&straddle, 1, __ATOMIC_RELAXED);
-    });
+    if (S.nseg > 1)
+        parallel_for(c->nel, [&](long b, long end) {
+            int bad = 0;
+            for (long e = b; e < end; e++) {
+                const int g = slice_seg[c->conn[8 * e] >> 6];
+                for (int a = 1; a < 8; a++) bad |= slice_seg[c->conn[8 * e + a] >> 6] != g;
+            }
+            if (bad) __atomic_store_n(&straddle, 1, __ATOMIC_RELAXED);
+        });
     if (straddle) fail(TG_BAD_INPUT, "element connects two segments");
     S.d_slice_seg.alloc((size_t)S.nslices);
     S.d_seg_slice.alloc((size_t)S.nseg + 1);
     S.d_active.alloc((size_t)S.nseg);
-    S.d_elem_seg.alloc((size_t)c->nel);
     S.d_scal.alloc((size_t)S_NSCAL * S.nseg);
     S.max_slices = 0;
     for (int g = 0; g < S.nseg; g++) S.max_slices = std::max(S.max_slices, (long)(seg_slice[g + 1] - seg_slice[g]));
@@ -186,7 +191,6 @@ static void setup_segments(tg_ctx* c)
     up(S.d_seg_grp.p, seg_grp);
     TG_HIP(hipMemcpyAsync(S.d_grp.p, grp.data(), sizeof(int4) * grp.size(), hipMemcpyHostToDevice, c->stream));
     up(S.d_active.p, ones);
-    up(S.d_elem_seg.p, S.elem_seg);
     TG_HIP(hipMemsetAsync(S.d_scal.p, 0, sizeof(double) * S_NSCAL * S.nseg, c->stream));
     TG_HIP(hipMemsetAsync(S.d_segstat.p, 0, sizeof(int) * S.nseg, c->stream));
     // every copy and clear of the context goes through its own stream (a
@@ -243,6 +247,21 @@ static void check_status(tg_ctx* c)
         clear_status(c);
         fail(code, "zero or negative jacobian");
     }
+}
+
+// ||R|| of the residual pass just launched; raises on an inverted element.
+// The norm and the flag come back together, written by the kernel that adds
+// the norm's partials: one wait.
+static double residual_norm(tg_ctx* c)
+{
+    launch_residual_result(c);
+    TG_HIP(hipStreamSynchronize(c->stream));
+    if (c->hscal[1] != 0.0) {
+        const int code = (int)c->hscal[1];
+        clear_status(c);
+        fail(code, "zero or negative jacobian");
+    }
+    return std::sqrt(c->hscal[0]);
 }
 
 // After a residual pass of a batch: the segments whose elements inverted
@@ -318,6 +337,7 @@ int tg_create(tg_ctx** out, int device)
         TG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         TG_HIP(hipHostMalloc((void**)&c->hscal, sizeof(double) * 16, hipHostMallocDefault));
         TG_HIP(hipHostMalloc((void**)&c->hstatus, sizeof(int) * 4, hipHostMallocDefault));
+        TG_HIP(hipHostMalloc((void**)&c->hstage, sizeof(double) * HOST_STAGE, hipHostMallocDefault));
         c->dstatus.alloc(4);
         TG_HIP(hipMemsetAsync(c->dstatus.p, 0, sizeof(int) * 4, c->stream));
         c->dscal.alloc(16);
@@ -355,6 +375,7 @@ int tg_destroy(tg_ctx* c)
         if (e) (void)hipEventDestroy(e);
     if (c->hscal) (void)hipHostFree(c->hscal);
     if (c->hstatus) (void)hipHostFree(c->hstatus);
+    if (c->hstage) (void)hipHostFree(c->hstage);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;  // DBuf destructors free device memory
     return TG_OK;
@@ -521,9 +542,7 @@ static void upload_mesh(tg_ctx* c, int nmat)
     c->dconn.alloc(8 * (size_t)c->nel);
     c->dmat.alloc((size_t)c->nel);
     c->deqn.alloc(nn);
-    c->dcolor_elems.alloc((size_t)c->nel);
     c->dmatprops.alloc((size_t)std::max(1, nmat));
-    c->dslot.alloc(300 * (size_t)c->nel);
     for (auto* v : {&c->vx, &c->vr, &c->vz, &c->vp, &c->vq, &c->vdinv, &c->vwork}) v->alloc(nn);
     const size_t sblocks = ((size_t)c->nnd + 255) / 256;
     c->dpart.alloc(2 * std::max<size_t>(sblocks, 1024) + 16);
@@ -574,9 +593,7 @@ int tg_initialize(tg_ctx* c, int* n_eq, long* msr_len)
         drop_pcg_graph(c);
         c->dfext.release();
         SetupTrace phase(c, "tg_initialize");
-        // equations; then the element colouring on a host thread of its own
-        // while this thread uploads the mesh and builds the structure on the
-        // device
+        // equations and segments on the host, then the structure on the device
         c->n_eq = equation_numbers(c->nnd, c->kbc_nodes, c->kbc_dofs, c->eqnos);
         phase("equation numbers");
         c->stiff_chunk_built = -2;
@@ -585,61 +602,29 @@ int tg_initialize(tg_ctx* c, int* n_eq, long* msr_len)
         c->dglist.release();
         c->debuf.release();
         c->debuf32.release();
-        {
-            std::exception_ptr colour_err, main_err;
-            using clk = std::chrono::steady_clock;
-            const auto t0 = clk::now();
-            clk::time_point t_colour, t_upload, t_graph;
-            std::thread colour([&] {
-                try {
-                    c->ncolors = color_elements(c->nnd, c->nel, c->conn.data(), c->color_ptr, c->color_elems);
-                } catch (...) {
-                    colour_err = std::current_exception();
-                }
-                t_colour = clk::now();
-            });
-            try {
-                upload_mesh(c, nmat);
-                t_upload = clk::now();
-                device_node_graph(c);
-                device_structure(c);
-                TG_HIP(hipStreamSynchronize(c->stream));
-                t_graph = clk::now();
-            } catch (...) {
-                main_err = std::current_exception();
-            }
-            colour.join();
-            for (auto& e : {main_err, colour_err})
-                if (e) std::rethrow_exception(e);
-            if (phase.on) {
-                auto ms = [&](clk::time_point t) { return std::chrono::duration<double, std::milli>(t - t0).count(); };
-                std::fprintf(stderr, "[tg_initialize]   upload %.1f ms, + device structure %.1f ms; colouring %.1f ms\n",
-                             ms(t_upload), ms(t_graph), ms(t_colour));
-            }
-        }
-        TG_HIP(hipMemcpyAsync(c->dcolor_elems.p, c->color_elems.data(), sizeof(int) * c->nel, hipMemcpyHostToDevice,
-                              c->stream));
+        c->colours_ready = false;
+        c->op_fresh = false;
+        setup_segments(c);
+        phase("segments");
+        upload_mesh(c, nmat);
+        phase("mesh upload");
+        device_node_graph(c);
+        device_structure(c);
         const bool mixed = mixed_operator(c);
-        phase("structure | colours");
         c->op.d_diag.alloc((size_t)c->nnd);
         launch_build_operator_diag(c);
-        if (c->formulation == TG_TOTAL_LAGRANGIAN)
-            c->op.d_oslot.alloc(72 * (size_t)c->nel);
-        else
-            c->op.d_oslot.release();
-        launch_element_slots(c);
+        rows_structure(c);
+        if (rows_assembly(c)) rows_buffers(c);
+        phase("structure");
         c->vbinv.alloc(c->precond == TG_PC_BLOCK_JACOBI ? 9 * (size_t)c->nnd : 0);
         c->op.d_val32.alloc(mixed || c->precond == TG_PC_AMG ? (size_t)c->op.nblocks_padded * 9 : 0);
-        phase("slot maps");
         if (c->precond == TG_PC_AMG) {
             amg_setup(c);
             phase("multigrid structure");
         } else {
             c->amg.clear();
         }
-        setup_segments(c);
         TG_HIP(hipStreamSynchronize(c->stream));
-        phase("segments");
         c->initialized = true;
         if (n_eq) *n_eq = c->n_eq;
         if (msr_len) *msr_len = c->msr_len;
@@ -762,11 +747,15 @@ int tg_form_rhs(tg_ctx* c, double* R_out, double* norm_out)
     if (!c) return TG_BAD_INPUT;
     return guarded(c, [&] {
         require_init(c);
-        launch_residual(c, c->du.p, c->dR.p);
-        if (norm_out || R_out) check_status(c);
-        if (norm_out) *norm_out = std::sqrt(device_dot(c, c->dR.p, c->dR.p, 3L * c->nnd));
-        if (R_out) {
-            node_to_eq(c, c->dR.p, c->vwork.p);
+        // a short result goes straight to the host staging buffer
+        const bool stage = R_out && (size_t)c->n_eq <= HOST_STAGE;
+        launch_residual(c, c->du.p, c->dR.p, !R_out ? nullptr : stage ? c->hstage : c->vwork.p);
+        if (!norm_out && !R_out) return;
+        const double norm = residual_norm(c);
+        if (norm_out) *norm_out = norm;
+        if (stage) {
+            std::memcpy(R_out, c->hstage, sizeof(double) * c->n_eq);
+        } else if (R_out) {
             TG_HIP(hipMemcpyAsync(R_out, c->vwork.p, sizeof(double) * c->n_eq, hipMemcpyDeviceToHost, c->stream));
             TG_HIP(hipStreamSynchronize(c->stream));
         }
@@ -805,7 +794,10 @@ static void prepare_preconditioner(tg_ctx* c)
 // is expanded (1/diag from the FP64 diagonal) and then narrowed
 static void prepare_operator(tg_ctx* c)
 {
-    if (mixed_stiffness(c)) {
+    if (c->op_fresh) {
+        // written with the MSR values by the assembly by rows
+        TimedRegion tr(c, T_EXPAND);
+    } else if (mixed_stiffness(c)) {
         launch_expand32(c);
     } else {
         launch_expand(c);
@@ -818,7 +810,7 @@ static void prepare_operator(tg_ctx* c)
 // operator (total-Lagrangian), or assembled into the MSR and expanded.
 static void newton_operator(tg_ctx* c)
 {
-    if (c->formulation == TG_TOTAL_LAGRANGIAN && c->newton_assembly == 1 && c->op.d_oslot.p) {
+    if (c->formulation == TG_TOTAL_LAGRANGIAN && c->newton_assembly == 1) {
         launch_stiffness_operator(c, c->du.p);
         launch_operator_dinv(c);
         prepare_preconditioner(c);
@@ -870,7 +862,7 @@ int tg_multx(tg_ctx* c, const double* x, double* b)
         fp64_values(c);
         TG_HIP(hipMemcpyAsync(c->vwork.p, x, sizeof(double) * c->n_eq, hipMemcpyHostToDevice, c->stream));
         eq_to_node(c, c->vwork.p, c->vx.p);
-        launch_expand(c);
+        if (!(c->op_fresh && !mixed_operator(c))) launch_expand(c);
         launch_spmv(c, c->vx.p, c->vq.p);
         node_to_eq(c, c->vq.p, c->vwork.p);
         TG_HIP(hipMemcpyAsync(b, c->vwork.p, sizeof(double) * c->n_eq, hipMemcpyDeviceToHost, c->stream));
@@ -968,8 +960,7 @@ int tg_solve_noalloc(tg_ctx* c, const double* b_dev, double* x_dev, double rtol,
 static void correction(tg_ctx* c, const tg_newton_opts* o, double* err_before, long* lin_its)
 {
     launch_residual(c, c->du.p, c->dR.p);
-    check_status(c);
-    *err_before = std::sqrt(device_dot(c, c->dR.p, c->dR.p, 3L * c->nnd));
+    *err_before = residual_norm(c);
     newton_operator(c);
     tg_lin_stats st{};
     solve_linear(c, c->dR.p, c->vx.p, o->lin_rtol, o->lin_maxit, &st);
@@ -1009,8 +1000,7 @@ int tg_newton(tg_ctx* c, const tg_newton_opts* o, tg_newton_stats* s)
     int rc = guarded(c, [&] {
         require_init(c);
         launch_residual(c, c->du.p, c->dR.p);
-        check_status(c);
-        const double err0 = std::sqrt(device_dot(c, c->dR.p, c->dR.p, 3L * c->nnd));
+        const double err0 = residual_norm(c);
         out.error0 = out.error = err0;
         if (err0 < o->abs_tolerance) return;
         int iter = -1;
@@ -1024,8 +1014,7 @@ int tg_newton(tg_ctx* c, const tg_newton_opts* o, tg_newton_stats* s)
             launch_axpy(c, c->du.p, c->vx.p, 1.0, 3L * c->nnd);
             iter++;
             launch_residual(c, c->du.p, c->dR.p);
-            check_status(c);
-            const double err = std::sqrt(device_dot(c, c->dR.p, c->dR.p, 3L * c->nnd));
+            const double err = residual_norm(c);
             out.error = err;
             out.iterations = iter + 1;
             out.lin_iterations = lin;
@@ -1170,12 +1159,15 @@ int tg_set_tuning(tg_ctx* c, int knob, long value)
         if (knob == TG_TUNE_STIFF_CHUNK) {
             if (value < -1) fail(TG_BAD_INPUT, "stiffness chunk must be -1, 0 or positive");
             c->stiff_chunk = value;
+            c->stiff_explicit = true;
         } else if (knob == TG_TUNE_STIFF_SHAPE) {
             if (value < 0 || value > 18) fail(TG_OUT_OF_RANGE, "stiffness shape must be 0..18");
             c->stiff_variant = (int)value;
+            c->stiff_explicit = true;
         } else if (knob == TG_TUNE_NEWTON_ASSEMBLY) {
             if (value < 0 || value > 1) fail(TG_OUT_OF_RANGE, "Newton assembly must be 0 or 1");
             c->newton_assembly = (int)value;
+            c->stiff_explicit = true;
         } else if (knob == TG_TUNE_PCG_GRAPH) {
             if (value < 0 || value > 1) fail(TG_OUT_OF_RANGE, "PCG graph must be 0 or 1");
             c->pcg_graph = (int)value;
@@ -1197,6 +1189,7 @@ int tg_set_tuning(tg_ctx* c, int knob, long value)
         } else if (knob == TG_TUNE_STIFF_GATHER) {
             if (value < 0 || value > 1) fail(TG_OUT_OF_RANGE, "stiffness gather must be 0 or 1");
             c->stiff_gather = (int)value;
+            c->stiff_explicit = true;
         } else if (knob == TG_TUNE_AMG_DEGREE) {
             if (value < 2 || value > 4) fail(TG_OUT_OF_RANGE, "multigrid smoother degree must be 2..4");
             c->amg.degree = (int)value;
@@ -1207,6 +1200,9 @@ int tg_set_tuning(tg_ctx* c, int knob, long value)
             c->amg.weight = (int)value;
             c->amg.gen++;
             c->amg.since = -1;
+        } else if (knob == TG_TUNE_STIFF_ROWS) {
+            if (value < 0 || value > 1) fail(TG_OUT_OF_RANGE, "assembly by rows must be 0 or 1");
+            c->stiff_explicit = value == 0;
         } else
             fail(TG_BAD_INPUT, "unknown tuning knob " + std::to_string(knob));
     });
@@ -1230,6 +1226,8 @@ int tg_get_tuning(tg_ctx* c, int knob, long* value)
             *value = pcg_fused(c) ? 1 : 0;
         else if (knob == TG_TUNE_STIFF_GATHER)
             *value = c->stiff_gather;
+        else if (knob == TG_TUNE_STIFF_ROWS)
+            *value = rows_assembly(c) ? 1 : 0;
         else if (knob == TG_TUNE_PCG_PERSIST)
             *value = pcg_persist(c);
         else if (knob == TG_TUNE_AMG_REUSE)

@@ -36,6 +36,12 @@ __device__ __forceinline__ void reduce_scatter8(const double r[24], int q, doubl
 // Position of (m, n), m <= n < 24, in the packed upper triangle.
 __device__ __forceinline__ int upper_index(int m, int n) { return m * 24 - (m * (m - 1)) / 2 + (n - m); }
 
+// rank of local node a among its element's nodes (k_rows.hip: 4 bits each)
+__device__ __forceinline__ int rank_of(unsigned perm, int a) { return (int)(perm >> (4 * a)) & 7; }
+
+// place of rank pair (r, s), r <= s, among the 36: row r holds 8 - r pairs
+__device__ __forceinline__ int pair_index(int r, int s) { return r * 8 - (r * (r - 1)) / 2 + (s - r); }
+
 // The element slot map holds, per element upper entry, the MSR value index
 // s, or -s-2 where that entry is the first contribution to s in the
 // stiffness launch order (the values are cleared before the passes, so the

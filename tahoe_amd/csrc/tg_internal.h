@@ -51,6 +51,10 @@ struct GraphWork {
     std::vector<std::vector<int>> stamp;
 };
 
+// doubles of the pinned buffer that kernels write short results to directly;
+// a longer one is faster as a copy after the kernel
+constexpr size_t HOST_STAGE = 16384;
+
 // Status raised inside the library; converted to the C status at the ABI.
 struct Error {
     int code;
@@ -258,13 +262,11 @@ struct Segments {
     long max_slices = 0;                  // slices of the largest segment
     long ngroups = 0;                     // groups of up to 4 slices of one segment
     std::vector<int> node_begin;          // [nseg+1]
-    std::vector<int> elem_seg;            // [nel] segment of each element (host)
     DBuf<int> d_slice_seg;                // [nslices]
     DBuf<int> d_seg_slice;                // [nseg+1] first slice of each segment
     DBuf<int> d_seg_grp;                  // [nseg+1] first group of each segment
     DBuf<int4> d_grp;                     // [ngroups] (first slice, slices, segment, 0)
     DBuf<int> d_active;                   // [nseg] 1 = solve this segment
-    DBuf<int> d_elem_seg;                 // [nel]
     DBuf<double> d_scal;                  // [S_NSCAL][nseg]
     DBuf<double> d_part;                  // [3][nslices]: r.z, r.r, p.q
     DBuf<double> d_out;                   // [nseg]
@@ -311,6 +313,18 @@ struct tg_ctx {
     tg::DBuf<int> g_neptr, g_nelist, g_fill, g_flag, g_nlist;
     tg::DBuf<long long> g_deg, g_nptr, g_rowlen, g_rows, g_most;
     tg::DBuf<unsigned char> g_scan;
+    // assembly by rows (k_rows.hip)
+    tg::DBuf<unsigned> r_perm;          // [nel] ranks of the element's nodes, 4 bits each
+    tg::DBuf<int2> r_upper;             // [nnd] slot of the row's diagonal block, upper blocks of the row
+    tg::DBuf<unsigned char> r_slot;     // [nel][8][8] upper slot of block (rank r, rank r + j) in the row of rank r
+    int r_up_most = 0;                  // most upper blocks of a row
+    tg::DBuf<double> r_force;           // [nel][8][3] element forces, by rank
+    tg::DBuf<double> r_blocks;          // [nel][36][9] element stiffness blocks
+    tg::DBuf<float> r_blocks32;
+    tg::DBuf<double> dpart_r;           // partials of R.R
+    bool stiff_explicit = false;        // a knob of the colour-ordered assembly was set: it runs
+    bool colours_ready = false;         // colours and slot maps of this mesh are built
+    bool op_fresh = false;              // operator and 1/diag are those of the MSR values
     // stiffness launch order: every segment's elements in ranges of
     // stiff_chunk (by rank inside the segment), all colours of range j
     // before range j+1 (0: whole colours)
@@ -368,6 +382,7 @@ struct tg_ctx {
     tg::DBuf<int> dstatus;              // device error flag (7 = bad Jacobian)
     double* hscal = nullptr;            // pinned host mirror of a few scalars
     int* hstatus = nullptr;
+    double* hstage = nullptr;           // pinned [HOST_STAGE]: short results a kernel writes to the host
 
     // Q1P0 per-element history
     tg::DBuf<double> dvol, dvol_last;
@@ -453,7 +468,18 @@ void device_node_graph(tg_ctx* c);
 void device_structure(tg_ctx* c);
 
 // kernels launched from the ABI (k_element.hip, k_solver.hip)
-void launch_residual(tg_ctx* c, const double* u, double* R_node);
+// R into R_node and, given, its active entries in equation order into R_eq
+void launch_residual(tg_ctx* c, const double* u, double* R_node, double* R_eq = nullptr);
+// assembly by rows (k_rows.hip)
+void rows_structure(tg_ctx* c);
+void rows_buffers(tg_ctx* c);
+bool rows_assembly(const tg_ctx* c);
+void launch_node_residual(tg_ctx* c, double* R_node, double* R_eq);
+// ||R||^2 of the last launch_residual and the status flag into hscal[0, 1]
+void launch_residual_result(tg_ctx* c);
+void launch_gather_rows(tg_ctx* c);
+void colour_structure(tg_ctx* c);
+std::vector<int> slice_segments(const tg_ctx* c);
 void launch_stiffness(tg_ctx* c, const double* u);
 // gather lists of the element-buffer assembly (k_gather.hip) for the
 // current launch order; dorder = elements in launch order
