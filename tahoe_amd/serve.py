@@ -33,7 +33,9 @@ from . import api, batch
 def footprint_bytes(req, precision=api.MIXED) -> int:
     """Device bytes of one request inside a batch context (upper bound for
     a cube of L^3 hexes): per element the 300-entry MSR slot map, the 72-entry
-    operator slot map, connectivity, material and colour lists; per node the
+    operator slot map (either these two or the row assembly's slots, block and
+    force buffers, which are smaller together), connectivity, material and
+    element lists; per node the
     upper MSR pattern and values (<= 123 entries), 27 operator blocks (column,
     9 FP64 values, 9 FP32 values in mixed precision, 9-entry expansion map)
     and about a dozen node-space vectors."""
@@ -117,8 +119,14 @@ def solve_request(req, precision, opts, device=0, log=None, precond=None, one_st
 
 class RVEServer:
     def __init__(self, precision=api.MIXED, workers=6, max_batch=32, budget_bytes=64 << 30, lin_rtol=None,
-                 device=0, keep_u=True, on_batch=None, log=None, reuse_contexts=True):
+                 device=0, keep_u=True, on_batch=None, log=None, reuse_contexts=True, linger=0.003):
         self.precision = precision
+        # while another worker solves, a mini-batch that is not full waits up
+        # to `linger` seconds for requests of its kind: a request joined costs
+        # the batch little, on its own it costs a whole set-up and launch
+        # chain.  An idle server starts at once.
+        self.linger = linger
+        self._solving = 0
         # each worker keeps one context per (formulation, size class,
         # preconditioner) alive between batches and sets it up again for the
         # next batch (batch.configure): no allocation once the kind's largest
@@ -154,29 +162,41 @@ class RVEServer:
         whose footprint fits the remaining budget; None if nothing fits."""
         if not self._queue:
             return None
-        head = self._queue[0]
-        form = head.formulation
-        picked, size = [], 0
-        for r in list(self._queue):
-            if r.formulation != form or size_class(r) != size_class(head):
-                continue
-            fb = footprint_bytes(r, self.precision)
-            if self._in_use + size + fb > self.budget and picked:
-                break
-            if self._in_use + size + fb > self.budget and self._in_use > 0:
-                break  # wait for memory to free up
-            picked.append(r)
-            size += fb
-            if len(picked) >= self.max_batch:
-                break
+        picked = []
+        size = self._extend_batch(self._queue[0], picked)
         if not picked:
             return None
-        for r in picked:
-            self._queue.remove(r)
-        self._in_use += size
         bid = self._next_batch
         self._next_batch += 1
+        self._solving += 1
+        end = time.perf_counter() + self.linger
+        while len(picked) < self.max_batch and self._solving > 1 and not self._closed:
+            left = end - time.perf_counter()
+            if left <= 0:
+                break
+            self._lock.wait(timeout=left)
+            size += self._extend_batch(picked[0], picked)
         return bid, picked, size
+
+    def _extend_batch(self, head, picked):
+        """Move queued requests of head's formulation and size class into
+        picked, up to max_batch and the budget; returns their footprint."""
+        size = 0
+        for r in list(self._queue):
+            if len(picked) >= self.max_batch:
+                break
+            if r.formulation != head.formulation or size_class(r) != size_class(head):
+                continue
+            fb = footprint_bytes(r, self.precision)
+            # a request beyond the budget waits for memory to free up, unless
+            # nothing else is admitted
+            if self._in_use + fb > self.budget and self._in_use > 0:
+                break
+            picked.append(r)
+            self._queue.remove(r)
+            self._in_use += fb
+            size += fb
+        return size
 
     # -- worker ---------------------------------------------------------
     def _solve_group(self, reqs):
@@ -275,6 +295,7 @@ class RVEServer:
             finally:
                 with self._lock:
                     self._in_use -= size
+                    self._solving -= 1
                     self._lock.notify_all()
             with self._lock:
                 for x in res:
