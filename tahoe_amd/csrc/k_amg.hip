@@ -4,7 +4,7 @@
 // Smoother: Chebyshev polynomial in D^-1 A (Adams, Brezina, Hu and
 // Tuminaro, J. Comput. Phys. 188 (2003) 593-610; the three-term recurrence
 // of Saad, Iterative Methods for Sparse Linear Systems, Alg. 12.1) on
-// [lmax / 30, lmax], with lmax a power-iteration estimate of the largest
+// [lmax / 14, lmax], with lmax a power-iteration estimate of the largest
 // eigenvalue of D^-1 A raised by 10 %.  Pre- and post-smoothing use the same
 // polynomial and the coarse correction is a Galerkin product, so the V-cycle
 // is a symmetric positive definite preconditioner for CG.  Matrices below
@@ -20,7 +20,11 @@ namespace tg {
 namespace {
 
 constexpr int AB = 256;          // threads per block of the vector/level kernels
-constexpr double CHEB_RATIO = 30.0;
+// Smoothing interval [lmax / CHEB_RATIO, lmax]: the coarse levels take what
+// lies below.  PCG iterations of one Newton step (128^3 mixed / 64^3 FP64 / 24^3
+// to 1e-10): ratio 30 94 / 82 / 141, 16 87 / 78 / 132, 12 87 / 78 / 131, 8 91 /
+// 80 / 133, 4 101 / 87 / 148.
+constexpr double CHEB_RATIO = 14.0;
 constexpr double CHEB_BOOST = 1.1;
 constexpr int POWER_ITS = 12;
 
@@ -28,44 +32,46 @@ inline unsigned blocks_for(long n) { return (unsigned)((n + AB - 1) / AB); }
 
 __device__ __forceinline__ bool skip(const double* done) { return done && *done != 0.0; }
 
-// Level 0: the solver's sliced-ELL operator (3x3 blocks), one thread per node.
-template <class MT>
+// Level 0: the solver's sliced-ELL operator (3x3 blocks), one lane per node.
+// add: y += the products of slots k0 .. k1 - 1 of the row of node t (lane l of
+// the slice at b0).  Padding slots (column -1) hold zeros and multiply the
+// row's own entries, so no branch stands between the loads.  SYM: a lower
+// block is read as its upper partner's transpose (k_pcg.hip, block_values).
+template <class MT, bool SYM>
 struct Op0 {
     static constexpr int NC = 3;
     int n;
     const int* sbase;
     const int* swidth;
     const int* col;
+    const int* tpos;
     const MT* val;
-    __host__ __device__ long units() const { return n; }
-    __device__ __forceinline__ void apply(long t, const double* __restrict__ x, double (&y)[3], long (&k)[3]) const
+    __device__ __forceinline__ void add(long b0, int k0, int k1, int l, int t, const double* __restrict__ x, double (&y)[3]) const
     {
-        const int s = (int)(t >> 6), l = (int)(t & 63);
-        const long b0 = sbase[s];
-        const int w = swidth[s];
-        double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-        for (int q = 0; q < w; q++) {
+#pragma unroll 3
+        for (int q = k0; q < k1; q++) {
             const long blk = b0 + q;
-            const int c = col[blk * 64 + l];
-            if (c < 0) continue;
-            const double x0 = x[3L * c], x1 = x[3L * c + 1], x2 = x[3L * c + 2];
-            const MT* v = val + blk * 576 + l;
-            y0 += (double)v[0] * x0 + (double)v[64] * x1 + (double)v[128] * x2;
-            y1 += (double)v[192] * x0 + (double)v[256] * x1 + (double)v[320] * x2;
-            y2 += (double)v[384] * x0 + (double)v[448] * x1 + (double)v[512] * x2;
+            const int cr = col[blk * 64 + l];
+            const int c = cr < 0 ? t : cr;
+            const bool tr = SYM && c < t;
+            long at = blk * 576 + l;
+            if (tr) at = tpos[blk * 64 + l];
+            double u[9], xc[3];
+#pragma unroll
+            for (int m = 0; m < 9; m++) u[m] = (double)val[at + 64 * m];
+#pragma unroll
+            for (int j = 0; j < 3; j++) xc[j] = x[3L * c + j];
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) y[r] += (tr ? u[3 * j + r] : u[3 * r + j]) * xc[j];
         }
-        y[0] = y0;
-        y[1] = y1;
-        y[2] = y2;
-        k[0] = 3 * t;
-        k[1] = 3 * t + 1;
-        k[2] = 3 * t + 2;
     }
 };
 
 // Levels >= 1: sliced 6x6 FP32 blocks (slot e of a slice: its 36 values at
 // val[(e / 64) * 2304 + comp * 64 + e % 64], coalesced over the slice's 64
-// rows), one thread per node and 6 outputs.
+// rows; padding zero), one lane per node and 6 outputs.
 struct OpC {
     static constexpr int NC = 6;
     int n;
@@ -73,18 +79,11 @@ struct OpC {
     const int* swidth;
     const int* col;
     const float* val;
-    __host__ __device__ long units() const { return n; }
-    __device__ __forceinline__ void apply(long t, const double* __restrict__ x, double (&y)[6], long (&k)[6]) const
+    __device__ __forceinline__ void add(long b0, int k0, int k1, int l, int t, const double* __restrict__ x, double (&y)[6]) const
     {
-        const int s = (int)(t >> 6), l = (int)(t & 63);
-        const long b0 = sbase[s];
-        const int w = swidth[s];
-#pragma unroll
-        for (int r = 0; r < 6; r++) y[r] = 0.0;
-        for (int q = 0; q < w; q++) {
-            const long slot = (b0 + q) * 64 + l;
-            const int c = col[slot];
-            if (c < 0) continue;
+        for (int q = k0; q < k1; q++) {
+            const int cr = col[(b0 + q) * 64 + l];
+            const int c = cr < 0 ? t : cr;
             double xc[6];
 #pragma unroll
             for (int j = 0; j < 6; j++) xc[j] = x[6L * c + j];
@@ -94,107 +93,113 @@ struct OpC {
 #pragma unroll
                 for (int j = 0; j < 6; j++) y[r] += (double)v[(6 * r + j) * 64] * xc[j];
         }
-#pragma unroll
-        for (int r = 0; r < 6; r++) k[r] = 6 * t + r;
     }
 };
 
-// y = A x
-template <class Op>
-__global__ void __launch_bounds__(AB) k_amg_spmv(Op op, const double* __restrict__ x, double* __restrict__ y)
-{
-    const long t = (long)blockIdx.x * AB + threadIdx.x;
-    if (t >= op.units()) return;
-    double q[Op::NC];
-    long k[Op::NC];
-    op.apply(t, x, q, k);
-#pragma unroll
-    for (int i = 0; i < Op::NC; i++) y[k[i]] = q[i];
-}
-
-// Chebyshev step s >= 1: r -= A d_prev; d_next = c1 d_prev + c2 D^-1 r;
-// x += d_next (+ d_prev when the pass started from a nonzero x)
-template <class Op>
-__global__ void __launch_bounds__(AB) k_amg_step(Op op, const double* __restrict__ dinv,
-                                                 const double* __restrict__ dprev, double* __restrict__ dnext,
-                                                 double* __restrict__ r, double* __restrict__ x,
-                                                 const double* __restrict__ coef, int ci, int add_prev,
-                                                 const double* done)
-{
-    if (skip(done)) return;
-    const long t = (long)blockIdx.x * AB + threadIdx.x;
-    if (t >= op.units()) return;
-    double q[Op::NC];
-    long k[Op::NC];
-    op.apply(t, dprev, q, k);
-    const double c1 = coef[ci], c2 = coef[ci + 1];
-#pragma unroll
-    for (int i = 0; i < Op::NC; i++) {
-        const long j = k[i];
-        const double ri = r[j] - q[i];
+// what follows a product q at dof j
+struct EStore {  // y = A x
+    double* y;
+    __device__ __forceinline__ void operator()(long j, double q) const { y[j] = q; }
+};
+// Chebyshev step: r -= A d_prev; d_next = c1 d_prev + c2 D^-1 r; x += d_next
+// (+ d_prev when the pass started from a nonzero x)
+struct EStep {
+    const double *dinv, *dprev, *coef;
+    double *dnext, *r, *x;
+    int ci, add_prev;
+    __device__ __forceinline__ void operator()(long j, double q) const
+    {
+        const double ri = r[j] - q, dp = dprev[j];
         r[j] = ri;
-        const double dn = c1 * dprev[j] + c2 * dinv[j] * ri;
+        const double dn = coef[ci] * dp + coef[ci + 1] * dinv[j] * ri;
         dnext[j] = dn;
-        x[j] += (add_prev ? dprev[j] : 0.0) + dn;
+        x[j] += (add_prev ? dp : 0.0) + dn;
     }
-}
-
-// r -= A d
-template <class Op>
-__global__ void __launch_bounds__(AB) k_amg_resid(Op op, const double* __restrict__ d, double* __restrict__ r,
-                                                  const double* done)
-{
-    if (skip(done)) return;
-    const long t = (long)blockIdx.x * AB + threadIdx.x;
-    if (t >= op.units()) return;
-    double q[Op::NC];
-    long k[Op::NC];
-    op.apply(t, d, q, k);
-#pragma unroll
-    for (int i = 0; i < Op::NC; i++) r[k[i]] -= q[i];
-}
-
-// start of post-smoothing: r = f - A x; d0 = D^-1 r / theta
-template <class Op>
-__global__ void __launch_bounds__(AB) k_amg_post(Op op, const double* __restrict__ dinv, const double* __restrict__ f,
-                                                 const double* __restrict__ x, double* __restrict__ r,
-                                                 double* __restrict__ d0, const double* __restrict__ coef,
-                                                 const double* done)
-{
-    if (skip(done)) return;
-    const long t = (long)blockIdx.x * AB + threadIdx.x;
-    if (t >= op.units()) return;
-    double q[Op::NC];
-    long k[Op::NC];
-    op.apply(t, x, q, k);
-    const double ith = coef[0];
-#pragma unroll
-    for (int i = 0; i < Op::NC; i++) {
-        const long j = k[i];
-        const double ri = f[j] - q[i];
+};
+// the first step of a pass from zero, d0 = D^-1 f / theta (k_amg_pre): r = f -
+// A d0, then as above with x = d0 + d1
+struct EFirst {
+    const double *dinv, *f, *coef, *d0;
+    double *dnext, *r, *x;
+    __device__ __forceinline__ void operator()(long j, double q) const
+    {
+        const double ri = f[j] - q, dp = d0[j];
         r[j] = ri;
-        d0[j] = ith * dinv[j] * ri;
+        const double dn = coef[1] * dp + coef[2] * dinv[j] * ri;
+        dnext[j] = dn;
+        x[j] = dp + dn;
     }
+};
+struct EResid {  // r -= A d
+    double* r;
+    __device__ __forceinline__ void operator()(long j, double q) const { r[j] -= q; }
+};
+struct EPost {  // start of post-smoothing: r = f - A x; d0 = D^-1 r / theta
+    const double *dinv, *f, *coef;
+    double *r, *d0;
+    __device__ __forceinline__ void operator()(long j, double q) const
+    {
+        const double ri = f[j] - q;
+        r[j] = ri;
+        d0[j] = coef[0] * dinv[j] * ri;
+    }
+};
+
+// A product with a level's operator and what follows it.  NW = 1: a lane per
+// row, four slices a workgroup; NW > 1: a slice a workgroup, its waves share
+// the row's slots and wave 0 adds their sums in order (the coarse levels have
+// few rows: at 128^3, 72, 12 and 2 slices took 30-40 us a product with a lane
+// per row, each walking 27 blocks of 36 values, and take 6-8 shared; 544
+// slices 38 and 27).  Each XCD takes a contiguous range of slices.  The two
+// large levels are bound by what passes the L2s: 2.15 M nodes FP32 (2.3 GB, the
+// lower z layer's blocks twice) 452 us, 270 k nodes of 6 dofs (1.07 GB) 236 us.
+template <class Op, int NW, class E>
+__global__ void __launch_bounds__(NW == 1 ? AB : 64 * NW) k_amg_rows(Op op, const double* __restrict__ x, E e,
+                                                                      const double* done)
+{
+    if (skip(done)) return;
+    const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int s = NW == 1 ? b * (AB / 64) + wv : b;
+    if (s >= (op.n + 63) >> 6) return;
+    const int t = 64 * s + l;
+    const bool own = t < op.n;
+    const long b0 = op.sbase[s];
+    const int w = op.swidth[s];
+    const int per = NW == 1 ? w : (w + NW - 1) / NW;
+    double q[Op::NC];
+#pragma unroll
+    for (int i = 0; i < Op::NC; i++) q[i] = 0.0;
+    op.add(b0, NW == 1 ? 0 : wv * per, NW == 1 ? w : min(w, (wv + 1) * per), l, own ? t : 0, x, q);
+    if (NW > 1) {
+        __shared__ double red[NW][Op::NC][64];
+#pragma unroll
+        for (int i = 0; i < Op::NC; i++) red[wv][i][l] = q[i];
+        __syncthreads();
+        if (wv > 0) return;
+        for (int j = 1; j < NW; j++)
+#pragma unroll
+            for (int i = 0; i < Op::NC; i++) q[i] += red[j][i][l];
+    }
+    if (own)
+#pragma unroll
+        for (int i = 0; i < Op::NC; i++) e((long)Op::NC * t + i, q[i]);
 }
 
-// start of pre-smoothing from x = 0: r = f; d0 = x = D^-1 f / theta
+// first direction of a smoothing pass from zero
 __global__ void __launch_bounds__(AB) k_amg_pre(long nd, const double* __restrict__ dinv, const double* __restrict__ f,
-                                                double* __restrict__ r, double* __restrict__ d0,
-                                                double* __restrict__ x, const double* __restrict__ coef,
+                                                const double* __restrict__ coef, double* __restrict__ d0,
                                                 const double* done)
 {
     if (skip(done)) return;
     const long j = (long)blockIdx.x * AB + threadIdx.x;
-    if (j >= nd) return;
-    const double fj = f[j];
-    const double d = coef[0] * dinv[j] * fj;
-    r[j] = fj;
-    d0[j] = d;
-    x[j] = d;
+    if (j < nd) d0[j] = coef[0] * dinv[j] * f[j];
 }
 
-// fc[A][c] = sum over members i of A of P_i^T r_i
-__global__ void __launch_bounds__(AB) k_amg_restrict(int nc, int bs, const int* __restrict__ mptr,
+// fc[A][c] = sum over members i of A of P_i^T r_i, four members' loads at a
+// time
+template <int BS>
+__global__ void __launch_bounds__(AB) k_amg_restrict(int nc, const int* __restrict__ mptr,
                                                      const int* __restrict__ mem, const float* __restrict__ P,
                                                      const double* __restrict__ r, double* __restrict__ fc,
                                                      const double* done)
@@ -203,43 +208,66 @@ __global__ void __launch_bounds__(AB) k_amg_restrict(int nc, int bs, const int* 
     const long t = (long)blockIdx.x * AB + threadIdx.x;
     if (t >= 6L * nc) return;
     const int a = (int)(t / 6), c = (int)(t - 6L * a);
+    const int m1 = mptr[a + 1];
     double s = 0.0;
-    for (int m = mptr[a]; m < mptr[a + 1]; m++) {
-        const int i = mem[m];
-        const float* p = P + (long)i * bs * 6 + c;
-        const double* ri = r + (long)i * bs;
-        for (int q = 0; q < bs; q++) s += (double)p[6 * q] * ri[q];
+    for (int m = mptr[a]; m < m1; m += 4) {
+        float p[4][BS];
+        double v[4][BS];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = mem[min(m + u, m1 - 1)];
+#pragma unroll
+            for (int q = 0; q < BS; q++) {
+                p[u][q] = P[(long)i * BS * 6 + 6 * q + c];
+                v[u][q] = r[(long)i * BS + q];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (m + u < m1)
+#pragma unroll
+                for (int q = 0; q < BS; q++) s += (double)p[u][q] * v[u][q];
     }
     fc[t] = s;
 }
 
 // x_i += w P_i xc[agg(i)]
-__global__ void __launch_bounds__(AB) k_amg_prolong(int n, int bs, const int* __restrict__ agg,
+template <int BS>
+__global__ void __launch_bounds__(AB) k_amg_prolong(int n, const int* __restrict__ agg,
                                                     const float* __restrict__ P, const double* __restrict__ xc,
                                                     double w, double* __restrict__ x, const double* done)
 {
     if (skip(done)) return;
     const long t = (long)blockIdx.x * AB + threadIdx.x;
-    if (t >= (long)n * bs) return;
-    const int i = (int)(t / bs), q = (int)(t - (long)i * bs);
+    if (t >= (long)n * BS) return;
+    const int i = (int)(t / BS);
     const int a = agg[i];
+    const float* p = P + 6 * t;
+    const double xt = x[t];
     if (a < 0) return;
-    const float* p = P + (long)i * bs * 6 + 6 * q;
     const double* e = xc + 6L * a;
-    x[t] += w * ((double)p[0] * e[0] + (double)p[1] * e[1] + (double)p[2] * e[2] + (double)p[3] * e[3] +
-                 (double)p[4] * e[4] + (double)p[5] * e[5]);
+    x[t] = xt + w * ((double)p[0] * e[0] + (double)p[1] * e[1] + (double)p[2] * e[2] + (double)p[3] * e[3] +
+                     (double)p[4] * e[4] + (double)p[5] * e[5]);
 }
 
-// coarsest level: x = C^-1 f (C^-1 dense, symmetric, column-major)
-__global__ void __launch_bounds__(AB) k_amg_dense(int n, const double* __restrict__ cinv, const double* __restrict__ f,
-                                                  double* __restrict__ x, const double* done)
+// coarsest level: x = C^-1 f (C^-1 dense, symmetric, column-major); a row's
+// columns in four parts, added in order
+__global__ void __launch_bounds__(4 * AB) k_amg_dense(int n, const double* __restrict__ cinv,
+                                                      const double* __restrict__ f, double* __restrict__ x,
+                                                      const double* done)
 {
     if (skip(done)) return;
-    const int r = blockIdx.x * AB + threadIdx.x;
-    if (r >= n) return;
+    __shared__ double red[3][AB];
+    const int t = threadIdx.x & (AB - 1), part = threadIdx.x / AB;
+    const int r = blockIdx.x * AB + t;
+    const int per = (n + 3) / 4, c1 = min(n, (part + 1) * per);
     double s = 0.0;
-    for (int c = 0; c < n; c++) s += cinv[(long)c * n + r] * f[c];
-    x[r] = s;
+    if (r < n)
+#pragma unroll 8
+        for (int c = part * per; c < c1; c++) s += cinv[(long)c * n + r] * f[c];
+    if (part > 0) red[part - 1][t] = s;
+    __syncthreads();
+    if (part == 0 && r < n) x[r] = ((s + red[0][t]) + red[1][t]) + red[2][t];
 }
 
 // Galerkin product, fine level = the sliced-ELL operator: one wave per
@@ -256,6 +284,7 @@ __global__ void __launch_bounds__(AB) k_amg_rap0(long nup, const int* __restrict
     if (u >= nup || lane >= 36) return;
     const int r = lane / 6, c = lane - 6 * (lane / 6);
     double s = 0.0;
+#pragma unroll 4
     for (long e = gptr[u]; e < gptr[u + 1]; e++) {
         const int fb = gl[2 * e], i = gl[2 * e + 1];
         const int j = fcol[fb];
@@ -401,13 +430,42 @@ constexpr int NPART = 1024;
 // host side
 // ---------------------------------------------------------------------------
 
-template <class MT>
-static Op0<MT> op0(tg_ctx* c, const MT* val)
+static OpC opc(const AmgLevel& L) { return OpC{L.n, L.d_sbase.p, L.d_swidth.p, L.d_col.p, L.d_val.p}; }
+
+template <class Op, class E>
+static void launch_rows(tg_ctx* c, const Op& op, const double* x, const E& e, const double* done, int nw)
 {
-    return Op0<MT>{c->nnd, c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val};
+    const int ns = (op.n + 63) / 64;
+    auto go = [&](auto kernel, int blocks, int threads) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(blocks + 7) / 8 * 8), dim3(threads), 0, c->stream, op, x, e, done);
+    };
+    if (nw == 9)
+        go(k_amg_rows<Op, 9, E>, ns, 64 * 9);
+    else if (nw == 3)
+        go(k_amg_rows<Op, 3, E>, ns, 64 * 3);
+    else
+        go(k_amg_rows<Op, 1, E>, (ns + AB / 64 - 1) / (AB / 64), AB);
 }
 
-static OpC opc(const AmgLevel& L) { return OpC{L.n, L.d_sbase.p, L.d_swidth.p, L.d_col.p, L.d_val.p}; }
+// y = A_l x and what follows.  Waves per row: as the PCG's (k_pcg.hip) at the
+// fine level, whose lower blocks are read through their partners from 2^17
+// nodes; the coarse levels' rows, four times as heavy, are shared by 9 waves
+// up to 640 slices and by 3 up to 2,048.
+template <class E>
+static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const double* done)
+{
+    const Bsell& B = c->op;
+    if (l > 0) {
+        const OpC op = opc(*c->amg.lv[l]);
+        launch_rows(c, op, x, e, done, op.n <= 64 * 640 ? 9 : op.n <= 64 * 2048 ? 3 : 1);
+    } else if (large_single(c)) {
+        launch_rows(c, Op0<float, true>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_tpos.p, B.d_val32.p},
+                    x, e, done, 1);
+    } else {
+        launch_rows(c, Op0<float, false>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_tpos.p, B.d_val32.p},
+                    x, e, done, c->nnd <= 64 * 640 ? 9 : pcg_small(c) ? 3 : 1);
+    }
+}
 
 static double* level_dinv(tg_ctx* c, int l) { return l == 0 ? c->vdinv.p : c->amg.lv[l]->dinv; }
 
@@ -424,18 +482,17 @@ static void reduce(tg_ctx* c, int kind, long nd, const double* a, const double* 
 
 // Largest eigenvalue of D^-1 A on level l by power iteration: the Rayleigh
 // quotient (v.Av)/(v.Dv) is left in red[0] / red[1].
-template <class Op>
-static void power_iteration(tg_ctx* c, const Op& op, long nd, const double* dinv, double* v, double* w, double* red)
+static void power_iteration(tg_ctx* c, int l, long nd, const double* dinv, double* v, double* w, double* red)
 {
-    const unsigned nb = blocks_for(op.units()), vb = blocks_for(nd);
+    const unsigned vb = blocks_for(nd);
     hipLaunchKernelGGL(k_amg_rand, dim3(vb), dim3(AB), 0, c->stream, nd, dinv, v);
     for (int it = 0; it < POWER_ITS; it++) {
-        hipLaunchKernelGGL(k_amg_spmv<Op>, dim3(nb), dim3(AB), 0, c->stream, op, v, w);
+        level_rows(c, l, v, EStore{w}, nullptr);
         hipLaunchKernelGGL(k_amg_jac, dim3(vb), dim3(AB), 0, c->stream, nd, dinv, w);
         reduce(c, 0, nd, w, w, red + 2);
         hipLaunchKernelGGL(k_amg_scale, dim3(vb), dim3(AB), 0, c->stream, nd, w, red + 2, v);
     }
-    hipLaunchKernelGGL(k_amg_spmv<Op>, dim3(nb), dim3(AB), 0, c->stream, op, v, w);
+    level_rows(c, l, v, EStore{w}, nullptr);
     reduce(c, 0, nd, v, w, red);
     reduce(c, 1, nd, v, dinv, red + 1);
 }
@@ -529,10 +586,7 @@ static void amg_numeric_t(tg_ctx* c, const MT* val0)
         AmgLevel& A = *G.lv[l];
         const long nd = (long)A.n * A.bs;
         double* red = G.d_red.p + 16 * l;
-        if (l == 0)
-            power_iteration(c, op0<MT>(c, val0), nd, level_dinv(c, 0), A.d_d0.p, A.d_d1.p, red);
-        else
-            power_iteration(c, opc(A), nd, level_dinv(c, l), A.d_d0.p, A.d_d1.p, red);
+        power_iteration(c, l, nd, level_dinv(c, l), A.d_d0.p, A.d_d1.p, red);
         TG_HIP(hipGetLastError());
     }
     std::vector<double> red(16 * (size_t)L);
@@ -592,32 +646,27 @@ void amg_numeric(tg_ctx* c)
     G.since = 0;
 }
 
-template <class Op>
-static void smooth_down(tg_ctx* c, const Op& op, long nd, const double* dinv, const double* f, double* x, AmgLevel& A,
-                        const double* cf, const double* done)
+static void smooth_down(tg_ctx* c, int l, const double* f, double* x, AmgLevel& A, const double* cf, const double* done)
 {
-    const unsigned nb = blocks_for(op.units());
-    hipLaunchKernelGGL(k_amg_pre, dim3(blocks_for(nd)), dim3(AB), 0, c->stream, nd, dinv, f, A.d_r.p, A.d_d0.p, x, cf,
-                       done);
-    double *dp = A.d_d0.p, *dn = A.d_d1.p;
-    for (int s = 1; s < c->amg.degree; s++) {
-        hipLaunchKernelGGL(k_amg_step<Op>, dim3(nb), dim3(AB), 0, c->stream, op, dinv, dp, dn, A.d_r.p, x, cf,
-                           2 * s - 1, 0, done);
+    const double* dinv = level_dinv(c, l);
+    const long nd = (long)A.n * A.bs;
+    double *dp = A.d_d1.p, *dn = A.d_d0.p;
+    hipLaunchKernelGGL(k_amg_pre, dim3(blocks_for(nd)), dim3(AB), 0, c->stream, nd, dinv, f, cf, dn, done);
+    level_rows(c, l, dn, EFirst{dinv, f, cf, dn, dp, A.d_r.p, x}, done);
+    for (int s = 2; s < c->amg.degree; s++) {
+        level_rows(c, l, dp, EStep{dinv, dp, cf, dn, A.d_r.p, x, 2 * s - 1, 0}, done);
         std::swap(dp, dn);
     }
-    hipLaunchKernelGGL(k_amg_resid<Op>, dim3(nb), dim3(AB), 0, c->stream, op, dp, A.d_r.p, done);
+    level_rows(c, l, dp, EResid{A.d_r.p}, done);
 }
 
-template <class Op>
-static void smooth_up(tg_ctx* c, const Op& op, const double* dinv, const double* f, double* x, AmgLevel& A,
-                      const double* cf, const double* done)
+static void smooth_up(tg_ctx* c, int l, const double* f, double* x, AmgLevel& A, const double* cf, const double* done)
 {
-    const unsigned nb = blocks_for(op.units());
-    hipLaunchKernelGGL(k_amg_post<Op>, dim3(nb), dim3(AB), 0, c->stream, op, dinv, f, x, A.d_r.p, A.d_d0.p, cf, done);
+    const double* dinv = level_dinv(c, l);
+    level_rows(c, l, x, EPost{dinv, f, cf, A.d_r.p, A.d_d0.p}, done);
     double *dp = A.d_d0.p, *dn = A.d_d1.p;
     for (int s = 1; s < c->amg.degree; s++) {
-        hipLaunchKernelGGL(k_amg_step<Op>, dim3(nb), dim3(AB), 0, c->stream, op, dinv, dp, dn, A.d_r.p, x, cf,
-                           2 * s - 1, s == 1 ? 1 : 0, done);
+        level_rows(c, l, dp, EStep{dinv, dp, cf, dn, A.d_r.p, x, 2 * s - 1, s == 1 ? 1 : 0}, done);
         std::swap(dp, dn);
     }
 }
@@ -626,39 +675,37 @@ static void smooth_up(tg_ctx* c, const Op& op, const double* dinv, const double*
 // solve has converged), so a captured chunk of iterations stays valid.
 void amg_vcycle(tg_ctx* c, const double* f0, double* z, const double* done)
 {
-    using MT = float;
-    const MT* val0 = c->op.d_val32.p;
     Amg& G = c->amg;
     const int L = (int)G.lv.size();
     for (int l = 0; l + 1 < L; l++) {
         AmgLevel& A = *G.lv[l];
         AmgLevel& C = *G.lv[l + 1];
-        const double* f = l == 0 ? f0 : A.d_f.p;
-        double* x = l == 0 ? z : A.d_x.p;
-        const double* cf = G.d_coef.p + 8 * l;
-        const long nd = (long)A.n * A.bs;
+        smooth_down(c, l, l == 0 ? f0 : A.d_f.p, l == 0 ? z : A.d_x.p, A, G.d_coef.p + 8 * l, done);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks_for(6L * C.n)), dim3(AB), 0, c->stream, C.n, A.d_mptr.p, A.d_mem.p,
+                               A.d_P.p, A.d_r.p, C.d_f.p, done);
+        };
         if (l == 0)
-            smooth_down(c, op0<MT>(c, val0), nd, level_dinv(c, 0), f, x, A, cf, done);
+            go(k_amg_restrict<3>);
         else
-            smooth_down(c, opc(A), nd, level_dinv(c, l), f, x, A, cf, done);
-        hipLaunchKernelGGL(k_amg_restrict, dim3(blocks_for(6L * C.n)), dim3(AB), 0, c->stream, C.n, A.bs, A.d_mptr.p,
-                           A.d_mem.p, A.d_P.p, A.d_r.p, C.d_f.p, done);
+            go(k_amg_restrict<6>);
     }
     AmgLevel& Cst = *G.lv[L - 1];
-    hipLaunchKernelGGL(k_amg_dense, dim3(blocks_for(G.ncd)), dim3(AB), 0, c->stream, G.ncd, G.d_cinv.p, Cst.d_f.p,
+    hipLaunchKernelGGL(k_amg_dense, dim3(blocks_for(G.ncd)), dim3(4 * AB), 0, c->stream, G.ncd, G.d_cinv.p, Cst.d_f.p,
                        Cst.d_x.p, done);
     for (int l = L - 2; l >= 0; l--) {
         AmgLevel& A = *G.lv[l];
         AmgLevel& C = *G.lv[l + 1];
-        const double* f = l == 0 ? f0 : A.d_f.p;
         double* x = l == 0 ? z : A.d_x.p;
-        const double* cf = G.d_coef.p + 8 * l;
-        hipLaunchKernelGGL(k_amg_prolong, dim3(blocks_for((long)A.n * A.bs)), dim3(AB), 0, c->stream, A.n, A.bs,
-                           A.d_agg.p, A.d_P.p, C.d_x.p, 0.01 * G.weight, x, done);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks_for((long)A.n * A.bs)), dim3(AB), 0, c->stream, A.n, A.d_agg.p,
+                               A.d_P.p, C.d_x.p, 0.01 * G.weight, x, done);
+        };
         if (l == 0)
-            smooth_up(c, op0<MT>(c, val0), level_dinv(c, 0), f, x, A, cf, done);
+            go(k_amg_prolong<3>);
         else
-            smooth_up(c, opc(A), level_dinv(c, l), f, x, A, cf, done);
+            go(k_amg_prolong<6>);
+        smooth_up(c, l, l == 0 ? f0 : A.d_f.p, x, A, G.d_coef.p + 8 * l, done);
     }
     TG_HIP(hipGetLastError());
 }

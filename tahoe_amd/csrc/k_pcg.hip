@@ -992,7 +992,10 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
         TG_HIP(hipGetLastError());
     }
     if (npers < nseg) {
-    const int CHUNK = PC == 2 ? 8 : 16;  // even: direction buffers and scalar slots alternate
+    // even: direction buffers and scalar slots alternate.  An iteration with the
+    // multigrid is some 60 kernels: chunks of two keep the launches queued past
+    // the last iteration few (chunks of eight cost 1.6 ms a solve at 128^3)
+    const int CHUNK = PC == 2 ? 2 : 16;
     double* pbuf[2] = {p, nullptr};
     if (fused) {
         if (!W.p2) fail(TG_GENERAL_FAIL, "fused PCG iteration without its second direction buffer");

@@ -361,6 +361,8 @@ void amg_setup(tg_ctx* c)
         }
         upload(c, nx->d_diagblk, diag);
         nx->d_val.alloc((size_t)nx->nslots * 36);
+        // padding slots stay zero (the products read them)
+        TG_HIP(hipMemsetAsync(nx->d_val.p, 0, sizeof(float) * (size_t)nx->nslots * 36, c->stream));
         nx->d_dinv_own.alloc(6 * (size_t)nagg);
         nx->dinv = nx->d_dinv_own.p;
         for (auto* v : {&nx->d_f, &nx->d_x, &nx->d_r, &nx->d_d0, &nx->d_d1}) v->alloc(6 * (size_t)nagg);
