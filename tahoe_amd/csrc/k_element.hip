@@ -702,9 +702,7 @@ __device__ __forceinline__ int node_major(int p) { return 3 * (p & 7) + (p >> 3)
 // MINW > 1 asks the compiler for registers that fit MINW waves per SIMD.
 // GATHER: the entries go to the element buffer, val = its row of the
 // launch's first element (no slot map, no loads); else into the MSR.
-// ROWS (with GATHER): to the block buffer of the assembly by rows, all
-// elements in mesh order (elems = nullptr, slot = the elements' ranks).
-template <class VT, int EPW, int MAT = MAT_SIMO, int MINW = 1, bool GATHER = false, bool ROWS = false>
+template <class VT, int EPW, int MAT = MAT_SIMO, int MINW = 1, bool GATHER = false>
 __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restrict__ elems, int count,
                                                         const int* __restrict__ conn, const int* __restrict__ emat,
                                                         const double2* __restrict__ props,
@@ -720,7 +718,7 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
     const int l = threadIdx.x;
     const long base = (long)blockIdx.x * EPW;
     const int nel = (int)(count - base < EPW ? count - base : EPW);
-    auto el = [&](int i) { return ROWS ? (int)(base + i) : elems[base + i]; };
+    auto el = [&](int i) { return elems[base + i]; };
     bool bad = false;
     if (l < 8 * EPW) {
         const int le = l >> 3, q = l & 7;
@@ -789,30 +787,7 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
             nold[k] = nsidx[k] >= 0 ? x : VT(0);
         }
     }
-    // ROWS: places of the entries in the element's 36 x 9 block values, formed
-    // again only when the ranks change (structured meshes: never)
-    unsigned pm = 0;
-    int dst[ROWS ? 12 : 1];
-    auto place = [&](int p, int q) {
-        // dofs p and q of the dof-major order: nodes p & 7, q & 7, directions p >> 3, q >> 3
-        const int rp = rank_of(pm, p & 7), rq = rank_of(pm, q & 7), i = p >> 3, j = q >> 3;
-        const bool keep = rp < rq || (rp == rq && i <= j);
-        return 9 * pair_index(min(rp, rq), max(rp, rq)) + (keep ? 3 * i + j : 3 * j + i);
-    };
     for (int le = 0; le < nel; le++) {
-        if (ROWS) {
-            const unsigned x = __builtin_amdgcn_readfirstlane((unsigned)slot[base + le]);
-            if (x != pm) {
-                pm = x;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int m = Mfma<VT>::row(kq, r);
-                    dst[ROWS ? r : 0] = m <= c ? place(m, c) : -1;
-                    dst[ROWS ? 4 + r : 0] = lo8 ? place(m, 16 + na) : -1;
-                    dst[ROWS ? 8 + r : 0] = (lo8 && m < 8 && m <= c) ? place(16 + m, 16 + na) : -1;
-                }
-            }
-        }
         int sidx[12];
         VT old[12];
 #pragma unroll
@@ -889,16 +864,6 @@ __global__ void __launch_bounds__(64, MINW) k_stiffness_mfma(const int* __restri
                 const VT x = val[nsidx[k] >= 0 ? nsidx[k] : 0];
                 nold[k] = nsidx[k] >= 0 ? x : VT(0);
             }
-        }
-        if (ROWS) {
-            VT* eb = val + 324L * (base + le);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                if (dst[ROWS ? r : 0] >= 0) eb[dst[ROWS ? r : 0]] = acc00[r];
-                if (dst[ROWS ? 4 + r : 0] >= 0) eb[dst[ROWS ? 4 + r : 0]] = acc01[r];
-                if (dst[ROWS ? 8 + r : 0] >= 0) eb[dst[ROWS ? 8 + r : 0]] = acc11[r];
-            }
-            continue;
         }
         if (GATHER) {
             VT* eb = val + 300L * (base + le);
@@ -1023,28 +988,156 @@ static bool gather_ready(tg_ctx* c)
     return true;
 }
 
-// Block buffer of the assembly by rows: the FP32 stiffness on the matrix
-// cores, FP64 in the 12-element block kernel (both the fastest untuned
-// shapes of their precision).
 static void launch_block_scatter(tg_ctx* c);
 
+// Blocks of the Simo material for the assembly by rows.  Its tangent is
+// c = A 1x1 + B I + C (s x 1 + 1 x s) (simo_moduli, sorted by tensor), so with
+//   v_a = C s g_a,  w_b = A g_b + v_b,  t_b = (B/2 + T) g_b
+// formed once per node and integration point, a block is three outer products
+// and a dot product,
+//   K_ab += g_a w_b^T + v_a g_b^T + B/2 g_b g_a^T + (g_a . t_b) 1,
+// 33 multiply-adds and 16 LDS values per point where the general form has 99
+// and 33.  Seven elements a workgroup: 252 of 256 lanes hold a block, one wave
+// per SIMD.  The blocks leave through LDS, so the buffer is written in
+// consecutive words.
+// Bound by instruction issue (FP64 or FP32) and the chain of its phases: 2.1 M
+// elements FP64 3.23 ms, FP32 2.35 ms; 62 k elements FP64 108 us, FP32 75 us.
+// The general form (10 elements a workgroup in FP64, matrix instructions for
+// the moduli products in FP32) took 168 us and 88 us at 62 k.  Two further
+// splits gave nothing: nodes' vectors in all lanes (3.44 ms) and the point
+// work in another wave from workgroup to workgroup.
+constexpr int BE = 7;
+constexpr int BQ = 97;  // values per element and point: 8 nodes x (g, v, w, t), B/2
+
+template <class VT>
+__global__ void __launch_bounds__(256) k_blocks_simo(int nel, const int* __restrict__ conn,
+                                                     const unsigned* __restrict__ perm, const int* __restrict__ emat,
+                                                     const double2* __restrict__ props, const double* __restrict__ X,
+                                                     const double* __restrict__ U, VT* __restrict__ eb,
+                                                     int* __restrict__ status)
+{
+    __shared__ double sxu[BE][8][6];
+    __shared__ VT sv[BE * 8 * BQ];
+    const int t = threadIdx.x;
+    const int e0 = blockIdx.x * BE;
+    bool bad = false;
+    if (t < 8 * BE) {
+        const int le = t >> 3, q = t & 7;
+        if (e0 + le < nel) {
+            const int node = conn[8L * (e0 + le) + q];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                sxu[le][q][c] = X[3L * node + c];
+                sxu[le][q][3 + c] = U[3L * node + c];
+            }
+        }
+    }
+    __syncthreads();
+    if (t < 8 * BE) {
+        const int le = t >> 3, q = t & 7;
+        if (e0 + le < nel) {
+            const double2 mk = props[emat[e0 + le]];
+            double d[3][8], j0[9], ji[9], g0[3][8], F[9], Fi[9], Jb = 1.0, bb[6] = {1, 1, 1, 0, 0, 0}, sig[6];
+            parent_derivs(q, d);
+            jacobian([&](int a, int c) { return sxu[le][a][c]; }, d, j0);
+            const double det0 = det3(j0);
+            bad |= !(det0 > 0.0);
+            inv3(j0, det0, ji);
+            spatial_derivs(ji, d, g0);
+            deformation_gradient([&](int a, int c) { return sxu[le][a][3 + c]; }, g0, F);
+            const double J = det3(F);
+            bad |= !(J > 0.0);
+            bad |= !material_stress<MAT_SIMO>(mk.x, mk.y, F, J, Jb, bb, sig);
+            inv3(F, J, Fi);
+            const double scale = bad ? 0.0 : det0 * J;  // weight 1
+            const double du = 0.5 * mk.y * (Jb - 1.0 / Jb), ddu = 0.5 * mk.y * (1.0 + 1.0 / (Jb * Jb));
+            const double tr = (bb[0] + bb[1] + bb[2]) / 3.0, mu_bar = mk.x * tr / Jb;
+            const double A = scale * (du + Jb * ddu - 2.0 / 3.0 * mu_bar), hB = scale * (mu_bar - du);
+            const double C = scale * (-2.0 / (3.0 * Jb)) * mk.x;  // times dev(b_bar)
+            const double s[6] = {C * (bb[0] - tr), C * (bb[1] - tr), C * (bb[2] - tr), C * bb[3], C * bb[4], C * bb[5]};
+            double T[6];
+#pragma unroll
+            for (int k = 0; k < 6; k++) T[k] = scale * sig[k] + (k < 3 ? hB : 0.0);
+            VT* out = sv + (le * 8 + q) * BQ;
+#pragma unroll
+            for (int a = 0; a < 8; a++) {
+                double g[3];
+#pragma unroll
+                for (int j = 0; j < 3; j++)
+                    g[j] = Fi[0 + 3 * j] * g0[0][a] + Fi[1 + 3 * j] * g0[1][a] + Fi[2 + 3 * j] * g0[2][a];
+                const double v[3] = {s[0] * g[0] + s[5] * g[1] + s[4] * g[2], s[5] * g[0] + s[1] * g[1] + s[3] * g[2],
+                                     s[4] * g[0] + s[3] * g[1] + s[2] * g[2]};
+                const double tt[3] = {T[0] * g[0] + T[5] * g[1] + T[4] * g[2], T[5] * g[0] + T[1] * g[1] + T[3] * g[2],
+                                      T[4] * g[0] + T[3] * g[1] + T[2] * g[2]};
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    out[12 * a + j] = (VT)g[j];
+                    out[12 * a + 3 + j] = (VT)v[j];
+                    out[12 * a + 6 + j] = (VT)(A * g[j] + v[j]);
+                    out[12 * a + 9 + j] = (VT)tt[j];
+                }
+            }
+            out[96] = (VT)hB;
+        }
+    }
+    __syncthreads();
+    const int le = t / 36, p = t - 36 * le;
+    const bool on = t < 36 * BE && e0 + le < nel;
+    int a, b;
+    upper_block(p, a, b);
+    VT K[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) K[i][j] = 0;
+    if (on) {
+#pragma unroll 2
+        for (int q = 0; q < 8; q++) {
+            const VT* in = sv + (le * 8 + q) * BQ;
+            const VT *ga = in + 12 * a, *gb = in + 12 * b;
+            const VT h = in[96];
+            const VT g0 = ga[0], g1 = ga[1], g2 = ga[2], v[3] = {ga[3], ga[4], ga[5]};
+            const VT gj[3] = {gb[0], gb[1], gb[2]}, w[3] = {gb[6], gb[7], gb[8]};
+            const VT gi[3] = {g0, g1, g2}, hg[3] = {h * g0, h * g1, h * g2};
+            const VT geo = g0 * gb[9] + g1 * gb[10] + g2 * gb[11];
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) K[i][j] += gi[i] * w[j] + v[i] * gj[j] + hg[j] * gj[i];
+#pragma unroll
+            for (int i = 0; i < 3; i++) K[i][i] += geo;
+        }
+    }
+    __syncthreads();  // past the last read of sv
+    if (on) {
+        const unsigned pm = perm[e0 + le];
+        const int ra = rank_of(pm, a), rb = rank_of(pm, b);
+        VT* out = sv + 324 * le + 9 * pair_index(min(ra, rb), max(ra, rb));
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                if (a != b || j >= i) out[ra <= rb ? 3 * i + j : 3 * j + i] = K[i][j];
+    }
+    __syncthreads();
+    const int n = 324 * min(BE, nel - e0);
+    for (int x = t; x < n; x += 256) eb[324L * e0 + x] = sv[x];
+    if (bad) atomicOr(status, 7);
+}
+
+// Block buffer of the assembly by rows.
 template <class VT>
 static void launch_blocks(tg_ctx* c, const double* u, VT* eb)
 {
     const int* ranks = reinterpret_cast<const int*>(c->r_perm.p);
     const int n = c->nel;
-    auto go = [&](auto kernel, int epb, int threads) {
-        hipLaunchKernelGGL(kernel, dim3((n + epb - 1) / epb), dim3(threads), 0, c->stream, nullptr, n, c->dconn.p,
-                           c->dmat.p, c->dmatprops.p, c->dX.p, u, ranks, c->deqn.p, eb, c->dstatus.p);
-    };
     if (c->material_model == TG_MAT_STVENANT)
-        go(k_stiffness_tl<VT, 12, false, false, 6, MAT_STVENANT>, 12, 36 * 12);
-    else if constexpr (sizeof(VT) == 4)
-        hipLaunchKernelGGL((k_stiffness_mfma<VT, 4, MAT_SIMO, 1, true, true>), dim3((n + 3) / 4), dim3(64), 0,
-                           c->stream, nullptr, n, c->dconn.p, c->dmat.p, c->dmatprops.p, c->dX.p, u, ranks, eb,
-                           c->dstatus.p);
+        hipLaunchKernelGGL((k_stiffness_tl<VT, 7, false, false, 6, MAT_STVENANT>), dim3((n + 6) / 7), dim3(36 * 7), 0,
+                           c->stream, nullptr, n, c->dconn.p, c->dmat.p, c->dmatprops.p, c->dX.p, u, ranks, c->deqn.p,
+                           eb, c->dstatus.p);
     else
-        go(k_stiffness_tl<VT, 12, false, false, 6, MAT_SIMO>, 12, 36 * 12);
+        hipLaunchKernelGGL(k_blocks_simo<VT>, dim3((n + BE - 1) / BE), dim3(256), 0, c->stream, n, c->dconn.p,
+                           c->r_perm.p, c->dmat.p, c->dmatprops.p, c->dX.p, u, eb, c->dstatus.p);
 }
 
 void launch_stiffness(tg_ctx* c, const double* u)
@@ -1252,6 +1345,7 @@ void launch_element_slots(tg_ctx* c)
 void colour_structure(tg_ctx* c)
 {
     if (c->colours_ready) return;
+    expansion_structure(c);
     c->ncolors = color_elements(c->nnd, c->nel, c->conn.data(), c->color_ptr, c->color_elems);
     c->dcolor_elems.alloc((size_t)c->nel);
     TG_HIP(hipMemcpyAsync(c->dcolor_elems.p, c->color_elems.data(), sizeof(int) * c->nel, hipMemcpyHostToDevice,
@@ -1405,6 +1499,13 @@ void launch_build_src(tg_ctx* c)
     hipLaunchKernelGGL(k_build_src, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, c->stream, c->nnd,
                        c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, c->deqn.p, c->dbindx.p,
                        c->op.d_src.p);
+    TG_HIP(hipGetLastError());
+}
+
+void launch_build_tpos(tg_ctx* c)
+{
+    const int bs = 256;
+    const long n = 64L * c->op.nslices;
     hipLaunchKernelGGL(k_build_tpos, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, c->stream, c->nnd,
                        c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, c->op.d_tpos.p);
     TG_HIP(hipGetLastError());

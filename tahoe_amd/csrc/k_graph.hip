@@ -297,7 +297,6 @@ void device_structure(tg_ctx* c)
     TG_HIP(hipMemcpyAsync(B.d_slice_base.p, B.slice_base.data(), sizeof(int) * B.nslices, hipMemcpyHostToDevice,
                           c->stream));
     B.d_col.alloc((size_t)B.nblocks_padded);
-    B.d_src.alloc((size_t)B.nblocks_padded * 9);
     B.d_tpos.alloc((size_t)B.nblocks_padded);
     B.d_val.alloc((size_t)B.nblocks_padded * 9);
     hipLaunchKernelGGL(k_block_columns, dim3(grid(64L * B.nslices, 256)), dim3(256), 0, c->stream, nnd, B.nslices,
@@ -323,18 +322,30 @@ void device_structure(tg_ctx* c)
                        c->g_rows.p, c->dbindx.p);
     TG_HIP(hipGetLastError());
     launch_msr_cols(c);  // the MSR columns from the block columns, before anything reads them
+    launch_build_tpos(c);
+    c->src_ready = false;
+}
+
+// What the expansion of the MSR values into the operator needs: the value map
+// and the half slices' value ranges; built when it first runs on a mesh (the
+// assembly by rows writes the operator itself).
+void expansion_structure(tg_ctx* c)
+{
+    if (c->src_ready) return;
+    Bsell& B = c->op;
+    B.d_src.alloc((size_t)B.nblocks_padded * 9);
     launch_build_src(c);
-    // half-slice value ranges of the expansion
     const int nhalf = 2 * B.nslices;
     B.d_srange.alloc((size_t)nhalf);
     c->g_most.alloc((size_t)nhalf);
-    hipLaunchKernelGGL(k_half_slice_ranges, dim3(grid(nhalf, 256)), dim3(256), 0, c->stream, nnd, nhalf, c->deqn.p,
+    hipLaunchKernelGGL(k_half_slice_ranges, dim3(grid(nhalf, 256)), dim3(256), 0, c->stream, c->nnd, nhalf, c->deqn.p,
                        c->dbindx.p, B.d_srange.p, c->g_most.p);
     TG_HIP(hipGetLastError());
     std::vector<long long> most((size_t)nhalf);
     TG_HIP(hipMemcpyAsync(most.data(), c->g_most.p, sizeof(long long) * nhalf, hipMemcpyDeviceToHost, c->stream));
     TG_HIP(hipStreamSynchronize(c->stream));
     B.lds_values = most.empty() ? 0 : (long)*std::max_element(most.begin(), most.end());
+    c->src_ready = true;
 }
 
 }  // namespace tg

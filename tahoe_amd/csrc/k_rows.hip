@@ -57,22 +57,38 @@ __global__ void k_sort_lists(int nnd, const int* __restrict__ ptr, int* __restri
 }
 
 // slot index of each row's diagonal block (the number of its lower blocks),
-// the row's upper slots, and their largest number over all rows
+// the row's upper slots, and their largest number over all rows; for each
+// upper slot 8 x (active dofs of the row's neighbours between it and the
+// diagonal) + mask of its node's active dofs: with the row's pointer, where
+// the block's MSR values are (a slice's rows one after the other)
 __global__ void k_row_upper(int nnd, const int* __restrict__ sbase, const int* __restrict__ swidth,
-                            const int* __restrict__ bcol, int2* __restrict__ upper, int* __restrict__ most)
+                            const int* __restrict__ bcol, const int* __restrict__ eqn, int2* __restrict__ upper,
+                            unsigned short* __restrict__ runs, int* __restrict__ most)
 {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= nnd) return;
-    const int s = a >> 6, l = a & 63;
     int lo = 0, n = 0;
-    for (int k = 0; k < swidth[s]; k++) {
-        const int c = bcol[((long)sbase[s] + k) * 64 + l];
-        if (c < 0) break;
-        n++;
-        lo += c < a;
+    if (a < nnd) {
+        const int s = a >> 6, l = a & 63;
+        int run = 0;
+        for (int k = 0; k < swidth[s]; k++) {
+            const long at = ((long)sbase[s] + k) * 64 + l;
+            const int c = bcol[at];
+            if (c < 0) break;
+            n++;
+            lo += c < a;
+            if (c < a) continue;
+            int mask = 0;
+#pragma unroll
+            for (int j = 0; j < 3; j++) mask |= (eqn[3L * c + j] >= 0) << j;
+            runs[64L * sbase[s] + (long)l * swidth[s] + k] = (unsigned short)(8 * run + mask);
+            if (c > a) run += __popc(mask);
+        }
+        upper[a] = make_int2(lo, n - lo);
     }
-    upper[a] = make_int2(lo, n - lo);
-    atomicMax(most, n - lo);
+    int m = n - lo;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(most, m);
 }
 
 // rslot[e][r][j] = upper slot (0: the diagonal) of the row of rank r that
@@ -184,22 +200,26 @@ __global__ void __launch_bounds__(1024) k_fin_residual(const double* __restrict_
 // ---- stiffness ----------------------------------------------------------------
 
 constexpr int GR = 32;  // rows of a workgroup (half a slice), 8 lanes each
+constexpr int GQ = 2;   // elements whose loads are in flight
 
 // Rows of half a slice: 8 lanes per row add the row's blocks of its elements,
-// in list order, into LDS (a row's lanes are in one wave, so its sums need
-// no barrier); then 32 consecutive lanes write one component of their rows'
-// blocks: the operator block and its transpose in the partner's row, the MSR
-// values, and 1/diag.  Prescribed dofs (src < 0) give zeros.
+// in list order, into LDS, a block a lane (a row's lanes are in one wave, so
+// its sums need no barrier), and write the row's MSR values and 1/diag; then
+// 32 consecutive lanes write one component of their rows' blocks, the operator
+// block and its transpose in the partner's row.  Prescribed dofs give zeros.
 // BT: block buffer and sums, MT: MSR values, OT: operator.
 // Bound by memory: the block buffer read once, every operator and MSR value
-// written once.  67 k nodes FP64: 144 us for 0.43 GB (3.0 TB/s); with the
-// element pass 168 us.  The colour passes with their clearing, expansion and
-// 1/diag took 265 + 18 + 105 us there; 1.15 M nodes FP32: 1.94 + 1.56 ms
-// against 2.30 + 1.05 ms, and the set-up's slot maps (4.7 ms) are gone.
+// written once.  67 k nodes FP64: 105 us for 0.37 GB (3.5 TB/s); with the
+// element pass 224 us.  The colour passes with their clearing, expansion and
+// 1/diag took 265 + 18 + 105 us there; 2.15 M nodes FP32: 2.13 + 2.35 ms.
+// (With single values a lane and the expansion's map of 36 B a block read
+// beside it the gather took 144 us and 3.25 ms.)
 template <class BT, class MT, class OT>
 __global__ void __launch_bounds__(256) k_gather_rows(int nnd, int n_eq, int up_most, const int* __restrict__ sbase,
                                                      const int* __restrict__ swidth, const int* __restrict__ tpos,
-                                                     const int* __restrict__ src, const int2* __restrict__ upper,
+                                                     const int2* __restrict__ upper,
+                                                     const unsigned short* __restrict__ runs,
+                                                     const int* __restrict__ eqn, const int* __restrict__ bindx,
                                                      const int* __restrict__ ptr, const int* __restrict__ list,
                                                      const unsigned char* __restrict__ rslot,
                                                      const BT* __restrict__ eb, MT* __restrict__ val,
@@ -210,50 +230,88 @@ __global__ void __launch_bounds__(256) k_gather_rows(int nnd, int n_eq, int up_m
     const int stride = 9 * up_most + 1;  // odd: consecutive rows fall into different banks
     const int s = blockIdx.x >> 1, h = blockIdx.x & 1;
     const int row0 = 64 * s + GR * h;
+    const long b0 = sbase[s];
+    const int w = swidth[s];
     if (blockIdx.x == 0 && threadIdx.x == 0) val[n_eq] = MT(0);  // the entry between diagonal and rows is no value
     {
         const int row = threadIdx.x >> 3, t = threadIdx.x & 7;
         const int a = row0 + row;
         if (a < nnd) {
             BT* my = acc + row * stride;
-            const int nup9 = 9 * upper[a].y;
-            for (int x = t; x < nup9; x += 8) my[x] = BT(0);
-            // value x = t + 8 m of a run is component c of block j of it
+            const int2 up = upper[a];
+            for (int x = t; x < 9 * up.y; x += 8) my[x] = BT(0);
+            // lane t takes block t of a run
             const int p1 = ptr[a + 1];
-            for (int p = ptr[a]; p < p1; p += 2) {
-                // two elements' loads in flight before their sums
-                BT v[2][9];
-                unsigned long long sl[2];
-                int len[2];
+            for (int p = ptr[a]; p < p1; p += GQ) {
+                // GQ elements' loads in flight before their sums
+                BT v[GQ][9];
+                int slot[GQ];
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const bool in = p + q < p1;
-                    const int code = in ? list[p + q] : 0;
+                for (int q = 0; q < GQ; q++) {
+                    const int code = list[min(p + q, p1 - 1)];
                     const int e = code >> 3, r = code & 7;
-                    len[q] = in ? 9 * (8 - r) : 0;
-                    sl[q] = reinterpret_cast<const unsigned long long*>(rslot)[code];
-                    const BT* run = eb + 324L * e + 9 * pair_index(r, r);
+                    const int j = min(t, 7 - r);
+                    slot[q] = p + q < p1 && t == j ? rslot[8L * code + j] : -1;
+                    const BT* blk = eb + 324L * e + 9 * (pair_index(r, r) + j);
 #pragma unroll
-                    for (int m = 0; m < 9; m++) v[q][m] = t + 8 * m < len[q] ? run[t + 8 * m] : BT(0);
+                    for (int c = 0; c < 9; c++) v[q][c] = blk[c];
                 }
 #pragma unroll
-                for (int q = 0; q < 2; q++)
+                for (int q = 0; q < GQ; q++) {
+                    if (slot[q] >= 0)
 #pragma unroll
-                    for (int m = 0; m < 9; m++)
-                        if (t + 8 * m < len[q]) {
-                            const int j = t >= m ? m : m - 1, c = t >= m ? t - m : t - m + 9;
-                            my[9 * (int)((sl[q] >> (8 * j)) & 255) + c] += v[q][m];
-                        }
-                // (lanes of a row read sums other lanes wrote: the wave's LDS
-                // operations stay in this order)
-                __builtin_amdgcn_wave_barrier();
+                        for (int c = 0; c < 9; c++) my[9 * slot[q] + c] += v[q][c];
+                    // (lanes of a row read sums other lanes wrote: the wave's
+                    // LDS operations stay in this order)
+                    __builtin_amdgcn_wave_barrier();
+                }
             }
+            // MSR values: row r[i] lists the node's own later dofs, then the
+            // neighbours'.  What is no entry becomes zero for the operator.
+            int r[3], first[3], own = 0;
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                r[i] = eqn[3L * a + i];
+                own |= (r[i] >= 0) << i;
+            }
+#pragma unroll
+            for (int i = 0; i < 3; i++) first[i] = r[i] >= 0 ? bindx[r[i]] + __popc(own >> (i + 1)) : 0;
+            const unsigned short* run = runs + 64 * b0 + (long)(GR * h + row) * w + up.x;
+            for (int kk = t; kk < up.y; kk += 8) {
+                const int rm = run[kk], mask = rm & 7;
+                BT* x = my + 9 * kk;
+                if (kk == 0) {
+                    // a diagonal block holds its upper entries
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+#pragma unroll
+                        for (int j = i; j < 3; j++) {
+                            const bool act = r[i] >= 0 && r[j] >= 0;
+                            const BT y = act ? x[3 * i + j] : BT(0);
+                            x[3 * i + j] = x[3 * j + i] = y;
+                            if (act)
+                                val[i == j ? r[i] : first[i] - __popc(own >> j)] = (MT)y;
+                            if (i == j) dinv[3L * a + i] = y != BT(0) ? 1.0 / (double)y : 0.0;
+                        }
+                } else {
+                    const int at = rm >> 3;
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+#pragma unroll
+                        for (int j = 0; j < 3; j++) {
+                            if (r[i] >= 0 && ((mask >> j) & 1))
+                                val[first[i] + at + __popc(mask & ((1 << j) - 1))] = (MT)x[3 * i + j];
+                            else
+                                x[3 * i + j] = BT(0);
+                        }
+                }
+            }
+            // rows of nodes that no element uses
+            if (up.y == 0 && t < 3) dinv[3L * a + t] = 0.0;
         }
     }
     __syncthreads();
     const int row = threadIdx.x & 31, a = row0 + row, l = GR * h + row;
-    const long b0 = sbase[s];
-    const int w = swidth[s];
     const int2 up = a < nnd ? upper[a] : make_int2(0, 0);
     const BT* my = acc + row * stride;
     for (int k = threadIdx.x >> 5; k < w; k += 8) {
@@ -270,21 +328,11 @@ __global__ void __launch_bounds__(256) k_gather_rows(int nnd, int n_eq, int up_m
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = 0; j < 3; j++) {
-                const int c = 3 * i + j;
-                // a diagonal block holds its upper entries
-                const BT x = my[9 * kk + (kk == 0 && j < i ? 3 * j + i : c)];
-                const int sv = src[o + 64 * c];
-                const BT v = sv >= 0 ? x : BT(0);
-                out[o + 64 * c] = (OT)v;
-                if (sv >= 0 && (kk > 0 || j >= i)) val[sv] = (MT)v;
-                if (kk > 0) out[lp + 64 * (3 * j + i)] = (OT)v;
-                if (kk == 0 && i == j) dinv[3L * a + i] = v != BT(0) ? 1.0 / (double)v : 0.0;
+                const OT v = (OT)my[9 * kk + 3 * i + j];
+                out[o + 64 * (3 * i + j)] = v;
+                if (kk > 0) out[lp + 64 * (3 * j + i)] = v;
             }
     }
-    // rows of nodes that no element uses
-    if (a < nnd && up.y == 0 && threadIdx.x < GR)
-#pragma unroll
-        for (int i = 0; i < 3; i++) dinv[3L * a + i] = 0.0;
 }
 
 unsigned grid(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -303,9 +351,10 @@ void rows_structure(tg_ctx* c)
     c->r_perm.alloc((size_t)nel);
     hipLaunchKernelGGL(k_ranks, dim3(grid(nel, 256)), dim3(256), 0, c->stream, nel, c->dconn.p, c->r_perm.p);
     c->r_upper.alloc((size_t)nnd);
+    c->r_run.alloc((size_t)B.nblocks_padded);
     TG_HIP(hipMemsetAsync(c->g_flag.p, 0, sizeof(int), c->stream));
     hipLaunchKernelGGL(k_row_upper, dim3(grid(nnd, 256)), dim3(256), 0, c->stream, nnd, B.d_slice_base.p,
-                       B.d_slice_width.p, B.d_col.p, c->r_upper.p, c->g_flag.p);
+                       B.d_slice_width.p, B.d_col.p, c->deqn.p, c->r_upper.p, c->r_run.p, c->g_flag.p);
     TG_HIP(hipGetLastError());
     TG_HIP(hipMemcpyAsync(&c->r_up_most, c->g_flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TG_HIP(hipStreamSynchronize(c->stream));
@@ -355,7 +404,8 @@ void launch_gather_rows(tg_ctx* c)
     const int most = std::max(c->r_up_most, 1);
     auto go = [&](auto kernel, size_t vb, const auto* eb, auto* val, auto* out) {
         hipLaunchKernelGGL(kernel, dim3(g), dim3(256), row * vb, c->stream, c->nnd, c->n_eq, most, B.d_slice_base.p,
-                           B.d_slice_width.p, B.d_tpos.p, B.d_src.p, c->r_upper.p, c->g_neptr.p, c->g_nelist.p,
+                           B.d_slice_width.p, B.d_tpos.p, c->r_upper.p, c->r_run.p, c->deqn.p, c->dbindx.p,
+                           c->g_neptr.p, c->g_nelist.p,
                            c->r_slot.p, eb, val, out, c->vdinv.p);
     };
     if (mixed_stiffness(c))

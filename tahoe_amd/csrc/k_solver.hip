@@ -335,6 +335,7 @@ static unsigned grid_for(long n)
 
 void launch_expand(tg_ctx* c)
 {
+    expansion_structure(c);
     TimedRegion tr(c, T_EXPAND);
     const long n = c->op.nblocks_padded;
     launch_expand_pass1<double>(c, c->dval.p, c->op.d_val.p);
@@ -348,6 +349,7 @@ void launch_expand(tg_ctx* c)
 
 void launch_expand32(tg_ctx* c)
 {
+    expansion_structure(c);
     TimedRegion tr(c, T_EXPAND);
     const long n = c->op.nblocks_padded;
     launch_expand_pass1<float>(c, c->dval32.p, c->op.d_val32.p);

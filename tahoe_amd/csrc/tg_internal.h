@@ -316,6 +316,7 @@ struct tg_ctx {
     // assembly by rows (k_rows.hip)
     tg::DBuf<unsigned> r_perm;          // [nel] ranks of the element's nodes, 4 bits each
     tg::DBuf<int2> r_upper;             // [nnd] slot of the row's diagonal block, upper blocks of the row
+    tg::DBuf<unsigned short> r_run;     // [nblocks_padded] upper slots: 8 x active dofs before + mask (k_row_upper)
     tg::DBuf<unsigned char> r_slot;     // [nel][8][8] upper slot of block (rank r, rank r + j) in the row of rank r
     int r_up_most = 0;                  // most upper blocks of a row
     tg::DBuf<double> r_force;           // [nel][8][3] element forces, by rank
@@ -324,6 +325,7 @@ struct tg_ctx {
     tg::DBuf<double> dpart_r;           // partials of R.R
     bool stiff_explicit = false;        // a knob of the colour-ordered assembly was set: it runs
     bool colours_ready = false;         // colours and slot maps of this mesh are built
+    bool src_ready = false;             // the expansion's value map (d_src) and LDS ranges of this mesh are built
     bool op_fresh = false;              // operator and 1/diag are those of the MSR values
     // stiffness launch order: every segment's elements in ranges of
     // stiff_chunk (by rank inside the segment), all colours of range j
@@ -489,6 +491,8 @@ void launch_stiffness_operator(tg_ctx* c, const double* u);
 void launch_element_slots(tg_ctx* c);
 void launch_msr_cols(tg_ctx* c);
 void launch_build_src(tg_ctx* c);
+void launch_build_tpos(tg_ctx* c);
+void expansion_structure(tg_ctx* c);
 void launch_operator_dinv(tg_ctx* c);
 void launch_block_inverse(tg_ctx* c);
 void launch_build_operator_diag(tg_ctx* c);

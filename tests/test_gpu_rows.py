@@ -79,6 +79,32 @@ def test_rows_equal_colours(n, form, model, precision):
     assert np.abs(us[0] - us[1]).max() <= (1e-4 if precision else 1e-9) * np.abs(us[1]).max()
 
 
+# 6, 7, 8 and 15 elements about a workgroup's 7; free and prescribed dofs in
+# every combination, nodes with none free included
+@pytest.mark.parametrize("n", [(3, 2, 1), (7, 1, 1), (2, 2, 2), (5, 3, 1)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_any_prescribed_dofs(n, precision):
+    from tahoe_amd import api, mesh as M
+    m = shuffled(n, 77)
+    rng = np.random.default_rng(78)
+    pick = rng.random((m.nnd, 3)) < 0.4
+    pick[0] = True
+    nodes, dofs = np.nonzero(pick)
+    kbc = M.KBC(nodes.astype(np.int32), dofs.astype(np.int32), np.zeros(len(nodes)))
+    vals, bs = [], []
+    for rows in (1, 0):
+        s = solid(m, kbc, 0, SIMO, precision)
+        s.set_tuning(api.TUNE_STIFF_ROWS, rows)
+        s.set_displacement(state(m))
+        s.form_lhs()
+        vals.append(s.msr_values())
+        bs.append(s.multx(np.random.default_rng(9).standard_normal(s.n_eq)))
+        s.close()
+    tol = 1e-6 if precision else 1e-13
+    assert np.abs(vals[0] - vals[1]).max() <= tol * np.abs(vals[1]).max()
+    assert np.abs(bs[0] - bs[1]).max() <= 10 * tol * np.abs(bs[1]).max()
+
+
 @pytest.mark.parametrize("form", [0, 1])
 def test_wide_rows_take_the_colours(form):
     from oracle import oracle as O
