@@ -158,9 +158,11 @@ int tg_set_segments(tg_ctx* ctx, int nseg, const int* node_begin);
  * Replaces FEManagerT::SetEquationSystem (FEManagerT.cpp:2248-2313) ->
  * NodeManagerT::SetEquationNumbers (NodeManagerT.cpp:712-760) and
  * GlobalMatrixT::Initialize -> MSRMatrixT::Initialize (MSRMatrixT.cpp:35-44).
- * The equation numbers and the colouring are formed on the host; the node
- * graph, the MSR pattern and the solver operator's structure on the device
- * (so tg_get_msr_bindx copies from the device).  A node shared by more than
+ * All of it is formed on the device: the equation numbers, the node graph, the
+ * row pointers and the solver operator's structure here, the MSR columns when
+ * tg_get_msr_bindx first asks for them, the element colouring (on the host)
+ * when a colour-ordered assembly first runs.  tg_get_eqnos and
+ * tg_get_msr_bindx copy from the device.  A node shared by more than
  * 64 elements is refused (TG_OUT_OF_RANGE).  With the environment variable
  * TG_SETUP_TRACE set, the time of each setup phase is printed to stderr. */
 int tg_initialize(tg_ctx* ctx, int* n_eq, long* msr_length);

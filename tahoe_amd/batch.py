@@ -44,8 +44,9 @@ def pack(problems: list) -> Packed:
     """The sub-problems one after another in one mesh: each starts on a
     multiple of 64 nodes (a slice of the solver operator), the padding nodes
     fully prescribed to zero; material ids map into one global (E, nu)
-    table.  Each array is one concatenation of the problems' own arrays and
-    views of shared padding arrays, plus one offset pass."""
+    table.  Each array is written once, straight from the problems' own
+    arrays: at a million nodes the pages of fresh arrays cost more than the
+    copies, so there are no temporaries."""
     mats, index, gids, gbeg = [], {}, [], [0]
     for p in problems:
         for E, nu in zip(p.E, p.nu):
@@ -60,47 +61,70 @@ def pack(problems: list) -> Packed:
     begins = np.zeros(len(problems) + 1, dtype=np.int64)
     begins[1:] = np.cumsum(nnds + pads)
     nels = np.array([p.mesh.conn.shape[0] for p in problems], dtype=np.int64)
-    zeros3 = np.zeros((64, 3))
+
+    def offsets(counts):
+        out = np.zeros(len(problems) + 1, dtype=np.int64)
+        out[1:] = np.cumsum(counts)
+        return out.tolist()
+
+    first, count, pad = begins.tolist(), nnds.tolist(), pads.tolist()
+    ebeg = offsets(nels)
+
+    def put(out, src, shift=0):
+        if np.shape(src) != out.shape:
+            raise ValueError(f"problem array of shape {np.shape(src)}, expected {out.shape}")
+        if shift:
+            np.add(src, shift, out=out, casting="unsafe")
+        else:
+            out[...] = src
 
     def nodal(field):
-        return np.concatenate([a for p, q in zip(problems, pads) for a in (field(p), zeros3[:q])])
+        out = np.empty((first[-1], 3))
+        for i, p in enumerate(problems):
+            a, n = first[i], count[i]
+            f = field(p)
+            if f is None:
+                out[a:a + n] = 0.0
+            else:
+                put(out[a:a + n], f)
+            out[a + n:first[i + 1]] = 0.0
+        return out
 
     def build_conn():
-        conn = np.concatenate([p.mesh.conn for p in problems]).astype(np.int32, copy=False)
-        conn += np.repeat(begins[:-1].astype(np.int32), nels)[:, None]
+        conn = np.empty((ebeg[-1], 8), dtype=np.int32)
+        for i, p in enumerate(problems):
+            put(conn[ebeg[i]:ebeg[i + 1]], p.mesh.conn, first[i])
         return conn
 
     def build_mat():
-        local = np.concatenate([p.mesh.mat for p in problems]).astype(np.int32, copy=False)
-        local += np.repeat(np.asarray(gbeg[:-1], dtype=np.int32), nels)
+        local = np.empty(ebeg[-1], dtype=np.int32)
+        for i, p in enumerate(problems):
+            put(local[ebeg[i]:ebeg[i + 1]], p.mesh.mat, gbeg[i])
         return np.asarray(gids, dtype=np.int32)[local]
 
     def build_kbc():
-        # each problem's cards, then its padding nodes' (3 dofs each): node
-        # numbers local to the problem's padding start, then one offset pass
+        # each problem's cards, then its padding nodes' (3 dofs each)
         node3 = np.repeat(np.arange(64, dtype=np.int32), 3)
         dof3 = np.tile(np.arange(3, dtype=np.int32), 64)
-        zero_v = np.zeros(192)
-        nks = np.array([len(p.kbc.nodes) for p in problems], dtype=np.int64)
-        kn = np.concatenate([a for p, q in zip(problems, pads)
-                             for a in (p.kbc.nodes, node3[:3 * q])]).astype(np.int32, copy=False)
-        kd = np.concatenate([a for p, q in zip(problems, pads)
-                             for a in (p.kbc.dofs, dof3[:3 * q])]).astype(np.int32, copy=False)
-        kv = np.concatenate([a for p, q in zip(problems, pads)
-                             for a in (p.kbc.values, zero_v[:3 * q])]).astype(np.float64, copy=False)
-        shift = np.empty(2 * len(problems), dtype=np.int32)
-        shift[0::2] = begins[:-1]               # a problem's own cards
-        shift[1::2] = begins[:-1] + nnds        # its padding nodes
-        lens = np.empty(2 * len(problems), dtype=np.int64)
-        lens[0::2] = nks
-        lens[1::2] = 3 * pads
-        kn += np.repeat(shift, lens)
+        nks = [len(p.kbc.nodes) for p in problems]
+        kbeg = offsets(np.asarray(nks, dtype=np.int64) + 3 * pads)
+        kn, kd = np.empty(kbeg[-1], dtype=np.int32), np.empty(kbeg[-1], dtype=np.int32)
+        kv = np.empty(kbeg[-1])
+        for i, p in enumerate(problems):
+            a, b, e = kbeg[i], kbeg[i] + nks[i], kbeg[i + 1]
+            put(kn[a:b], p.kbc.nodes, first[i])
+            put(kd[a:b], p.kbc.dofs)
+            put(kv[a:b], p.kbc.values)
+            if e > b:
+                put(kn[b:e], node3[:3 * pad[i]], first[i] + count[i])
+                put(kd[b:e], dof3[:3 * pad[i]])
+                kv[b:e] = 0.0
         return KBC(kn, kd, kv)
 
     jobs = [lambda: nodal(lambda p: p.mesh.X), build_conn, build_mat, build_kbc]
     if any(p.u0 is not None for p in problems):
-        jobs.append(lambda: nodal(lambda p: p.u0 if p.u0 is not None else np.zeros_like(p.mesh.X)))
-    if int(begins[-1]) >= max(1 << 16, 2048 * len(problems)):
+        jobs.append(lambda: nodal(lambda p: p.u0))
+    if int(begins[-1]) >= max(1 << 16, 8192 * len(problems)):
         # large problems: the copies release the interpreter lock, so the
         # arrays are built side by side (many small problems would contend
         # for the lock in the list building instead)

@@ -1447,19 +1447,21 @@ __global__ void k_build_src(int nnd, const int* __restrict__ sbase, const int* _
     }
 }
 
-// Lower blocks (column node B < row node A) are the transposes of upper
-// blocks (B, A): the slot k' of column A in row B gives the partner's value
-// index, so the expansion copies them from the operator itself instead of
-// gathering them from MSR rows of other nodes.
-__global__ void k_build_tpos(int nnd, const int* __restrict__ sbase, const int* __restrict__ swidth,
-                             const int* __restrict__ bcol, int* __restrict__ tpos)
+// Partners of the off-diagonal blocks: a lower block's (column < row) is the
+// value index of its upper block, an upper block's -index - 2 of its lower
+// block; -1 for diagonal blocks and padding.  Slot k of a slice's 64 rows per
+// wave, four slots a workgroup at a time; the lower block's lane finds the
+// column and writes both (the pattern is symmetric).
+__global__ void __launch_bounds__(256) k_build_tpos(int nnd, const int* __restrict__ sbase,
+                                                    const int* __restrict__ swidth, const int* __restrict__ bcol,
+                                                    int* __restrict__ tpos)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = a >> 6, l = a & 63;
-    if (s >= (nnd + 63) / 64) return;
-    for (int k = 0; k < swidth[s]; k++) {
+    const int s = blockIdx.x, l = threadIdx.x & 63, a = 64 * s + l;
+    const int w = swidth[s];
+    for (int k = threadIdx.x >> 6; k < w; k += 4) {
         const long g = (long)sbase[s] + k;
         const int B = a < nnd ? bcol[g * 64 + l] : -1;
+        if (B > a) continue;
         int out = -1;
         if (B >= 0 && B < a) {
             // row B lists its neighbours ascending, then padding (-1): a
@@ -1468,9 +1470,11 @@ __global__ void k_build_tpos(int nnd, const int* __restrict__ sbase, const int* 
             int lo = 0, hi = swidth[sB] - 1;
             while (lo <= hi) {
                 const int mid = (lo + hi) >> 1;
-                const int x = bcol[((long)sbase[sB] + mid) * 64 + lB];
+                const long at = ((long)sbase[sB] + mid) * 64 + lB;
+                const int x = bcol[at];
                 if (x == a) {
-                    out = (int)((((long)sbase[sB] + mid) * 9) * 64 + lB);
+                    out = (int)(((long)sbase[sB] + mid) * 9 * 64 + lB);
+                    tpos[at] = -(int)(g * 9 * 64 + l) - 2;
                     break;
                 }
                 if (x >= 0 && x < a)
@@ -1504,9 +1508,7 @@ void launch_build_src(tg_ctx* c)
 
 void launch_build_tpos(tg_ctx* c)
 {
-    const int bs = 256;
-    const long n = 64L * c->op.nslices;
-    hipLaunchKernelGGL(k_build_tpos, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, c->stream, c->nnd,
+    hipLaunchKernelGGL(k_build_tpos, dim3((unsigned)c->op.nslices), dim3(256), 0, c->stream, c->nnd,
                        c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, c->op.d_tpos.p);
     TG_HIP(hipGetLastError());
 }

@@ -16,7 +16,49 @@ namespace tg {
 
 namespace {
 
-constexpr int GB = 64;  // threads per workgroup of the neighbour kernels
+// ---- equation numbers ---------------------------------------------------------
+// NodeManagerT::SetEquationNumbers (tahoe/src/nodes/NodeManagerT.cpp:712-760)
+// -> FieldT::InitEquations/SetEquations (tahoe/src/nodes/FieldT.cpp:635-690):
+// dofs with a kinematic card get none, the others 0.. in node-major, dof-minor
+// order (the interface counts from 1).
+
+__global__ void k_all_active(long n, int* __restrict__ eqn)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) eqn[k] = 1;
+}
+
+__global__ void k_prescribed(long n, const int* __restrict__ idx, int* __restrict__ eqn)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) eqn[idx[k]] = 0;
+}
+
+// eqn: 1 where active, sum: their inclusive sum; mask[a] = node a's active dofs
+__global__ void k_numbers(int nnd, const int* __restrict__ sum, int* __restrict__ eqn, unsigned char* __restrict__ mask)
+{
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a >= nnd) return;
+    int m = 0;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const bool act = eqn[3L * a + i] != 0;
+        eqn[3L * a + i] = act ? sum[3L * a + i] - 1 : -1;
+        m |= act << i;
+    }
+    mask[a] = (unsigned char)m;
+}
+
+// a few integers for the host, written straight into its memory
+__global__ void k_to_host(const int* __restrict__ a, const int* __restrict__ b, const long long* __restrict__ l,
+                          double* __restrict__ out)
+{
+    if (a) out[0] = (double)*a;
+    if (b) out[1] = (double)*b;
+    if (l) out[2] = (double)*l;
+}
+
+// ---- node graph ---------------------------------------------------------------
 
 // incidence k of the connectivity (element k / 8, node conn[k]): count per
 // node into cnt[node + 1]
@@ -48,96 +90,94 @@ __device__ __forceinline__ int candidate(const int* conn, const int* list, int p
     return conn[(long)(list[p0 + (t >> 3)] & ~7) + (t & 7)];
 }
 
+// The distinct values among one wave's n <= 64 K candidates (lane l of pass k
+// holds candidate 64 k + l, lanes past the last one a value above every node):
+// their number, and per held candidate whether it is its value's first
+// occurrence (bit k of first) and how many distinct values lie below it.
+template <int K>
+__device__ __forceinline__ int distinct(int n, const int (&v)[K], int& first, int (&below)[K])
+{
+    const int lane = threadIdx.x & 63;
+    unsigned long long rest[K];  // candidates whose value has not been taken
+    int m = 0;
+    first = 0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        below[k] = 0;
+        rest[k] = __ballot(64 * k + lane < n);
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        while (rest[k]) {
+            const int l = __ffsll(rest[k]) - 1;
+            const int x = __builtin_amdgcn_readlane(v[k], l);
+            m++;
+            first |= (lane == l) << k;
+#pragma unroll
+            for (int q = 0; q < K; q++) {
+                rest[q] &= ~(unsigned long long)__ballot(v[q] == x);
+                below[q] += x < v[q];
+            }
+        }
+    return m;
+}
+
 // FILL = false: deg[a] = the number of distinct candidates of node a (its
 // neighbours, itself included).  FILL = true: those neighbours ascending
-// into nlist[nptr[a] ..).  A node of at most 8 elements (64 candidates)
-// keeps its candidates in its own LDS column and marks first occurrences in
-// a 64-bit mask; a neighbour's place is the number of distinct candidates
-// below it.  A node of 9..64 elements reads its candidates from memory and
-// inserts each new one into its sorted output range.  More than 64
-// elements on a node raise the flag.
+// into nlist[nptr[a] ..), each at the number of distinct candidates below it.
+// One wave per node, its candidates in the lanes' registers.  More than 64
+// elements on a node raise the flag.  Bound by the chain of a node's distinct
+// values (27 inside a grid): 2,200 nodes 8 + 9 us, 1.09 M nodes 325 + 414 us.
+// With a lane per node and its candidates in LDS they took 52 + 122 us (34
+// waves, each with 64 x 64 dependent reads) and 427 + 1,142 us.
 template <bool FILL>
-__global__ void __launch_bounds__(GB) k_neighbours(int nnd, const int* __restrict__ ne_ptr,
-                                                  const int* __restrict__ list, const int* __restrict__ conn,
-                                                  long long* __restrict__ deg, const long long* __restrict__ nptr,
-                                                  int* __restrict__ nlist, int* __restrict__ flag)
+__global__ void __launch_bounds__(256) k_neighbours(int nnd, const int* __restrict__ ne_ptr,
+                                                   const int* __restrict__ list, const int* __restrict__ conn,
+                                                   long long* __restrict__ deg, const long long* __restrict__ nptr,
+                                                   int* __restrict__ nlist, int* __restrict__ flag)
 {
-    __shared__ int cand[64][GB];
-    const int tid = threadIdx.x;
-    const int a = blockIdx.x * GB + tid;
-    if (a >= nnd) return;  // no barrier below: each thread works in its own column
+    const int lane = threadIdx.x & 63;
+    const int a = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (a >= nnd) return;
     const int p0 = ne_ptr[a], ne = ne_ptr[a + 1] - p0;
     if (ne > 64) {
-        if (!FILL) {
+        if (!FILL && lane == 0) {
             atomicOr(flag, 1);
             deg[a] = 0;
         }
         return;
     }
-    const int n = 8 * ne;
-    if (n <= 64) {
-        for (int t = 0; t < n; t++) cand[t][tid] = candidate(conn, list, p0, t);
-        unsigned long long first = 0;
-        for (int t = 0; t < n; t++) {
-            const int x = cand[t][tid];
-            bool f = true;
-            for (int u = 0; u < t; u++) f &= cand[u][tid] != x;
-            if (f) first |= 1ull << t;
+    auto node = [&](auto pass) {
+        constexpr int K = decltype(pass)::value;
+        const int n = 8 * ne;
+        int v[K], below[K], first;
+#pragma unroll
+        for (int k = 0; k < K; k++) v[k] = 64 * k + lane < n ? candidate(conn, list, p0, 64 * k + lane) : 0x7fffffff;
+        const int m = distinct<K>(n, v, first, below);
+        if (FILL) {
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                if ((first >> k) & 1) nlist[nptr[a] + below[k]] = v[k];
+        } else if (lane == 0) {
+            deg[a] = m;
         }
-        if (!FILL) {
-            deg[a] = __popcll(first);
-            return;
-        }
-        const long long o = nptr[a];
-        for (int t = 0; t < n; t++) {
-            if (!((first >> t) & 1ull)) continue;
-            const int x = cand[t][tid];
-            int r = 0;
-            for (int u = 0; u < n; u++) r += (int)((first >> u) & 1ull) & (cand[u][tid] < x ? 1 : 0);
-            nlist[o + r] = x;
-        }
-        return;
-    }
-    if (!FILL) {
-        int m = 0;
-        for (int t = 0; t < n; t++) {
-            const int x = candidate(conn, list, p0, t);
-            bool f = true;
-            for (int u = 0; u < t && f; u++) f = candidate(conn, list, p0, u) != x;
-            m += f ? 1 : 0;
-        }
-        deg[a] = m;
-        return;
-    }
-    const long long o = nptr[a];
-    const int cap = (int)(nptr[a + 1] - o);
-    int m = 0;
-    for (int t = 0; t < n; t++) {
-        const int x = candidate(conn, list, p0, t);
-        int lo = 0, hi = m;  // first entry >= x
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (nlist[o + mid] < x)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        if (lo < m && nlist[o + lo] == x) continue;
-        if (m >= cap) break;  // the count pass saw the same distinct set: never taken
-        for (int v = m; v > lo; v--) nlist[o + v] = nlist[o + v - 1];
-        nlist[o + lo] = x;
-        m++;
-    }
+    };
+    if (ne <= 8)
+        node(std::integral_constant<int, 1>{});
+    else
+        node(std::integral_constant<int, 8>{});
 }
 
-// widest row of each slice of 64 nodes
-__global__ void k_slice_width(int nnd, int nslices, const long long* __restrict__ deg, int* __restrict__ swidth)
+// widest row of each slice of 64 nodes; one wave per slice
+__global__ void __launch_bounds__(256) k_slice_width(int nnd, int nslices, const long long* __restrict__ deg,
+                                                     int* __restrict__ swidth)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const int s = blockIdx.x * 4 + (threadIdx.x >> 6), a = 64 * s + (threadIdx.x & 63);
     if (s >= nslices) return;
-    long long w = 0;
-    for (int a = 64 * s; a < 64 * s + 64 && a < nnd; a++) w = deg[a] > w ? deg[a] : w;
-    swidth[s] = (int)w;
+    int w = a < nnd ? (int)deg[a] : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) w = max(w, __shfl_xor(w, o));
+    if ((threadIdx.x & 63) == 0) swidth[s] = w;
 }
 
 // block columns: row node a (slice s, lane l) lists its neighbours in its
@@ -161,7 +201,8 @@ __global__ void k_block_columns(int nnd, int nslices, const int* __restrict__ sb
 // included, and empty rows.  rl[0] = n_eq + 1 and rl[r + 1] = the length of row r,
 // so that the inclusive sum of rl is bindx[0 .. n_eq].
 __global__ void k_msr_rowlen(int nnd, int n_eq, const long long* __restrict__ nptr, const int* __restrict__ nlist,
-                             const int* __restrict__ eqn, long long* __restrict__ rl)
+                             const int* __restrict__ eqn, const unsigned char* __restrict__ mask,
+                             long long* __restrict__ rl)
 {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a == 0) rl[0] = n_eq + 1;
@@ -170,7 +211,7 @@ __global__ void k_msr_rowlen(int nnd, int n_eq, const long long* __restrict__ np
     int later = 0;
     for (long long k = nptr[a]; k < nptr[a + 1]; k++) {
         const int b = nlist[k];
-        if (b > a) later += (eqn[3L * b] >= 0) + (eqn[3L * b + 1] >= 0) + (eqn[3L * b + 2] >= 0);
+        if (b > a) later += __popc(mask[b]);
     }
     for (int i = 0; i < 3; i++) {
         const int r = eqn[3L * a + i];
@@ -227,8 +268,41 @@ void inclusive_sum(tg_ctx* c, const T* in, T* out, long n)
 
 }  // namespace
 
+// Equation numbers (deqn) and the nodes' masks of active dofs (g_mask) from
+// the prescribed dofs' indices (dkbc_idx).
+void launch_equation_numbers(tg_ctx* c, long nkbc)
+{
+    const long n3 = 3L * c->nnd;
+    int* sum = reinterpret_cast<int*>(c->vwork.p);  // scratch until the first solve
+    c->g_mask.alloc((size_t)c->nnd);
+    hipLaunchKernelGGL(k_all_active, dim3(grid(n3, 256)), dim3(256), 0, c->stream, n3, c->deqn.p);
+    if (nkbc > 0)
+        hipLaunchKernelGGL(k_prescribed, dim3(grid(nkbc, 256)), dim3(256), 0, c->stream, nkbc, c->dkbc_idx.p,
+                           c->deqn.p);
+    inclusive_sum(c, c->deqn.p, sum, n3);
+    hipLaunchKernelGGL(k_numbers, dim3(grid(c->nnd, 256)), dim3(256), 0, c->stream, c->nnd, sum, c->deqn.p,
+                       c->g_mask.p);
+    TG_HIP(hipGetLastError());
+}
+
+// the interface's equation numbers (from 1, prescribed -1), copied when they
+// are first asked for
+const std::vector<int>& host_eqnos(tg_ctx* c)
+{
+    if (!c->eqnos_ready) {
+        c->eqnos.resize(3 * (size_t)c->nnd);
+        TG_HIP(hipMemcpyAsync(c->eqnos.data(), c->deqn.p, sizeof(int) * c->eqnos.size(), hipMemcpyDeviceToHost,
+                              c->stream));
+        TG_HIP(hipStreamSynchronize(c->stream));
+        for (int& e : c->eqnos) e = e >= 0 ? e + 1 : -1;
+        c->eqnos_ready = true;
+    }
+    return c->eqnos;
+}
+
 // Node graph on the device: g_neptr/g_nelist (elements per node), g_deg and
-// g_nptr/g_nlist (sorted unique neighbours per node).
+// g_nptr/g_nlist (sorted unique neighbours per node); n_eq with the graph's
+// size, in one read.
 void device_node_graph(tg_ctx* c)
 {
     const int nnd = c->nnd;
@@ -248,81 +322,69 @@ void device_node_graph(tg_ctx* c)
     TG_HIP(hipMemcpyAsync(c->g_fill.p, c->g_neptr.p, sizeof(int) * nnd, hipMemcpyDeviceToDevice, c->stream));
     hipLaunchKernelGGL(k_ne_fill, dim3(grid(n8, 256)), dim3(256), 0, c->stream, n8, c->dconn.p, c->g_fill.p,
                        c->g_nelist.p);
-    hipLaunchKernelGGL(k_neighbours<false>, dim3(grid(nnd, GB)), dim3(GB), 0, c->stream, nnd, c->g_neptr.p,
+    hipLaunchKernelGGL(k_neighbours<false>, dim3(grid(nnd, 4)), dim3(256), 0, c->stream, nnd, c->g_neptr.p,
                        c->g_nelist.p, c->dconn.p, c->g_deg.p, nullptr, nullptr, c->g_flag.p);
-    TG_HIP(hipGetLastError());
-    int flag = 0;
-    TG_HIP(hipMemcpyAsync(&flag, c->g_flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     // nptr[0] = 0, nptr[a + 1] = deg[0] + .. + deg[a]
     TG_HIP(hipMemsetAsync(c->g_nptr.p, 0, sizeof(long long), c->stream));
     inclusive_sum(c, c->g_deg.p, c->g_nptr.p + 1, (long)nnd);
-    long long total = 0;
-    TG_HIP(hipMemcpyAsync(&total, c->g_nptr.p + nnd, sizeof(long long), hipMemcpyDeviceToHost, c->stream));
+    const int* last_sum = reinterpret_cast<const int*>(c->vwork.p) + (3L * nnd - 1);
+    hipLaunchKernelGGL(k_to_host, dim3(1), dim3(1), 0, c->stream, last_sum, c->g_flag.p, c->g_nptr.p + nnd, c->hscal);
+    TG_HIP(hipGetLastError());
     TG_HIP(hipStreamSynchronize(c->stream));
-    if (flag) fail(TG_OUT_OF_RANGE, "a node is shared by more than 64 elements");
-    if (total > 0x7fffffffLL) fail(TG_OUT_OF_RANGE, "node graph exceeds 32-bit indexing");
-    c->g_nlist.alloc((size_t)total);
-    hipLaunchKernelGGL(k_neighbours<true>, dim3(grid(nnd, GB)), dim3(GB), 0, c->stream, nnd, c->g_neptr.p,
+    c->n_eq = (int)c->hscal[0];
+    if (c->hscal[1] != 0.0) fail(TG_OUT_OF_RANGE, "a node is shared by more than 64 elements");
+    if (c->hscal[2] > 2147483647.0) fail(TG_OUT_OF_RANGE, "node graph exceeds 32-bit indexing");
+    c->g_nlist.alloc((size_t)c->hscal[2]);
+    hipLaunchKernelGGL(k_neighbours<true>, dim3(grid(nnd, 4)), dim3(256), 0, c->stream, nnd, c->g_neptr.p,
                        c->g_nelist.p, c->dconn.p, c->g_deg.p, c->g_nptr.p, c->g_nlist.p, c->g_flag.p);
     TG_HIP(hipGetLastError());
 }
 
-// The solver operator's layout (slice widths and bases, block columns) and
-// the MSR row pointers from the device node graph; the MSR columns, the
-// expansion's value map, the lower blocks' partners and the half-slice
-// value ranges follow.  Allocates the MSR value arrays (their length is
-// known only here).
+// The solver operator's layout (slice widths and bases, block columns, the
+// blocks' partners) and the MSR row pointers from the device node graph.  The
+// MSR columns follow when they are asked for (tg_get_msr_bindx), the
+// expansion's maps when it first runs.  Allocates the MSR value arrays (their
+// length is known only here).
 void device_structure(tg_ctx* c)
 {
     Bsell& B = c->op;
-    const int nnd = c->nnd;
+    const int nnd = c->nnd, n_eq = c->n_eq;
     B.nslices = (nnd + 63) / 64;
     B.d_slice_width.alloc(B.nslices);
-    B.d_slice_base.alloc(B.nslices);
-    hipLaunchKernelGGL(k_slice_width, dim3(grid(B.nslices, 256)), dim3(256), 0, c->stream, nnd, B.nslices,
-                       c->g_deg.p, B.d_slice_width.p);
-    TG_HIP(hipGetLastError());
-    B.slice_width.resize((size_t)B.nslices);
-    TG_HIP(hipMemcpyAsync(B.slice_width.data(), B.d_slice_width.p, sizeof(int) * B.nslices, hipMemcpyDeviceToHost,
-                          c->stream));
-    TG_HIP(hipStreamSynchronize(c->stream));
-    B.slice_base.resize((size_t)B.nslices);
-    long base = 0;
-    for (int s = 0; s < B.nslices; s++) {
-        B.slice_base[s] = (int)base;
-        base += B.slice_width[s];
-    }
-    B.nblocks_padded = base * 64;
-    if (B.nblocks_padded * 9 > 0x7fffffffL) fail(TG_OUT_OF_RANGE, "block operator exceeds 32-bit indexing");
-    TG_HIP(hipMemcpyAsync(B.d_slice_base.p, B.slice_base.data(), sizeof(int) * B.nslices, hipMemcpyHostToDevice,
-                          c->stream));
-    B.d_col.alloc((size_t)B.nblocks_padded);
-    B.d_tpos.alloc((size_t)B.nblocks_padded);
-    B.d_val.alloc((size_t)B.nblocks_padded * 9);
-    hipLaunchKernelGGL(k_block_columns, dim3(grid(64L * B.nslices, 256)), dim3(256), 0, c->stream, nnd, B.nslices,
-                       B.d_slice_base.p, B.d_slice_width.p, c->g_nptr.p, c->g_nlist.p, B.d_col.p);
+    B.d_slice_base.alloc((size_t)B.nslices + 1);
+    hipLaunchKernelGGL(k_slice_width, dim3(grid(B.nslices, 4)), dim3(256), 0, c->stream, nnd, B.nslices, c->g_deg.p,
+                       B.d_slice_width.p);
+    // (the widths' sum is at most the graph's size, which fits an int)
+    TG_HIP(hipMemsetAsync(B.d_slice_base.p, 0, sizeof(int), c->stream));
+    inclusive_sum(c, B.d_slice_width.p, B.d_slice_base.p + 1, (long)B.nslices);
     // MSR row pointers, summed in 64 bits
-    const int n_eq = c->n_eq;
     c->g_rowlen.alloc((size_t)n_eq + 1);
     c->g_rows.alloc((size_t)n_eq + 1);
     TG_HIP(hipMemsetAsync(c->g_rowlen.p, 0, sizeof(long long) * ((size_t)n_eq + 1), c->stream));
     hipLaunchKernelGGL(k_msr_rowlen, dim3(grid(nnd, 256)), dim3(256), 0, c->stream, nnd, n_eq, c->g_nptr.p,
-                       c->g_nlist.p, c->deqn.p, c->g_rowlen.p);
-    TG_HIP(hipGetLastError());
+                       c->g_nlist.p, c->deqn.p, c->g_mask.p, c->g_rowlen.p);
     inclusive_sum(c, c->g_rowlen.p, c->g_rows.p, (long)n_eq + 1);
-    long long len = 0;
-    TG_HIP(hipMemcpyAsync(&len, c->g_rows.p + n_eq, sizeof(long long), hipMemcpyDeviceToHost, c->stream));
+    hipLaunchKernelGGL(k_to_host, dim3(1), dim3(1), 0, c->stream, B.d_slice_base.p + B.nslices, nullptr,
+                       c->g_rows.p + n_eq, c->hscal);
+    TG_HIP(hipGetLastError());
     TG_HIP(hipStreamSynchronize(c->stream));
-    if (len > 0x7fffffffLL) fail(TG_OUT_OF_RANGE, "MSR pattern exceeds 32-bit indexing");
-    c->msr_len = (long)len;
+    B.nblocks_padded = (long)c->hscal[0] * 64;
+    if (B.nblocks_padded * 9 > 0x7fffffffL) fail(TG_OUT_OF_RANGE, "block operator exceeds 32-bit indexing");
+    if (c->hscal[2] > 2147483647.0) fail(TG_OUT_OF_RANGE, "MSR pattern exceeds 32-bit indexing");
+    c->msr_len = (long)c->hscal[2];
+    B.d_col.alloc((size_t)B.nblocks_padded);
+    B.d_tpos.alloc((size_t)B.nblocks_padded);
+    B.d_val.alloc((size_t)B.nblocks_padded * 9);
     c->dbindx.alloc((size_t)c->msr_len);
     c->dval.alloc((size_t)c->msr_len);
     c->dval32.alloc(mixed_stiffness(c) ? (size_t)c->msr_len : 0);
+    hipLaunchKernelGGL(k_block_columns, dim3(grid(64L * B.nslices, 256)), dim3(256), 0, c->stream, nnd, B.nslices,
+                       B.d_slice_base.p, B.d_slice_width.p, c->g_nptr.p, c->g_nlist.p, B.d_col.p);
     hipLaunchKernelGGL(k_narrow, dim3(grid((long)n_eq + 1, 256)), dim3(256), 0, c->stream, (long)n_eq + 1,
                        c->g_rows.p, c->dbindx.p);
     TG_HIP(hipGetLastError());
-    launch_msr_cols(c);  // the MSR columns from the block columns, before anything reads them
     launch_build_tpos(c);
+    c->cols_ready = false;
     c->src_ready = false;
 }
 

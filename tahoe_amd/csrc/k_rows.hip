@@ -62,8 +62,8 @@ __global__ void k_sort_lists(int nnd, const int* __restrict__ ptr, int* __restri
 // diagonal) + mask of its node's active dofs: with the row's pointer, where
 // the block's MSR values are (a slice's rows one after the other)
 __global__ void k_row_upper(int nnd, const int* __restrict__ sbase, const int* __restrict__ swidth,
-                            const int* __restrict__ bcol, const int* __restrict__ eqn, int2* __restrict__ upper,
-                            unsigned short* __restrict__ runs, int* __restrict__ most)
+                            const int* __restrict__ bcol, const unsigned char* __restrict__ act,
+                            int2* __restrict__ upper, unsigned short* __restrict__ runs, int* __restrict__ most)
 {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     int lo = 0, n = 0;
@@ -77,9 +77,7 @@ __global__ void k_row_upper(int nnd, const int* __restrict__ sbase, const int* _
             n++;
             lo += c < a;
             if (c < a) continue;
-            int mask = 0;
-#pragma unroll
-            for (int j = 0; j < 3; j++) mask |= (eqn[3L * c + j] >= 0) << j;
+            const int mask = act[c];
             runs[64L * sbase[s] + (long)l * swidth[s] + k] = (unsigned short)(8 * run + mask);
             if (c > a) run += __popc(mask);
         }
@@ -127,18 +125,7 @@ __global__ void k_row_slots(int nel, const int* __restrict__ conn, const unsigne
     reinterpret_cast<unsigned long long*>(rslot)[t] = out;
 }
 
-// the partner of an upper off-diagonal block, coded -index - 2, beside the
-// lower blocks' partners (which stay >= 0)
-__global__ void k_upper_partners(long n, const int* __restrict__ tpos_in, int* __restrict__ tpos)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int t = tpos_in[i];
-    if (t < 0) return;
-    // value index t = (blk * 9) * 64 + l of the upper block
-    const long blk = (t >> 6) / 9, l = t & 63;
-    tpos[blk * 64 + l] = -(int)(((i >> 6) * 9) * 64 + (i & 63)) - 2;
-}
+__global__ void k_most_to_host(const int* __restrict__ most, double* __restrict__ out) { *out = (double)*most; }
 
 // ---- residual ---------------------------------------------------------------
 
@@ -343,6 +330,7 @@ unsigned grid(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 // FP64 sums (64 KB): a row of a hexahedral grid has 14
 constexpr int ROWS_UP_MOST = 27;
 
+// (the caller waits for the stream before it reads the widest row, hscal[0])
 void rows_structure(tg_ctx* c)
 {
     const int nnd = c->nnd, nel = c->nel;
@@ -354,15 +342,13 @@ void rows_structure(tg_ctx* c)
     c->r_run.alloc((size_t)B.nblocks_padded);
     TG_HIP(hipMemsetAsync(c->g_flag.p, 0, sizeof(int), c->stream));
     hipLaunchKernelGGL(k_row_upper, dim3(grid(nnd, 256)), dim3(256), 0, c->stream, nnd, B.d_slice_base.p,
-                       B.d_slice_width.p, B.d_col.p, c->deqn.p, c->r_upper.p, c->r_run.p, c->g_flag.p);
-    TG_HIP(hipGetLastError());
-    TG_HIP(hipMemcpyAsync(&c->r_up_most, c->g_flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    TG_HIP(hipStreamSynchronize(c->stream));
+                       B.d_slice_width.p, B.d_col.p, c->g_mask.p, c->r_upper.p, c->r_run.p, c->g_flag.p);
     c->r_slot.alloc(64 * (size_t)nel);
     hipLaunchKernelGGL(k_row_slots, dim3(grid(8L * nel, 256)), dim3(256), 0, c->stream, nel, c->dconn.p, c->r_perm.p,
                        B.d_slice_base.p, B.d_col.p, c->r_upper.p, c->r_slot.p);
-    hipLaunchKernelGGL(k_upper_partners, dim3(grid(B.nblocks_padded, 256)), dim3(256), 0, c->stream, B.nblocks_padded,
-                       B.d_tpos.p, B.d_tpos.p);
+    TG_HIP(hipGetLastError());
+    // the widest row decides whether the rows are used: read with the rest
+    hipLaunchKernelGGL(k_most_to_host, dim3(1), dim3(1), 0, c->stream, c->g_flag.p, c->hscal);
     TG_HIP(hipGetLastError());
     c->r_force.alloc(24 * (size_t)nel);
     c->dpart_r.alloc(grid(3L * nnd, 256));

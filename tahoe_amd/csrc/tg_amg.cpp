@@ -160,10 +160,15 @@ void amg_setup(tg_ctx* c)
         g.ptr.swap(ptr);
     }
     std::vector<double> xyz(c->X);
+    const std::vector<int>& eqnos = host_eqnos(c);
+    std::vector<int> sbase((size_t)c->op.nslices);
+    TG_HIP(hipMemcpyAsync(sbase.data(), c->op.d_slice_base.p, sizeof(int) * sbase.size(), hipMemcpyDeviceToHost,
+                          c->stream));
+    TG_HIP(hipStreamSynchronize(c->stream));
     std::vector<char> active((size_t)nnd, 0);
     for (int i = 0; i < nnd; i++)
         for (int k = 0; k < 3; k++)
-            if (c->eqnos[3L * i + k] > 0) active[i] = 1;
+            if (eqnos[3L * i + k] > 0) active[i] = 1;
     std::vector<double> B;  // [n][bs][6] near-null-space rows of the current level (levels >= 1)
 
     AmgLevel* cur = new AmgLevel;
@@ -212,7 +217,7 @@ void amg_setup(tg_ctx* c)
                                  dz = xyz[3L * i + 2] - cen[3L * a + 2];
                     const double rb[3][6] = {{1, 0, 0, 0, dz, -dy}, {0, 1, 0, -dz, 0, dx}, {0, 0, 1, dy, -dx, 0}};
                     for (int p = 0; p < 3; p++)
-                        if (c->eqnos[3L * i + p] > 0)
+                        if (eqnos[3L * i + p] > 0)
                             for (int k = 0; k < 6; k++) rows[6 * p + k] = rb[p][k];
                 } else {
                     std::memcpy(rows, B.data() + (size_t)i * 36, sizeof(double) * 36);
@@ -299,7 +304,7 @@ void amg_setup(tg_ctx* c)
                     int j, fb;
                     if (level == 0) {
                         j = g.adj[g.ptr[i] + k];
-                        fb = (int)(((long)c->op.slice_base[i >> 6] + k) * 64 + (i & 63));
+                        fb = (int)(((long)sbase[i >> 6] + k) * 64 + (i & 63));
                     } else {
                         const int q = (int)(cur->rowptr[i] + k);
                         j = cur->col[q];

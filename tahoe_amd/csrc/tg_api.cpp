@@ -122,7 +122,7 @@ static void require_init(const tg_ctx* c)
     if (!c->initialized) fail(TG_GENERAL_FAIL, "tg_initialize has not been called");
 }
 
-static void build_persist_list(tg_ctx* c);
+static void persist_segments(tg_ctx* c);
 
 // segment of each slice
 std::vector<int> slice_segments(const tg_ctx* c)
@@ -134,8 +134,36 @@ std::vector<int> slice_segments(const tg_ctx* c)
     return out;
 }
 
+// Host-to-device copies of one set-up.  Short ones go through the context's
+// pinned stage while it has room (a pageable copy costs the host 10 us or
+// more); what is copied from elsewhere lives until done().
+struct Upload {
+    tg_ctx* c;
+    size_t used = 0;
+    std::vector<std::vector<int>> kept;
+    explicit Upload(tg_ctx* ctx) : c(ctx) {}
+    ~Upload() { done(); }
+    void operator()(void* dst, const void* src, size_t bytes)
+    {
+        if (bytes == 0) return;
+        if (used + bytes <= sizeof(double) * HOST_STAGE) {
+            char* at = reinterpret_cast<char*>(c->hstage) + used;
+            std::memcpy(at, src, bytes);
+            used += (bytes + 63) / 64 * 64;
+            src = at;
+        }
+        TG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+    }
+    void operator()(int* dst, std::vector<int>&& v)
+    {
+        kept.push_back(std::move(v));
+        (*this)(dst, kept.back().data(), sizeof(int) * kept.back().size());
+    }
+    void done() { (void)hipStreamSynchronize(c->stream); }
+};
+
 // Segment tables: slice -> segment, segment -> first slice and group.
-static void setup_segments(tg_ctx* c)
+static void setup_segments(tg_ctx* c, Upload& up)
 {
     Segments& S = c->seg;
     if (S.node_begin.size() != (size_t)S.nseg + 1 || S.node_begin.back() != c->nnd) {
@@ -146,7 +174,7 @@ static void setup_segments(tg_ctx* c)
     std::vector<int> seg_slice((size_t)S.nseg + 1);
     for (int g = 0; g < S.nseg; g++) seg_slice[g] = S.node_begin[g] / 64;
     seg_slice[S.nseg] = (int)S.nslices;
-    const std::vector<int> slice_seg = slice_segments(c);
+    std::vector<int> slice_seg = slice_segments(c);
     // every element inside one segment
     int straddle = 0;
     if (S.nseg > 1)
@@ -157,7 +185,7 @@ static void setup_segments(tg_ctx* c)
                 for (int a = 1; a < 8; a++) bad |= slice_seg[c->conn[8 * e + a] >> 6] != g;
             }
             if (bad) __atomic_store_n(&straddle, 1, __ATOMIC_RELAXED);
-        });
+        }, 1L << 14);
     if (straddle) fail(TG_BAD_INPUT, "element connects two segments");
     S.d_slice_seg.alloc((size_t)S.nslices);
     S.d_seg_slice.alloc((size_t)S.nseg + 1);
@@ -166,44 +194,39 @@ static void setup_segments(tg_ctx* c)
     S.max_slices = 0;
     for (int g = 0; g < S.nseg; g++) S.max_slices = std::max(S.max_slices, (long)(seg_slice[g + 1] - seg_slice[g]));
     std::vector<int> seg_grp((size_t)S.nseg + 1, 0);
-    std::vector<int4> grp;
-    grp.reserve((size_t)S.nslices / 4 + S.nseg);
+    std::vector<int> grp;  // int4 rows
+    grp.reserve((size_t)S.nslices + 4 * (size_t)S.nseg);
     for (int g = 0; g < S.nseg; g++) {
         for (int s = seg_slice[g]; s < seg_slice[g + 1]; s += 4)
-            grp.push_back(make_int4(s, std::min(4, seg_slice[g + 1] - s), g, 0));
-        seg_grp[g + 1] = (int)grp.size();
+            grp.insert(grp.end(), {s, std::min(4, seg_slice[g + 1] - s), g, 0});
+        seg_grp[g + 1] = (int)(grp.size() / 4);
     }
-    S.ngroups = (long)grp.size();
+    S.ngroups = (long)(grp.size() / 4);
     S.d_seg_grp.alloc(seg_grp.size());
-    S.d_grp.alloc(grp.size());
+    S.d_grp.alloc(grp.size() / 4);
     S.d_part.alloc(3 * (size_t)S.nslices);
     S.d_out.alloc((size_t)S.nseg);
     S.d_ndone.alloc(1);
     S.d_segstat.alloc((size_t)S.nseg);
     S.h_scal.assign((size_t)S_NSCAL * S.nseg, 0.0);
     S.d_persist.alloc((size_t)S.nseg);
-    std::vector<int> ones((size_t)S.nseg, 1);
-    auto up = [&](int* dst, const std::vector<int>& v) {
-        TG_HIP(hipMemcpyAsync(dst, v.data(), sizeof(int) * v.size(), hipMemcpyHostToDevice, c->stream));
-    };
-    up(S.d_slice_seg.p, slice_seg);
-    up(S.d_seg_slice.p, seg_slice);
-    up(S.d_seg_grp.p, seg_grp);
-    TG_HIP(hipMemcpyAsync(S.d_grp.p, grp.data(), sizeof(int4) * grp.size(), hipMemcpyHostToDevice, c->stream));
-    up(S.d_active.p, ones);
+    up(S.d_slice_seg.p, std::move(slice_seg));
+    up(S.d_seg_slice.p, std::move(seg_slice));
+    up(S.d_seg_grp.p, std::move(seg_grp));
+    up(reinterpret_cast<int*>(S.d_grp.p), std::move(grp));
+    up(S.d_active.p, std::vector<int>((size_t)S.nseg, 1));
     TG_HIP(hipMemsetAsync(S.d_scal.p, 0, sizeof(double) * S_NSCAL * S.nseg, c->stream));
     TG_HIP(hipMemsetAsync(S.d_segstat.p, 0, sizeof(int) * S.nseg, c->stream));
-    // every copy and clear of the context goes through its own stream (a
-    // null-stream operation is not ordered with a non-blocking stream), and
-    // the host vectors copied from must outlive the copies
-    TG_HIP(hipStreamSynchronize(c->stream));
-    build_persist_list(c);
+    // (every copy and clear of the context goes through its own stream: a
+    // null-stream operation is not ordered with a non-blocking stream)
+    persist_segments(c);
+    if (!S.h_persist.empty()) up(S.d_persist.p, S.h_persist.data(), sizeof(int) * S.h_persist.size());
 }
 
 // Segments of at most pcg_persist(c) slices, for the persistent PCG kernel.
 // The device list holds every segment's room (allocated with the segment
 // tables), so a rebuild only copies.
-static void build_persist_list(tg_ctx* c)
+static void persist_segments(tg_ctx* c)
 {
     Segments& S = c->seg;
     const int thr = std::min(pcg_persist(c), PCG_PERSIST_MAX);
@@ -214,12 +237,18 @@ static void build_persist_list(tg_ctx* c)
             const long se = g + 1 < S.nseg ? S.node_begin[g + 1] / 64 : S.nslices;
             if (se - sb <= thr) S.h_persist.push_back(g);
         }
+    S.persist_built = pcg_persist(c);
+}
+
+static void build_persist_list(tg_ctx* c)
+{
+    Segments& S = c->seg;
+    persist_segments(c);
     if (!S.h_persist.empty()) {
         TG_HIP(hipMemcpyAsync(S.d_persist.p, S.h_persist.data(), sizeof(int) * S.h_persist.size(),
                               hipMemcpyHostToDevice, c->stream));
         TG_HIP(hipStreamSynchronize(c->stream));  // h_persist outlives its copy
     }
-    S.persist_built = pcg_persist(c);
 }
 
 void drop_pcg_graph(tg_ctx* c)
@@ -401,7 +430,7 @@ int tg_set_mesh(tg_ctx* c, int nnd, int nel, const double* X, const int* conn, c
                 if (mat) f |= mat[e] < 0 ? 4 : 0;
             }
             if (f) __atomic_fetch_or(&found, f, __ATOMIC_RELAXED);
-        });
+        }, 1L << 13);
         if (found & 1) fail(TG_OUT_OF_RANGE, "connectivity refers to a missing node");
         if (found & 2) fail(TG_BAD_INPUT, "degenerate element (repeated node) is not supported");
         if (found & 4) fail(TG_BAD_INPUT, "negative material id");
@@ -531,7 +560,7 @@ int tg_set_kbc(tg_ctx* c, int nkbc, const int* nodes, const int* dofs, const dou
 // Device storage of the mesh and the vectors, and the uploads that need
 // neither the node graph nor the colouring (tg_initialize colours the
 // elements on another host thread meanwhile).
-static void upload_mesh(tg_ctx* c, int nmat)
+static void upload_mesh(tg_ctx* c, int nmat, Upload& up)
 {
     // device storage
     const size_t nn = 3 * (size_t)c->nnd;
@@ -546,30 +575,22 @@ static void upload_mesh(tg_ctx* c, int nmat)
     for (auto* v : {&c->vx, &c->vr, &c->vz, &c->vp, &c->vq, &c->vdinv, &c->vwork}) v->alloc(nn);
     const size_t sblocks = ((size_t)c->nnd + 255) / 256;
     c->dpart.alloc(2 * std::max<size_t>(sblocks, 1024) + 16);
-    std::vector<int> eqn0(nn);
-    for (size_t k = 0; k < nn; k++) eqn0[k] = c->eqnos[k] > 0 ? c->eqnos[k] - 1 : -1;
     std::vector<double2> props((size_t)std::max(1, nmat));
     for (int m = 0; m < nmat; m++) props[m] = make_double2(c->mu[m], c->kappa[m]);
     std::vector<int> kidx(c->kbc_nodes.size());
     for (size_t k = 0; k < kidx.size(); k++) kidx[k] = 3 * c->kbc_nodes[k] + c->kbc_dofs[k];
     c->dkbc_idx.alloc(kidx.size());
     c->dkbc_val.alloc(kidx.size());
-    TG_HIP(hipMemcpyAsync(c->dX.p, c->X.data(), sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
+    c->hprops = std::move(props);
+    up(c->dmatprops.p, c->hprops.data(), sizeof(double2) * c->hprops.size());
+    up(c->dkbc_val.p, c->kbc_vals.data(), sizeof(double) * kidx.size());
+    up(c->dmat.p, c->mat.data(), sizeof(int) * c->mat.size());
+    up(c->dkbc_idx.p, std::move(kidx));
+    up(c->dX.p, c->X.data(), sizeof(double) * nn);
+    up(c->dconn.p, c->conn.data(), sizeof(int) * c->conn.size());
     TG_HIP(hipMemsetAsync(c->du.p, 0, sizeof(double) * nn, c->stream));
     TG_HIP(hipMemsetAsync(c->du_last.p, 0, sizeof(double) * nn, c->stream));
-    TG_HIP(hipMemcpyAsync(c->dconn.p, c->conn.data(), sizeof(int) * c->conn.size(), hipMemcpyHostToDevice,
-                          c->stream));
-    TG_HIP(hipMemcpyAsync(c->dmat.p, c->mat.data(), sizeof(int) * c->mat.size(), hipMemcpyHostToDevice, c->stream));
-    TG_HIP(hipMemcpyAsync(c->deqn.p, eqn0.data(), sizeof(int) * nn, hipMemcpyHostToDevice, c->stream));
-    TG_HIP(hipMemcpyAsync(c->dmatprops.p, props.data(), sizeof(double2) * props.size(), hipMemcpyHostToDevice,
-                          c->stream));
-    if (!kidx.empty()) {
-        TG_HIP(hipMemcpyAsync(c->dkbc_idx.p, kidx.data(), sizeof(int) * kidx.size(), hipMemcpyHostToDevice,
-                              c->stream));
-        TG_HIP(hipMemcpyAsync(c->dkbc_val.p, c->kbc_vals.data(), sizeof(double) * kidx.size(),
-                              hipMemcpyHostToDevice, c->stream));
-    }
-    TG_HIP(hipStreamSynchronize(c->stream));  // the host sources above are locals
+    launch_equation_numbers(c, (long)c->kbc_nodes.size());
 }
 
 int tg_initialize(tg_ctx* c, int* n_eq, long* msr_len)
@@ -593,9 +614,9 @@ int tg_initialize(tg_ctx* c, int* n_eq, long* msr_len)
         drop_pcg_graph(c);
         c->dfext.release();
         SetupTrace phase(c, "tg_initialize");
-        // equations and segments on the host, then the structure on the device
-        c->n_eq = equation_numbers(c->nnd, c->kbc_nodes, c->kbc_dofs, c->eqnos);
-        phase("equation numbers");
+        // segments on the host, the rest on the device
+        Upload up(c);
+        c->eqnos_ready = false;
         c->stiff_chunk_built = -2;
         c->gather_built = -2;
         c->dgptr.release();
@@ -604,16 +625,18 @@ int tg_initialize(tg_ctx* c, int* n_eq, long* msr_len)
         c->debuf32.release();
         c->colours_ready = false;
         c->op_fresh = false;
-        setup_segments(c);
+        setup_segments(c, up);
         phase("segments");
-        upload_mesh(c, nmat);
-        phase("mesh upload");
+        upload_mesh(c, nmat, up);
+        phase("mesh upload, equations");
         device_node_graph(c);
         device_structure(c);
         const bool mixed = mixed_operator(c);
         c->op.d_diag.alloc((size_t)c->nnd);
         launch_build_operator_diag(c);
         rows_structure(c);
+        TG_HIP(hipStreamSynchronize(c->stream));
+        c->r_up_most = (int)c->hscal[0];
         if (rows_assembly(c)) rows_buffers(c);
         phase("structure");
         c->vbinv.alloc(c->precond == TG_PC_BLOCK_JACOBI ? 9 * (size_t)c->nnd : 0);
@@ -635,17 +658,23 @@ int tg_get_eqnos(const tg_ctx* c, int* eqnos)
 {
     if (!c || !eqnos) return TG_BAD_INPUT;
     if (!c->initialized) return TG_GENERAL_FAIL;
-    std::memcpy(eqnos, c->eqnos.data(), sizeof(int) * c->eqnos.size());
-    return TG_OK;
+    tg_ctx* m = const_cast<tg_ctx*>(c);
+    return guarded(m, [&] {
+        const std::vector<int>& e = host_eqnos(m);
+        std::memcpy(eqnos, e.data(), sizeof(int) * e.size());
+    });
 }
 
 int tg_get_msr_bindx(const tg_ctx* c, int* bindx)
 {
     if (!c || !bindx) return TG_BAD_INPUT;
     if (!c->initialized) return TG_GENERAL_FAIL;
-    // the pattern lives on the device (its columns are written there)
+    // the pattern lives on the device; its columns are written there when
+    // they are first asked for
     tg_ctx* m = const_cast<tg_ctx*>(c);
     return guarded(m, [&] {
+        if (!m->cols_ready) launch_msr_cols(m);
+        m->cols_ready = true;
         TG_HIP(hipMemcpyAsync(bindx, m->dbindx.p, sizeof(int) * (size_t)m->msr_len, hipMemcpyDeviceToHost, m->stream));
         TG_HIP(hipStreamSynchronize(m->stream));
     });

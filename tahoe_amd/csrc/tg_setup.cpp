@@ -1,5 +1,4 @@
-// Host-side setup of the equation system: equation numbers, element
-// colouring, and the node graph the multigrid's aggregation reads (the
+// Host-side setup of the equation system: element colouring and the node graph the multigrid's aggregation reads (the
 // operator's structure itself is built on the device, k_graph.hip).  Runs
 // once per mesh (the reference does the same work in
 // FEManagerT::SetEquationSystem, tahoe/src/main/FEManagerT.cpp:2248-2313).
@@ -10,20 +9,6 @@
 #include "tg_internal.h"
 
 namespace tg {
-
-// NodeManagerT::SetEquationNumbers (tahoe/src/nodes/NodeManagerT.cpp:712-760)
-// -> FieldT::InitEquations/SetEquations (tahoe/src/nodes/FieldT.cpp:635-690):
-// dofs with a kinematic card get -1, the others 1.. in node-major, dof-minor
-// order.
-int equation_numbers(int nnd, const std::vector<int>& kn, const std::vector<int>& kd, std::vector<int>& eqnos)
-{
-    eqnos.assign((size_t)nnd * 3, 0);
-    for (size_t k = 0; k < kn.size(); k++) eqnos[(size_t)kn[k] * 3 + kd[k]] = -1;
-    int n = 0;
-    for (auto& e : eqnos)
-        if (e == 0) e = ++n;
-    return n;
-}
 
 // node -> incident elements (CSR).  Counted and filled by all workers with
 // atomic increments, so the order of a node's elements varies from run to
