@@ -304,7 +304,8 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
  *                      from 98,304 nodes, else 0 (there, untuned, several
  *                      waves share a row's blocks). */
 /* TG_TUNE_AMG_DEGREE   multigrid: Chebyshev degree of each pre- and
- *                      post-smoothing pass, 2 (default) .. 4. */
+ *                      post-smoothing pass, 2 (default) .. 4.  Until it is
+ *                      set, levels of 393,216 and more dofs take one step. */
 /* TG_TUNE_AMG_WEIGHT   multigrid: weight of the coarse-grid correction in
  *                      percent, 100 .. 190 (default 150: unsmoothed
  *                      aggregation under-corrects; any weight in (0, 2)

@@ -25,6 +25,10 @@ constexpr int AB = 256;          // threads per block of the vector/level kernel
 // to 1e-10): ratio 30 94 / 82 / 141, 16 87 / 78 / 132, 12 87 / 78 / 131, 8 91 /
 // 80 / 133, 4 101 / 87 / 148.
 constexpr double CHEB_RATIO = 14.0;
+// With one step (amg_level_degree) the interval is [lmax / 4, lmax], a damped
+// Jacobi step with 1.6 / lmax: 128^3 mixed, fine and first coarse level so,
+// PCG iterations of a Newton step: ratio 4 109, 10 114; 96^3: 3 112, 4 112.
+constexpr double JACOBI_RATIO = 4.0;
 constexpr double CHEB_BOOST = 1.1;
 constexpr int POWER_ITS = 12;
 
@@ -133,6 +137,16 @@ struct EFirst {
 struct EResid {  // r -= A d
     double* r;
     __device__ __forceinline__ void operator()(long j, double q) const { r[j] -= q; }
+};
+struct EDefect {  // r = f - A x
+    const double* f;
+    double* r;
+    __device__ __forceinline__ void operator()(long j, double q) const { r[j] = f[j] - q; }
+};
+struct EJacobi {  // x = x0 + D^-1 (f - A x0) / theta
+    const double *dinv, *f, *coef, *x0;
+    double* x;
+    __device__ __forceinline__ void operator()(long j, double q) const { x[j] = x0[j] + coef[0] * dinv[j] * (f[j] - q); }
 };
 struct EPost {  // start of post-smoothing: r = f - A x; d0 = D^-1 r / theta
     const double *dinv, *f, *coef;
@@ -467,6 +481,20 @@ static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const doub
     }
 }
 
+// Chebyshev degree of a level's smoothing passes.  Untuned, the levels that
+// memory bounds take one step, two products a cycle instead of four: the PCG
+// iterations grow by a fifth and each costs two fifths less.  Mixed precision,
+// ms a Newton step and PCG iterations, degree 2 everywhere / 1 at the fine level
+// / 1 at the first coarse level too: 128^3 440 (86) / 379 (99) / 341 (109), 96^3
+// 214 / 180 / 170, 80^3 127 / 110 / 108, 56^3 50.8 / 46.7 / 47.8, 48^3 27.4 /
+// 26.8 / 27.5, 32^3 16.8 / 17.2 / 17.9.  So from 3 * 2^17 dofs of a level: 2^17
+// nodes of the fine one, 2^16 of a coarse one.
+static int level_degree(const tg_ctx* c, int l)
+{
+    const AmgLevel& A = *c->amg.lv[l];
+    return c->amg.degree_auto && (long)A.n * A.bs >= 3L << 17 ? 1 : c->amg.degree;
+}
+
 static double* level_dinv(tg_ctx* c, int l) { return l == 0 ? c->vdinv.p : c->amg.lv[l]->dinv; }
 
 static void reduce(tg_ctx* c, int kind, long nd, const double* a, const double* b, double* out)
@@ -602,12 +630,13 @@ static void amg_numeric_t(tg_ctx* c, const MT* val0)
         if (!(lmax > 0.0) || !std::isfinite(lmax)) lmax = 1.0;
         lmax *= CHEB_BOOST;
         G.lv[l]->lmax = lmax;
-        const double lmin = lmax / CHEB_RATIO;
+        const int degree = level_degree(c, l);
+        const double lmin = lmax / (degree == 1 ? JACOBI_RATIO : CHEB_RATIO);
         const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin), sigma = theta / delta;
         double* cf = coef.data() + 8 * l;
         cf[0] = 1.0 / theta;
         double rho = 1.0 / sigma;
-        for (int s = 1; s < G.degree; s++) {
+        for (int s = 1; s < degree; s++) {
             const double rn = 1.0 / (2.0 * sigma - rho);
             cf[2 * s - 1] = rn * rho;
             cf[2 * s] = 2.0 * rn / delta;
@@ -624,7 +653,7 @@ static void amg_numeric_t(tg_ctx* c, const MT* val0)
 // The multigrid works on the FP32 copy of the fine operator in either
 // precision (the solver's own operator when it is FP32; refreshed from the
 // FP64 one by the caller otherwise): a preconditioner needs no more, and the
-// smoother's four fine-level products per cycle move half the bytes.
+// smoother's fine-level products (two to four a cycle) move half the bytes.
 // The coarse levels' numeric set-up (Galerkin products, smoother intervals,
 // coarsest inverse) for the current fine operator.  With reuse = k > 0 one
 // set-up serves the next k tangents of the same Newton solve too: the
@@ -646,14 +675,20 @@ void amg_numeric(tg_ctx* c)
     G.since = 0;
 }
 
+// pre-smoothing from zero, then r = f - A x; with one step x stays in d0
 static void smooth_down(tg_ctx* c, int l, const double* f, double* x, AmgLevel& A, const double* cf, const double* done)
 {
     const double* dinv = level_dinv(c, l);
     const long nd = (long)A.n * A.bs;
+    const int degree = level_degree(c, l);
     double *dp = A.d_d1.p, *dn = A.d_d0.p;
     hipLaunchKernelGGL(k_amg_pre, dim3(blocks_for(nd)), dim3(AB), 0, c->stream, nd, dinv, f, cf, dn, done);
+    if (degree == 1) {
+        level_rows(c, l, dn, EDefect{f, A.d_r.p}, done);
+        return;
+    }
     level_rows(c, l, dn, EFirst{dinv, f, cf, dn, dp, A.d_r.p, x}, done);
-    for (int s = 2; s < c->amg.degree; s++) {
+    for (int s = 2; s < degree; s++) {
         level_rows(c, l, dp, EStep{dinv, dp, cf, dn, A.d_r.p, x, 2 * s - 1, 0}, done);
         std::swap(dp, dn);
     }
@@ -663,9 +698,14 @@ static void smooth_down(tg_ctx* c, int l, const double* f, double* x, AmgLevel& 
 static void smooth_up(tg_ctx* c, int l, const double* f, double* x, AmgLevel& A, const double* cf, const double* done)
 {
     const double* dinv = level_dinv(c, l);
+    const int degree = level_degree(c, l);
+    if (degree == 1) {
+        level_rows(c, l, A.d_d0.p, EJacobi{dinv, f, cf, A.d_d0.p, x}, done);
+        return;
+    }
     level_rows(c, l, x, EPost{dinv, f, cf, A.d_r.p, A.d_d0.p}, done);
     double *dp = A.d_d0.p, *dn = A.d_d1.p;
-    for (int s = 1; s < c->amg.degree; s++) {
+    for (int s = 1; s < degree; s++) {
         level_rows(c, l, dp, EStep{dinv, dp, cf, dn, A.d_r.p, x, 2 * s - 1, s == 1 ? 1 : 0}, done);
         std::swap(dp, dn);
     }
@@ -697,9 +737,10 @@ void amg_vcycle(tg_ctx* c, const double* f0, double* z, const double* done)
         AmgLevel& A = *G.lv[l];
         AmgLevel& C = *G.lv[l + 1];
         double* x = l == 0 ? z : A.d_x.p;
+        double* xp = level_degree(c, l) == 1 ? A.d_d0.p : x;
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(blocks_for((long)A.n * A.bs)), dim3(AB), 0, c->stream, A.n, A.d_agg.p,
-                               A.d_P.p, C.d_x.p, 0.01 * G.weight, x, done);
+                               A.d_P.p, C.d_x.p, 0.01 * G.weight, xp, done);
         };
         if (l == 0)
             go(k_amg_prolong<3>);

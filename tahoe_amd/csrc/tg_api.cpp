@@ -1222,6 +1222,7 @@ int tg_set_tuning(tg_ctx* c, int knob, long value)
         } else if (knob == TG_TUNE_AMG_DEGREE) {
             if (value < 2 || value > 4) fail(TG_OUT_OF_RANGE, "multigrid smoother degree must be 2..4");
             c->amg.degree = (int)value;
+            c->amg.degree_auto = false;
             c->amg.gen++;
             c->amg.since = -1;
         } else if (knob == TG_TUNE_AMG_WEIGHT) {

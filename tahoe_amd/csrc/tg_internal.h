@@ -219,6 +219,7 @@ struct AmgLevel {
 struct Amg {
     int gen = 0;                             // bumped on every rebuild or knob change (captured PCG graphs key on it)
     int degree = 2;                          // Chebyshev degree per smoothing pass
+    bool degree_auto = true;                 // not set by the caller: large levels take one step (k_amg.hip: level_degree)
     int weight = 150;                        // coarse-grid correction weight, percent
     int reuse = 6;                           // further tangents of one Newton solve served by one numeric set-up
                                              // of the coarse levels (a 128^3 Newton step: 1.4x faster, fewer PCG

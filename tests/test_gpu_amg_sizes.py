@@ -30,3 +30,30 @@ def test_amg_solve_equals_jacobi(n):
         assert np.abs(x1 - x0).max() <= 1e-7 * np.abs(x0).max()
     finally:
         s.close()
+
+
+def test_amg_one_step_on_two_levels():
+    """From 65,536 nodes of the first coarse level (81^3 elements: 68,921) it
+    takes one smoothing step too, as the fine level does; with the degree set
+    by the caller both take Chebyshev passes.  Either gives the solution."""
+    from tahoe_amd import api, mesh as M
+    m = M.cube(81, seed=8)
+    kbc = M.kbc_uniaxial(m, 0.002)
+    s = api.Solid(0)
+    try:
+        s.set_mesh(m.X, m.conn, m.mat)
+        s.set_material(0, *api.mu_kappa(1000.0, 0.3))
+        s.set_kbc(kbc.nodes, kbc.dofs, kbc.values)
+        s.set_preconditioner(api.PC_AMG)
+        s.initialize()
+        s.apply_kbc(1.0)
+        R, _ = s.form_rhs()
+        s.form_lhs()
+        x0, st0 = s.solve(R, rtol=1e-11)
+        s.set_tuning(api.TUNE_AMG_DEGREE, 2)
+        x1, st1 = s.solve(R, rtol=1e-11)
+        assert st0.converged and st1.converged and st1.iterations < st0.iterations < 2 * st1.iterations
+        # residuals below 1e-11 of R, condition number < 1e5
+        assert np.abs(x1 - x0).max() <= 1e-6 * np.abs(x0).max()
+    finally:
+        s.close()
