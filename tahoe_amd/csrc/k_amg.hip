@@ -73,29 +73,50 @@ struct Op0 {
     }
 };
 
-// Levels >= 1: sliced 6x6 FP32 blocks (slot e of a slice: its 36 values at
-// val[(e / 64) * 2304 + comp * 64 + e % 64], coalesced over the slice's 64
-// rows; padding zero), one lane per node and 6 outputs.
+// Levels >= 1: sliced 6x6 FP32 blocks, one lane per node and 6 outputs.  The
+// values of a slot are kept as nine groups of four, a group's 64 lanes side by
+// side (amg_at), so a lane takes a block by nine 16-byte loads; padding slots
+// are zero.  SYM: a lower block (column below the row) is read as its upper
+// partner's transpose, slot part[slot], of the same bits: half the level's
+// values come from HBM and half from the caches.  16-byte loads make that pay:
+// a partner's lanes start anywhere in a cache line, so a 256-byte load of 64
+// floats takes three lines for two, one of 1 KB nine for eight.  65^3 nodes
+// (1.07 GB): 236 us with 4-byte loads, 216 with 16-byte ones, 175 so; with
+// 4-byte loads the symmetric read took 266.
+template <bool SYM>
 struct OpC {
     static constexpr int NC = 6;
     int n;
     const int* sbase;
     const int* swidth;
     const int* col;
+    const int* part;
     const float* val;
     __device__ __forceinline__ void add(long b0, int k0, int k1, int l, int t, const double* __restrict__ x, double (&y)[6]) const
     {
+#pragma unroll(SYM ? 3 : 1)
         for (int q = k0; q < k1; q++) {
-            const int cr = col[(b0 + q) * 64 + l];
+            int e = (int)(b0 + q) * 64 + l;
+            const int cr = col[e];
             const int c = cr < 0 ? t : cr;
+            const bool tr = SYM && c < t;
+            if (tr) e = part[e];
+            float u[36];
             double xc[6];
 #pragma unroll
+            for (int m = 0; m < 9; m++) {
+                const float4 g = *(const float4*)(val + amg_at(e, 4 * m));
+                u[4 * m] = g.x;
+                u[4 * m + 1] = g.y;
+                u[4 * m + 2] = g.z;
+                u[4 * m + 3] = g.w;
+            }
+#pragma unroll
             for (int j = 0; j < 6; j++) xc[j] = x[6L * c + j];
-            const float* v = val + (b0 + q) * 2304 + l;
 #pragma unroll
             for (int r = 0; r < 6; r++)
 #pragma unroll
-                for (int j = 0; j < 6; j++) y[r] += (double)v[(6 * r + j) * 64] * xc[j];
+                for (int j = 0; j < 6; j++) y[r] += (double)(tr ? u[6 * j + r] : u[6 * r + j]) * xc[j];
         }
     }
 };
@@ -315,8 +336,8 @@ __global__ void __launch_bounds__(AB) k_amg_rap0(long nup, const int* __restrict
         s += t;
     }
     const int ab = up[2 * u], ba = up[2 * u + 1];
-    cval[(long)(ab >> 6) * 2304 + (ab & 63) + (6 * r + c) * 64] = (float)s;
-    if (ba >= 0) cval[(long)(ba >> 6) * 2304 + (ba & 63) + (6 * c + r) * 64] = (float)s;
+    cval[amg_at(ab, 6 * r + c)] = (float)s;
+    if (ba >= 0) cval[amg_at(ba, 6 * c + r)] = (float)s;
 }
 
 // Galerkin product, fine level = a sliced 6x6 level
@@ -333,7 +354,6 @@ __global__ void __launch_bounds__(AB) k_amg_rapc(long nup, const int* __restrict
     for (long e = gptr[u]; e < gptr[u + 1]; e++) {
         const int fb = gl[2 * e], i = gl[2 * e + 1];
         const int j = fcol[fb];
-        const float* v = fval + (long)(fb >> 6) * 2304 + (fb & 63);
         const float* pi = P + (long)i * 36 + r;
         const float* pj = P + (long)j * 36 + c;
         double t = 0.0;
@@ -341,14 +361,14 @@ __global__ void __launch_bounds__(AB) k_amg_rapc(long nup, const int* __restrict
         for (int p = 0; p < 6; p++) {
             double ap = 0.0;
 #pragma unroll
-            for (int q = 0; q < 6; q++) ap += (double)v[(6 * p + q) * 64] * pj[6 * q];
+            for (int q = 0; q < 6; q++) ap += (double)fval[amg_at(fb, 6 * p + q)] * pj[6 * q];
             t += (double)pi[6 * p] * ap;
         }
         s += t;
     }
     const int ab = up[2 * u], ba = up[2 * u + 1];
-    cval[(long)(ab >> 6) * 2304 + (ab & 63) + (6 * r + c) * 64] = (float)s;
-    if (ba >= 0) cval[(long)(ba >> 6) * 2304 + (ba & 63) + (6 * c + r) * 64] = (float)s;
+    cval[amg_at(ab, 6 * r + c)] = (float)s;
+    if (ba >= 0) cval[amg_at(ba, 6 * c + r)] = (float)s;
 }
 
 // inverse diagonal of a sliced 6x6 level (0 for inactive dofs)
@@ -359,7 +379,7 @@ __global__ void __launch_bounds__(AB) k_amg_dinv(int n, const int* __restrict__ 
     if (t >= 6L * n) return;
     const int a = (int)(t / 6), r = (int)(t - 6L * a);
     const int e = diagblk[a];
-    const double d = (double)val[(long)(e >> 6) * 2304 + (e & 63) + 7 * r * 64];
+    const double d = (double)val[amg_at(e, 7 * r)];
     dinv[t] = d > 0.0 ? 1.0 / d : 0.0;
 }
 
@@ -444,7 +464,11 @@ constexpr int NPART = 1024;
 // host side
 // ---------------------------------------------------------------------------
 
-static OpC opc(const AmgLevel& L) { return OpC{L.n, L.d_sbase.p, L.d_swidth.p, L.d_col.p, L.d_val.p}; }
+template <bool SYM>
+static OpC<SYM> opc(const AmgLevel& L)
+{
+    return {L.n, L.d_sbase.p, L.d_swidth.p, L.d_col.p, L.d_part.p, L.d_val.p};
+}
 
 template <class Op, class E>
 static void launch_rows(tg_ctx* c, const Op& op, const double* x, const E& e, const double* done, int nw)
@@ -470,8 +494,11 @@ static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const doub
 {
     const Bsell& B = c->op;
     if (l > 0) {
-        const OpC op = opc(*c->amg.lv[l]);
-        launch_rows(c, op, x, e, done, op.n <= 64 * 640 ? 9 : op.n <= 64 * 2048 ? 3 : 1);
+        const AmgLevel& A = *c->amg.lv[l];
+        if (A.n >= AMG_SYM_NODES)
+            launch_rows(c, opc<true>(A), x, e, done, 9);
+        else
+            launch_rows(c, opc<false>(A), x, e, done, A.n <= 64 * 640 ? 9 : 3);
     } else if (large_single(c)) {
         launch_rows(c, Op0<float, true>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_tpos.p, B.d_val32.p},
                     x, e, done, 1);
@@ -534,9 +561,8 @@ static void coarse_inverse(const AmgLevel& L, const std::vector<float>& val, std
     for (int a = 0; a < L.n; a++)
         for (int q = L.rowptr[a]; q < L.rowptr[a + 1]; q++) {
             const int b = L.col[q], e = L.slot[q];
-            const size_t v0 = (size_t)(e >> 6) * 2304 + (e & 63);
             for (int r = 0; r < 6; r++)
-                for (int s = 0; s < 6; s++) A[(size_t)(6 * a + r) * n + 6 * b + s] = val[v0 + (6 * r + s) * 64];
+                for (int s = 0; s < 6; s++) A[(size_t)(6 * a + r) * n + 6 * b + s] = val[amg_at(e, 6 * r + s)];
         }
     double dmax = 0.0;
     for (int i = 0; i < n; i++) dmax = std::max(dmax, A[(size_t)i * n + i]);

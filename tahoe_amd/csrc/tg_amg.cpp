@@ -362,7 +362,14 @@ void amg_setup(tg_ctx* c)
             upload(c, nx->d_col, col_slot);
             upload(c, nx->d_sbase, nx->sbase);
             upload(c, nx->d_swidth, nx->swidth);
-            TG_HIP(hipStreamSynchronize(c->stream));  // col_slot outlives its copy
+            std::vector<int> part;
+            if (nagg >= AMG_SYM_NODES) {
+                part.assign((size_t)nx->nslots, 0);
+                for (size_t k = 0; k < up.size(); k += 2)
+                    if (up[k + 1] >= 0) part[(size_t)up[k + 1]] = up[k];
+                upload(c, nx->d_part, part);
+            }
+            TG_HIP(hipStreamSynchronize(c->stream));  // col_slot and part outlive their copies
         }
         upload(c, nx->d_diagblk, diag);
         nx->d_val.alloc((size_t)nx->nslots * 36);

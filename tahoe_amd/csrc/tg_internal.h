@@ -190,17 +190,26 @@ struct Timing {
 // solver's block operator (3 dofs per node); every coarser level has 6 dofs
 // per node (the rigid-body modes of an aggregate) and its matrix is a block
 // CSR of 6x6 FP32 blocks, row-major inside a block.
+//
+// Index of component m of slot e: components in groups of four, a group's 64
+// rows side by side, so that a lane reads a group by one 16-byte load.
+__host__ __device__ inline long amg_at(int e, int m) { return (long)(e >> 6) * 2304 + (m >> 2) * 256 + (e & 63) * 4 + (m & 3); }
+// a level of at least this many nodes reads lower blocks through their
+// partners: below, its values (27 blocks of 144 bytes a node) stay in the
+// 256 MB last-level cache, which serves both halves alike
+constexpr int AMG_SYM_NODES = 1 << 16;
 struct AmgLevel {
     int n = 0, bs = 3;                       // nodes, dofs per node
     std::vector<int> rowptr, col;            // pattern (levels >= 1; sorted, diagonal included)
     // levels >= 1 are stored sliced like the fine operator: slice s holds
     // block rows [64 s, 64 s + 64); entry k of row a is slot
     // (sbase[a / 64] + k) * 64 + a % 64; the 36 values of slot e (row-major
-    // inside the block) are val[(e / 64) * 2304 + comp * 64 + e % 64]
+    // inside the block) are val[amg_at(e, comp)]
     std::vector<int> sbase, swidth, slot;    // slot: CSR entry -> slot
     long nslots = 0;
     DBuf<int> d_sbase, d_swidth, d_col, d_diagblk;  // d_col: column node per slot, -1 padding; d_diagblk: slot
-    DBuf<float> d_val;                       // [nslots][36], component-major per slice
+    DBuf<int> d_part;                        // [nslots] lower slot -> slot of its upper partner (n >= AMG_SYM_NODES)
+    DBuf<float> d_val;                       // [nslots][36], four components of 64 rows at a time (amg_at)
     DBuf<double> d_dinv_own;                 // [n*bs] inverse diagonal (levels >= 1)
     double* dinv = nullptr;                  // level 0: the PCG's Jacobi vector
     DBuf<double> d_f, d_x, d_r, d_d0, d_d1;  // V-cycle vectors [n*bs]
