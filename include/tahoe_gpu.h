@@ -301,8 +301,9 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
  *                      variant gives bitwise the same product.  0 .. 7, or
  *                      -1 (default): 7 for a single problem of 2^17 nodes
  *                      or more, 2 for a batch of 2^17 nodes or more, 3
- *                      from 98,304 nodes, else 0 (there, untuned, several
- *                      waves share a row's blocks). */
+ *                      from 98,304 nodes, else 0; untuned, several waves
+ *                      share a row's blocks up to 98,304 nodes and, in a
+ *                      single problem, from 2^17 (FP64: up to 786,431). */
 /* TG_TUNE_AMG_DEGREE   multigrid: Chebyshev degree of each pre- and
  *                      post-smoothing pass, 2 (default) .. 4.  Until it is
  *                      set, levels of 393,216 and more dofs take one step. */

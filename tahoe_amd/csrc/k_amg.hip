@@ -39,36 +39,34 @@ __device__ __forceinline__ bool skip(const double* done) { return done && *done 
 // Level 0: the solver's sliced-ELL operator (3x3 blocks), one lane per node.
 // add: y += the products of slots k0 .. k1 - 1 of the row of node t (lane l of
 // the slice at b0).  Padding slots (column -1) hold zeros and multiply the
-// row's own entries, so no branch stands between the loads.  SYM: a lower
-// block is read as its upper partner's transpose (k_pcg.hip, block_values).
-template <class MT, bool SYM>
+// row's own entries, so no branch stands between the loads.  NT: non-temporal
+// loads, for an operator that the last-level cache cannot hold (op_streams).
+template <class MT, bool NT>
 struct Op0 {
     static constexpr int NC = 3;
     int n;
     const int* sbase;
     const int* swidth;
     const int* col;
-    const int* tpos;
     const MT* val;
     __device__ __forceinline__ void add(long b0, int k0, int k1, int l, int t, const double* __restrict__ x, double (&y)[3]) const
     {
 #pragma unroll 3
         for (int q = k0; q < k1; q++) {
             const long blk = b0 + q;
-            const int cr = col[blk * 64 + l];
+            const int* pc = col + blk * 64 + l;
+            const int cr = NT ? __builtin_nontemporal_load(pc) : *pc;
             const int c = cr < 0 ? t : cr;
-            const bool tr = SYM && c < t;
-            long at = blk * 576 + l;
-            if (tr) at = tpos[blk * 64 + l];
+            const MT* pv = val + blk * 576 + l;
             double u[9], xc[3];
 #pragma unroll
-            for (int m = 0; m < 9; m++) u[m] = (double)val[at + 64 * m];
+            for (int m = 0; m < 9; m++) u[m] = (double)(NT ? __builtin_nontemporal_load(pv + 64 * m) : pv[64 * m]);
 #pragma unroll
             for (int j = 0; j < 3; j++) xc[j] = x[3L * c + j];
 #pragma unroll
             for (int r = 0; r < 3; r++)
 #pragma unroll
-                for (int j = 0; j < 3; j++) y[r] += (tr ? u[3 * j + r] : u[3 * r + j]) * xc[j];
+                for (int j = 0; j < 3; j++) y[r] += u[3 * r + j] * xc[j];
         }
     }
 };
@@ -180,42 +178,39 @@ struct EPost {  // start of post-smoothing: r = f - A x; d0 = D^-1 r / theta
     }
 };
 
-// A product with a level's operator and what follows it.  NW = 1: a lane per
-// row, four slices a workgroup; NW > 1: a slice a workgroup, its waves share
-// the row's slots and wave 0 adds their sums in order (the coarse levels have
-// few rows: at 128^3, 72, 12 and 2 slices took 30-40 us a product with a lane
-// per row, each walking 27 blocks of 36 values, and take 6-8 shared; 544
-// slices 38 and 27).  Each XCD takes a contiguous range of slices.  The two
-// large levels are bound by what passes the L2s: 2.15 M nodes FP32 (2.3 GB, the
-// lower z layer's blocks twice) 452 us, 270 k nodes of 6 dofs (1.07 GB) 236 us.
+// A product with a level's operator and what follows it: a slice a workgroup,
+// its NW waves share the row's slots and wave 0 adds their sums in order.  A
+// lane per row instead walks its 27 blocks alone: at 128^3 the coarse levels of
+// 72, 12 and 2 slices took 30-40 us a product so and take 6-8 shared, 544 slices
+// 38 and 27.  ranges: each XCD takes a contiguous range of slices.  The large levels are
+// bound by what passes the L2s: 2.15 M nodes FP32, 2.3 GB, 452 us with a lane per
+// row, 432 so when lower blocks came from their partners, 419 with three waves
+// and non-temporal loads; 275 k nodes 76 with the partners, 48 without; 270 k
+// nodes of 6 dofs (1.07 GB) 236 and, as OpC reads them now, 165 us.
 template <class Op, int NW, class E>
-__global__ void __launch_bounds__(NW == 1 ? AB : 64 * NW) k_amg_rows(Op op, const double* __restrict__ x, E e,
-                                                                      const double* done)
+__global__ void __launch_bounds__(64 * NW) k_amg_rows(Op op, const double* __restrict__ x, E e, int ranges,
+                                                         const double* done)
 {
     if (skip(done)) return;
     const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const int s = NW == 1 ? b * (AB / 64) + wv : b;
+    const int s = ranges ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     if (s >= (op.n + 63) >> 6) return;
     const int t = 64 * s + l;
     const bool own = t < op.n;
     const long b0 = op.sbase[s];
-    const int w = op.swidth[s];
-    const int per = NW == 1 ? w : (w + NW - 1) / NW;
+    const int w = op.swidth[s], per = (w + NW - 1) / NW;
     double q[Op::NC];
 #pragma unroll
     for (int i = 0; i < Op::NC; i++) q[i] = 0.0;
-    op.add(b0, NW == 1 ? 0 : wv * per, NW == 1 ? w : min(w, (wv + 1) * per), l, own ? t : 0, x, q);
-    if (NW > 1) {
-        __shared__ double red[NW][Op::NC][64];
+    op.add(b0, wv * per, min(w, (wv + 1) * per), l, own ? t : 0, x, q);
+    __shared__ double red[NW][Op::NC][64];
 #pragma unroll
-        for (int i = 0; i < Op::NC; i++) red[wv][i][l] = q[i];
-        __syncthreads();
-        if (wv > 0) return;
-        for (int j = 1; j < NW; j++)
+    for (int i = 0; i < Op::NC; i++) red[wv][i][l] = q[i];
+    __syncthreads();
+    if (wv > 0) return;
+    for (int j = 1; j < NW; j++)
 #pragma unroll
-            for (int i = 0; i < Op::NC; i++) q[i] += red[j][i][l];
-    }
+        for (int i = 0; i < Op::NC; i++) q[i] += red[j][i][l];
     if (own)
 #pragma unroll
         for (int i = 0; i < Op::NC; i++) e((long)Op::NC * t + i, q[i]);
@@ -473,22 +468,17 @@ static OpC<SYM> opc(const AmgLevel& L)
 template <class Op, class E>
 static void launch_rows(tg_ctx* c, const Op& op, const double* x, const E& e, const double* done, int nw)
 {
-    const int ns = (op.n + 63) / 64;
-    auto go = [&](auto kernel, int blocks, int threads) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(blocks + 7) / 8 * 8), dim3(threads), 0, c->stream, op, x, e, done);
-    };
+    const unsigned nb = (unsigned)((op.n + 63) / 64 + 7) / 8 * 8;
+    const int ranges = op.n < 1 << 19;  // as the PCG's product (k_pcg.hip: k_share_spmv)
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(nb), dim3(64 * nw), 0, c->stream, op, x, e, ranges, done); };
     if (nw == 9)
-        go(k_amg_rows<Op, 9, E>, ns, 64 * 9);
-    else if (nw == 3)
-        go(k_amg_rows<Op, 3, E>, ns, 64 * 3);
+        go(k_amg_rows<Op, 9, E>);
     else
-        go(k_amg_rows<Op, 1, E>, (ns + AB / 64 - 1) / (AB / 64), AB);
+        go(k_amg_rows<Op, 3, E>);
 }
 
-// y = A_l x and what follows.  Waves per row: as the PCG's (k_pcg.hip) at the
-// fine level, whose lower blocks are read through their partners from 2^17
-// nodes; the coarse levels' rows, four times as heavy, are shared by 9 waves
-// up to 640 slices and by 3 up to 2,048.
+// y = A_l x and what follows.  Nine waves share a row up to 640 slices and where
+// lower blocks come from their partners, three otherwise.
 template <class E>
 static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const double* done)
 {
@@ -499,12 +489,12 @@ static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const doub
             launch_rows(c, opc<true>(A), x, e, done, 9);
         else
             launch_rows(c, opc<false>(A), x, e, done, A.n <= 64 * 640 ? 9 : 3);
-    } else if (large_single(c)) {
-        launch_rows(c, Op0<float, true>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_tpos.p, B.d_val32.p},
-                    x, e, done, 1);
     } else {
-        launch_rows(c, Op0<float, false>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_tpos.p, B.d_val32.p},
-                    x, e, done, c->nnd <= 64 * 640 ? 9 : pcg_small(c) ? 3 : 1);
+        auto go = [&](const auto& op) { launch_rows(c, op, x, e, done, c->nnd <= 64 * 640 ? 9 : 3); };
+        if (op_streams(c, sizeof(float)))
+            go(Op0<float, true>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_val32.p});
+        else
+            go(Op0<float, false>{c->nnd, B.d_slice_base.p, B.d_slice_width.p, B.d_col.p, B.d_val32.p});
     }
 }
 

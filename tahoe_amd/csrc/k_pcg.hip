@@ -297,7 +297,7 @@ __device__ __forceinline__ int row_block()
 // partner), so the values are the same, while the partner's row, just
 // streamed by a nearby workgroup, serves them from L2 or the last-level
 // cache instead of HBM.  Only the lanes of lower blocks read tpos.
-template <class MT, bool SYM>
+template <class MT, bool SYM, bool NT = false>
 __device__ __forceinline__ void block_values(const MT* __restrict__ bval, const int* __restrict__ tpos, long blk,
                                              int l, bool lower, double v[9])
 {
@@ -306,7 +306,7 @@ __device__ __forceinline__ void block_values(const MT* __restrict__ bval, const 
     if (tr) base = tpos[blk * 64 + l];
     double u[9];
 #pragma unroll
-    for (int m = 0; m < 9; m++) u[m] = (double)bval[base + m * 64];
+    for (int m = 0; m < 9; m++) u[m] = (double)(NT ? __builtin_nontemporal_load(bval + base + m * 64) : bval[base + m * 64]);
     v[0] = u[0];
     v[4] = u[4];
     v[8] = u[8];
@@ -324,6 +324,7 @@ __device__ __forceinline__ void block_values(const MT* __restrict__ bval, const 
 // take a group each, with the same rounding.  Nine groups of three are the
 // 27 blocks of an interior node of a hexahedral mesh.
 constexpr int RG = 3;
+constexpr int SHARE_WAVES = 3; // waves of a workgroup of k_share_spmv
 
 // y += A_blk x for one slot of a row
 __device__ __forceinline__ void block_mac(const double (&v)[9], double x0, double x1, double x2, double (&y)[3])
@@ -337,7 +338,7 @@ __device__ __forceinline__ void block_mac(const double (&v)[9], double x0, doubl
 // padding slots (column -1) hold zero values: they multiply the row's own x,
 // which keeps the loop branch-free so its loads can be issued ahead; adding
 // the zero products leaves the sums unchanged.
-template <class MT, bool UNR, bool SYM, class X>
+template <class MT, bool UNR, bool SYM, bool NT = false, class X>
 __device__ __forceinline__ void row_sum(const int* __restrict__ bcol, const MT* __restrict__ bval,
                                         const int* __restrict__ tpos, long b0, int w, int l, int a, X x,
                                         double (&y)[3])
@@ -349,12 +350,12 @@ __device__ __forceinline__ void row_sum(const int* __restrict__ bcol, const MT* 
 #pragma unroll(UNR ? RG : 1)
         for (int i = 0; i < RG; i++) {
             const long blk = b0 + k + i;
-            const int cr = bcol[blk * 64 + l];
+            const int cr = NT ? __builtin_nontemporal_load(bcol + blk * 64 + l) : bcol[blk * 64 + l];
             if (!UNR && cr < 0) continue;
             const int c = cr < 0 ? a : cr;
             double x0, x1, x2, v[9];
             x(c, x0, x1, x2);
-            block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
+            block_values<MT, SYM, NT>(bval, tpos, blk, l, c < a, v);
             block_mac(v, x0, x1, x2, g);
         }
 #pragma unroll
@@ -365,12 +366,12 @@ __device__ __forceinline__ void row_sum(const int* __restrict__ bcol, const MT* 
 #pragma unroll 1
         for (; k < w; k++) {
             const long blk = b0 + k;
-            const int cr = bcol[blk * 64 + l];
+            const int cr = NT ? __builtin_nontemporal_load(bcol + blk * 64 + l) : bcol[blk * 64 + l];
             if (!UNR && cr < 0) continue;
             const int c = cr < 0 ? a : cr;
             double x0, x1, x2, v[9];
             x(c, x0, x1, x2);
-            block_values<MT, SYM>(bval, tpos, blk, l, c < a, v);
+            block_values<MT, SYM, NT>(bval, tpos, blk, l, c < a, v);
             block_mac(v, x0, x1, x2, g);
         }
 #pragma unroll
@@ -380,8 +381,11 @@ __device__ __forceinline__ void row_sum(const int* __restrict__ bcol, const MT* 
 
 // q = A p on the block operator, with per-slice partials of p.q.  MT is the
 // storage type of the operator values (double, or float in mixed
-// precision); products and sums are FP64.
-template <class MT, bool XCD, bool UNR, bool SYM>
+// precision); products and sums are FP64.  NT: an operator that the last-level
+// cache cannot hold (op_streams) is read past it by non-temporal loads, which
+// leaves the caches to the vectors: 384 RVEs of edge 4-24 (1.2 GB) 88.4 ms a
+// solve without, 84.6 with.
+template <class MT, bool XCD, bool UNR, bool SYM, bool NT = false>
 __global__ void __launch_bounds__(PB) k_seg_spmv(SegTab T, int nnd,
                                                  const int* __restrict__ sbase, const int* __restrict__ swidth,
                                                  const int* __restrict__ bcol, const MT* __restrict__ bval,
@@ -397,7 +401,7 @@ __global__ void __launch_bounds__(PB) k_seg_spmv(SegTab T, int nnd,
     double dv = 0.0;
     if (a < nnd) {
         double yi[3];
-        row_sum<MT, UNR, SYM>(bcol, bval, tpos, sbase[s], swidth[s], l, a, [&](int c, double& x0, double& x1, double& x2) {
+        row_sum<MT, UNR, SYM, NT>(bcol, bval, tpos, sbase[s], swidth[s], l, a, [&](int c, double& x0, double& x1, double& x2) {
             x0 = x[3L * c];
             x1 = x[3L * c + 1];
             x2 = x[3L * c + 2];
@@ -405,6 +409,88 @@ __global__ void __launch_bounds__(PB) k_seg_spmv(SegTab T, int nnd,
         y[3L * a] = yi[0];
         y[3L * a + 1] = yi[1];
         y[3L * a + 2] = yi[2];
+        dv = yi[0] * x[3L * a] + yi[1] * x[3L * a + 1] + yi[2] * x[3L * a + 2];
+    }
+    dv = wsum(dv);
+    if (l == 0) ppq[s] = dv;
+}
+
+// The same product with a row shared by three waves, a workgroup a slice:
+// from 2^17 nodes, where the operator's bytes bound it.  A wave takes nine
+// consecutive slots, leaves each group's sum in LDS and wave 0 adds the groups
+// in order: bitwise k_seg_spmv.  Three short chains a row keep more loads in
+// flight than one of 27 blocks.  NT: an operator that the last-level cache
+// cannot hold (op_streams) is read past it by non-temporal loads, which leaves
+// the caches to the vectors.  XCD: below 2^19 nodes; beyond, slices in
+// index order.  ms a Newton step, Jacobi, rtol 1e-3, symmetric read (7) /
+// XCD / XCD NT / index order NT: mixed 140 k nodes 69.5 / 54.8 / 59.3 / 64.5,
+// 275 k 127 / 112 / 109 / 110, 531 k 290 / 278 / 258 / 254, 912 k 617 / 608 /
+// 570 / 559, 2.15 M 1344 / 1442 / 1372 / 1339 (FP32: 5.5 TB/s); FP64 140 k 99.9
+// / 89.5 / 87.2 / 93.0, 275 k 188 / 187 / 162 / 168, 531 k 422 / 440 / 404 /
+// 404, 912 k 891 / 961 / 906 / 896.
+template <class MT, bool XCD, bool NT>
+__global__ void __launch_bounds__(64 * SHARE_WAVES) k_share_spmv(SegTab T, int nnd, const int* __restrict__ sbase,
+                                                                 const int* __restrict__ swidth,
+                                                                 const int* __restrict__ bcol,
+                                                                 const MT* __restrict__ bval,
+                                                                 const double* __restrict__ x, double* __restrict__ y,
+                                                                 double* __restrict__ ppq, const double* __restrict__ sc)
+{
+    constexpr int GW = 3, ROUND = SHARE_WAVES * GW * RG;  // groups a wave and slots a workgroup take at a time
+    __shared__ double red[SHARE_WAVES * GW][3][64];
+    const int s = row_block<XCD>(), l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (s >= T.nslices) return;
+    const int g = T.slice_seg[s];
+    if (*sf((double*)sc, S_DONE, T.nseg, g) != 0.0) return;
+    const int a = 64 * s + l;
+    const bool own = a < nnd;
+    const long b0 = sbase[s];
+    const int w = swidth[s];
+    double yi[3] = {0.0, 0.0, 0.0};
+    for (int r0 = 0; r0 < w; r0 += ROUND) {
+#pragma unroll 1
+        for (int j = 0; j < GW; j++) {
+            const int k0 = r0 + RG * (GW * wv + j);
+            if (k0 >= w) break;
+            // past the row's last slot that slot again (not used): no branch
+            // stands around a load
+            double xc[RG][3];
+            MT v[RG][9];
+#pragma unroll
+            for (int i = 0; i < RG; i++) {
+                const long blk = b0 + min(k0 + i, w - 1);
+                const int* pc = bcol + blk * 64 + l;
+                const int cr = NT ? __builtin_nontemporal_load(pc) : *pc;
+                const int c = cr >= 0 ? cr : own ? a : 0;
+                const MT* pv = bval + blk * 576 + l;
+#pragma unroll
+                for (int m = 0; m < 9; m++) v[i][m] = NT ? __builtin_nontemporal_load(pv + 64 * m) : pv[64 * m];
+#pragma unroll
+                for (int m = 0; m < 3; m++) xc[i][m] = x[3L * c + m];
+            }
+            double gs[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int i = 0; i < RG; i++) {
+                double vd[9];
+#pragma unroll
+                for (int m = 0; m < 9; m++) vd[m] = (double)v[i][m];
+                if (k0 + i < w) block_mac(vd, xc[i][0], xc[i][1], xc[i][2], gs);
+            }
+#pragma unroll
+            for (int i = 0; i < 3; i++) red[GW * wv + j][i][l] = gs[i];
+        }
+        __syncthreads();
+        if (wv == 0)
+            for (int j = 0; j < SHARE_WAVES * GW && r0 + RG * j < w; j++)
+#pragma unroll
+                for (int i = 0; i < 3; i++) yi[i] += red[j][i][l];
+        if (r0 + ROUND < w) __syncthreads();
+    }
+    if (wv > 0) return;
+    double dv = 0.0;
+    if (own) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) y[3L * a + i] = yi[i];
         dv = yi[0] * x[3L * a] + yi[1] * x[3L * a + 1] + yi[2] * x[3L * a + 2];
     }
     dv = wsum(dv);
@@ -1005,6 +1091,13 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
     double* ppq = fold ? W.ppq : W.part;
     // rows split over the waves of a workgroup
     const int split = fold && fused ? pcg_split(c) : 0;
+    // the unfused iteration's product: 1..4 by three waves a row (+ 1 streaming,
+    // + 2 contiguous ranges of slices for the XCDs), 5 the batch's variant
+    // streaming, 0 the variant as it is
+    const bool streams = op_streams(c, sizeof(MT));
+    const int share = fused || c->spmv_xcd >= 0 ? 0
+                      : pcg_share(c, sizeof(MT)) ? 1 + (streams ? 1 : 0) + (c->nnd < 1 << 19 ? 2 : 0)
+                                                 : (variant == 2 && streams ? 5 : 0);
     auto update = [&](const double* pk, int o) {
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(ng), dim3(PB), 0, c->stream, T, c->nnd, pk, q, dinv, x, r, z, ppq, W.part, o,
@@ -1087,13 +1180,30 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
         for (int k = 0; k < CHUNK; k++) {
             {
                 TimedRegion tr(c, T_SPMV);
-                spmv_dispatch(variant, [&](auto V) {
-                    constexpr int v = decltype(V)::value;
-                    hipLaunchKernelGGL((k_seg_spmv<MT, (v & 1) != 0, (v & 2) != 0, (v & 4) != 0>),
-                                       dim3((v & 1) ? (nb + 7) / 8 * 8 : nb), dim3(PB), 0, c->stream, T, c->nnd,
-                                       c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val,
-                                       c->op.d_tpos.p, p, q, ppq, W.scal);
-                });
+                auto go_share = [&](auto kernel) {
+                    hipLaunchKernelGGL(kernel, dim3((unsigned)(ns + 7) / 8 * 8), dim3(64 * SHARE_WAVES), 0, c->stream, T,
+                                       c->nnd, c->op.d_slice_base.p, c->op.d_slice_width.p, c->op.d_col.p, val, p, q, ppq,
+                                       W.scal);
+                };
+                if (share == 4)
+                    go_share(k_share_spmv<MT, true, true>);
+                else if (share == 3)
+                    go_share(k_share_spmv<MT, true, false>);
+                else if (share == 2)
+                    go_share(k_share_spmv<MT, false, true>);
+                else if (share == 1)
+                    go_share(k_share_spmv<MT, false, false>);
+                auto go = [&](auto kernel, unsigned blocks) {
+                    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(PB), 0, c->stream, T, c->nnd, c->op.d_slice_base.p,
+                                       c->op.d_slice_width.p, c->op.d_col.p, val, c->op.d_tpos.p, p, q, ppq, W.scal);
+                };
+                if (share == 5)
+                    go(k_seg_spmv<MT, false, true, false, true>, nb);
+                else if (share == 0)
+                    spmv_dispatch(variant, [&](auto V) {
+                        constexpr int v = decltype(V)::value;
+                        go(k_seg_spmv<MT, (v & 1) != 0, (v & 2) != 0, (v & 4) != 0>, (v & 1) ? (nb + 7) / 8 * 8 : nb);
+                    });
             }
             {
                 TimedRegion tr(c, T_VECTOR);
@@ -1126,7 +1236,7 @@ static void pcg_loop(tg_ctx* c, const MT* val, const double* dinv, const double*
         // every address and size the chunk's launches take (tg_initialize
         // also drops the graph, as buffers may come back at old addresses)
         const void* key[24] = {val, dinv, x, r, p, q, W.part, W.scal, W.ndone,
-                               (const void*)(long)(PC + 4L * (variant + 8L * ((int)fused + 2L * (split + 16L * c->amg.gen)))),
+                               (const void*)(long)(PC + 4L * (variant + 8L * ((int)fused + 2L * (split + 16L * (share + 8L * c->amg.gen))))),
                                (const void*)(long)sizeof(MT), (const void*)(long)c->nnd, (const void*)(long)nseg,
                                (const void*)ns, S.d_grp.p, S.d_slice_seg.p, c->op.d_slice_base.p,
                                c->op.d_slice_width.p, c->op.d_col.p, pbuf[1], z,

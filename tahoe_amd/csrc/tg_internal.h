@@ -432,15 +432,29 @@ inline int stiffness_shape(const tg_ctx* c) { return c->stiff_variant >= 0 ? c->
 //  - above, the operator's bytes bound it and the fused direction's second
 //    gathered vector costs more than the direction pass: 124 k nodes, mixed:
 //    38.6 fused and split, 35.4 with the unrolled row loop (variant 3);
-//  - a single problem of 2^17 nodes or more reads lower blocks through their
-//    partners (7), a batch of that size the full operator in index order (2;
-//    its rows are mostly boundary rows, where the symmetric read diverges).
+//  - from 2^17 nodes of a single problem three waves share a row (k_pcg.hip:
+//    k_share_spmv, whose comment has the times); reading lower blocks through
+//    their partners (7) takes two scattered cache lines for one and only pays
+//    where HBM is far behind: FP64 from 3 * 2^18 nodes.  A batch of that size
+//    takes the full operator a lane per row in index order (2): contiguous
+//    ranges would leave XCDs idle when their segments have finished.
 inline bool large_single(const tg_ctx* c) { return c->seg.nseg <= 1 && c->nnd >= (1 << 17); }
 inline bool large_total(const tg_ctx* c) { return c->nnd >= (1 << 17); }
 inline bool pcg_small(const tg_ctx* c) { return c->nnd <= 64 * 1536; }
 inline int spmv_variant(const tg_ctx* c)
 {
     return c->spmv_xcd >= 0 ? c->spmv_xcd : (large_single(c) ? 7 : large_total(c) ? 2 : pcg_small(c) ? 0 : 3);
+}
+inline bool pcg_share(const tg_ctx* c, size_t value_bytes)
+{
+    return c->spmv_xcd < 0 && large_single(c) && !(value_bytes == 8 && c->nnd >= 3 << 18);
+}
+// The operator's values and columns are more than the 256 MB last-level cache
+// holds: non-temporal loads (k_share_spmv: 287 and 297 MB gain 3 %, 151 MB
+// loses 8 %; a batch of 12 Q1P0 RVEs, 160 MB, 112 ms without and 125 with).
+inline bool op_streams(const tg_ctx* c, size_t value_bytes)
+{
+    return (double)c->op.nblocks_padded * (9.0 * value_bytes + 4.0) > 268e6;
 }
 inline bool pcg_fused(const tg_ctx* c) { return c->pcg_fused >= 0 ? c->pcg_fused != 0 : pcg_small(c); }
 // waves that share a slice's rows in the fused SpMV (untuned SpMV variant

@@ -101,3 +101,37 @@ def test_split_rows_batch_bitwise(precision):
         assert st == res[0][1]
         assert all(np.array_equal(a, b) for a, b in zip(us, res[0][0]))
     assert all(x[0] == 0 for x in res[0][1])
+
+
+# the first size whose rows three waves share again (2^17 nodes: FP32 by plain
+# loads, FP64 by non-temporal ones) and the node row before it, the first size
+# that takes the slices in index order (2^19), and rows of 75 blocks, more than
+# a round of the three waves
+@pytest.mark.parametrize("n", [(63, 31, 63), (63, 31, 62), (127, 63, 63), None])
+@pytest.mark.parametrize("precision,pc", [(0, 0), (1, 1)])
+def test_shared_rows_bitwise(n, precision, pc):
+    from tahoe_amd import mesh as M
+    m = fan(nz=5300) if n is None else M.cube(0, seed=23, nxyz=n)
+    s = solid(m, M.kbc_uniaxial(m, 0.001), precision)
+    try:
+        corrections(s, pc, 21)
+    finally:
+        s.close()
+
+
+def test_streamed_batch_bitwise():
+    """A batch whose operator exceeds the last-level cache (40 cubes of 18^3:
+    296 MB in FP32) by non-temporal loads, and by plain ones."""
+    from tahoe_amd import api, batch, rve
+    pk = batch.pack([rve.Request(i, 18, api.TOTAL_LAGRANGIAN, 0.3, 90 + i).problem() for i in range(40)])
+    res = []
+    for variant in (-1, 2):
+        s = batch.make_solid(pk, precision=api.MIXED)
+        try:
+            s.set_tuning(api.TUNE_SPMV_XCD, variant)
+            us, st = batch.solve_one_step_partial(s, pk, api.Solid.opts(lin_rtol=1e-3))
+            res.append((us, [(x.status, x.iterations, x.lin_iterations) for x in st]))
+        finally:
+            s.close()
+    assert res[0][1] == res[1][1] and all(x[0] == 0 for x in res[0][1])
+    assert all(np.array_equal(a, b) for a, b in zip(res[0][0], res[1][0]))
