@@ -336,7 +336,8 @@ def bench_cube(a):
                  "chunk": s.tuning(api.TUNE_STIFF_CHUNK), "ms": {}}
     else:
         tuned = autotune.tune_stiffness(s, reps=1, run_correction=short_pcg)
-    log(f"Newton assembly {tuned['assembly']} stiffness shape {tuned['shape']} chunk {tuned['chunk']} "
+    log(f"Newton assembly {'by rows, else ' if tuned.get('rows') else ''}{tuned['assembly']} stiffness shape "
+        f"{tuned['shape']} chunk {tuned['chunk']} "
         f"(autotune ms: {tuned['ms']})")
     explicit = a.spmv_xcd is not None or a.pcg_fused is not None
     tuned_spmv = (autotune.tune_spmv_xcd(s, short_pcg) if a.profile or (a.autotune and not explicit)
@@ -435,8 +436,10 @@ def bench_cube(a):
                                "the first Newton correction's state; one full Newton correction ("
                                f"{PC_NAME[a.precond]}-PCG to {a.lin_rtol:g}) timed once beside it",
                    "elements": m.nel, "nodes": m.nnd, "equations": n_eq, "msr_upper_nnz": msr_len - 1,
-                   "newton_assembly": "operator" if tuned["assembly"] == 1 else "msr+expansion",
-                   "stiffness_shape_elements_per_workgroup": api.STIFF_SHAPE_EPB[tuned["shape"]],
+                   "newton_assembly": ("rows" if tuned.get("rows") else
+                                       "operator" if tuned["assembly"] == 1 else "msr+expansion"),
+                   "stiffness_shape_elements_per_workgroup": (None if tuned.get("rows") else
+                                                              api.STIFF_SHAPE_EPB[tuned["shape"]]),
                    "stiffness_chunk": tuned["chunk"], "spmv_variant": tuned_spmv["xcd"], "pcg_fused": bool(fused),
                    "precision": a.precision, "preconditioner": a.precond},
         "value_is": "elements / (residual pass + stiffness pass device time), HIP events on the solver stream",
@@ -458,7 +461,9 @@ def bench_cube(a):
                           "unit": "TFLOP/s", "frac": stf_gflops * 1e9 / stf_peak, "avg_pass_ms": k_ms,
                           "flop_per_element": STIFF_FLOP_PER_EL,
                           "hbm_GBps_min_bytes": stf_bytes / (k_ms * 1e-3) / 1e9,
-                          "kernel": ("k_stiffness_mfma (16x16x4 MFMA tiles)" if api.STIFF_SHAPE_MFMA[tuned["shape"]]
+                          "kernel": ("k_blocks_simo + k_gather_rows (3x3 blocks, VALU, then a gather by rows; MSR "
+                                     "and operator written)" if tuned.get("rows") else
+                                     "k_stiffness_mfma (16x16x4 MFMA tiles)" if api.STIFF_SHAPE_MFMA[tuned["shape"]]
                                      else "k_stiffness_tl / k_stiffness_db (VALU 3x3 node blocks)"),
                           "note": "dense 24x24 B^T C B count per element; peak: " +
                                   ("FP64 (vector and matrix peaks are equal on MI355X)" if a.precision == "fp64"

@@ -20,6 +20,8 @@ Knobs:
   matrix rows it touches stay in the memory-side cache across the colour
   passes cuts HBM traffic of the scatter; too small a range under-fills the
   GPU.
+  TUNE_STIFF_ROWS -- the assembly by rows that an untuned context uses, timed
+  against the best of the colour-ordered forms above.
 """
 from __future__ import annotations
 
@@ -53,10 +55,13 @@ def _time_stiffness(solid: api.Solid, reps: int, run_correction=None) -> float:
 
 def tune_stiffness(solid: api.Solid, shapes=None, chunks=None, reps: int = 2, run_correction=None) -> dict:
     """Best (Newton assembly path, shape) at the default chunk, then the best
-    chunk.  With run_correction the Newton tangent is timed on both paths --
+    chunk, then the assembly by rows against that.  With run_correction the
+    Newton tangent is timed on both paths --
     straight into the block operator, or into the MSR and expanded -- and
     the faster is kept (TUNE_NEWTON_ASSEMBLY); without it the MSR assembly of
-    tg_form_lhs is tuned.  Returns {"assembly", "shape", "chunk", "ms"}."""
+    tg_form_lhs is tuned.  Returns {"assembly", "shape", "chunk", "rows",
+    "ms"}; with rows true the first three are the best colour-ordered form,
+    not in use."""
     if shapes is None:
         shapes = list(range(len(api.STIFF_SHAPE_EPB)))
     if chunks is None:
@@ -79,10 +84,19 @@ def tune_stiffness(solid: api.Solid, shapes=None, chunks=None, reps: int = 2, ru
             t_chunk[v] = _time_stiffness(solid, reps, run_correction)
         best_chunk = min(t_chunk, key=t_chunk.get) if t_chunk else -1
         solid.set_tuning(api.TUNE_STIFF_CHUNK, best_chunk)
+        # by rows (a mesh it does not take stays colour-ordered)
+        t_colour = min([t_shape[(best_mode, best_shape)], *t_chunk.values()])
+        solid.set_tuning(api.TUNE_STIFF_ROWS, 1)
+        rows = solid.tuning(api.TUNE_STIFF_ROWS) == 1
+        t_rows = _time_stiffness(solid, reps, run_correction) if rows else None
+        if rows and t_rows >= t_colour:
+            solid.set_tuning(api.TUNE_STIFF_ROWS, 0)
+            rows = False
     finally:
         solid.timing_enable(False)
-    return {"assembly": best_mode, "shape": best_shape, "chunk": best_chunk,
-            "ms": {"assembly_shape": {f"{m}/{v}": t for (m, v), t in t_shape.items()}, "chunk": t_chunk}}
+    return {"assembly": best_mode, "shape": best_shape, "chunk": best_chunk, "rows": rows,
+            "ms": {"assembly_shape": {f"{m}/{v}": t for (m, v), t in t_shape.items()}, "chunk": t_chunk,
+                   "rows": {} if t_rows is None else {1: t_rows}}}
 
 
 def tune_spmv_xcd(solid: api.Solid, run_pcg, fused=(1, 0), reps: int = 2, variants=range(8)) -> dict:

@@ -139,3 +139,32 @@ def test_colour_knobs_select_the_colours_and_rows_take_it_back():
             assert s.tuning(api.TUNE_STIFF_ROWS) == 0
     finally:
         s.close()
+
+
+def test_tuner_times_the_assembly_by_rows():
+    """tune_stiffness leaves the assembly that it reports in place, and the
+    residual and the tangent are those of an untuned context."""
+    from tahoe_amd import api, autotune, mesh as M
+    m = M.cube(6, seed=4)
+    kbc = M.kbc_uniaxial(m, 0.01)
+    out = []
+    for tune in (False, True):
+        s = api.Solid(0)
+        try:
+            s.set_mesh(m.X, m.conn, m.mat)
+            s.set_material(0, *api.mu_kappa(1000.0, 0.3))
+            s.set_kbc(kbc.nodes, kbc.dofs, kbc.values)
+            s.initialize()
+            s.apply_kbc(1.0)
+            if tune:
+                t = autotune.tune_stiffness(s, shapes=[0], chunks=[0], reps=1)
+                assert s.tuning(api.TUNE_STIFF_ROWS) == int(t["rows"])
+                assert set(t["ms"]["rows"]) == {1}
+            R, _ = s.form_rhs()
+            s.form_lhs()
+            out.append((R, s.msr_values()))
+        finally:
+            s.close()
+    # the two assemblies sum an entry's contributions in another order
+    for a, b in zip(out[0], out[1]):
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max()
