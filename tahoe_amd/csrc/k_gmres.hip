@@ -27,31 +27,48 @@ constexpr int GNB = 512;  // blocks of the partial-sum kernels
 
 inline unsigned nblocks(long n) { return (unsigned)((n + GB - 1) / GB); }
 
-// y = A x on the block operator (storage MT, FP64 sums)
-template <class MT>
-__global__ void __launch_bounds__(GB) k_gm_spmv(int nnd, const int* __restrict__ sbase, const int* __restrict__ swidth,
-                                                const int* __restrict__ col, const MT* __restrict__ val,
-                                                const double* __restrict__ x, double* __restrict__ y)
+// y = A x on the block operator (storage MT, FP64 sums), or y = M A x with m,
+// the point Jacobi preconditioner 1/diag.  A slice a workgroup, its NW waves
+// share the row's slots and wave 0 adds their sums in order: nine waves to 640
+// slices, three beyond (as the PCG's products, k_pcg.hip).  With a lane per row,
+// a chain of 27 blocks, problems of 64 to 576 elements took 13.9 us here and 3.0
+// more for 1/diag, and take 5.1 (their steps are bound by the launches); a
+// correction of 30^3 elements 2.66 -> 2.43 ms, 50^3 mixed 5.42 -> 5.10 ms.
+template <class MT, int NW>
+__global__ void __launch_bounds__(64 * NW) k_gm_spmv(int nnd, const int* __restrict__ sbase,
+                                                     const int* __restrict__ swidth, const int* __restrict__ col,
+                                                     const MT* __restrict__ val, const double* __restrict__ m,
+                                                     const double* __restrict__ x, double* __restrict__ y)
 {
-    const int a = blockIdx.x * GB + threadIdx.x;
-    if (a >= nnd) return;
-    const int s = a >> 6, l = a & 63;
+    __shared__ double red[NW][3][64];
+    const int s = blockIdx.x, l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int a = 64 * s + l;
+    const bool own = a < nnd;
     const long b0 = sbase[s];
-    const int w = swidth[s];
-    double y0 = 0.0, y1 = 0.0, y2 = 0.0;
-    for (int q = 0; q < w; q++) {
+    const int w = swidth[s], per = (w + NW - 1) / NW;
+    const int q1 = min(w, (wv + 1) * per);
+    double yi[3] = {0.0, 0.0, 0.0};
+    // padding slots hold zeros and multiply the row's own entries
+#pragma unroll 3
+    for (int q = wv * per; q < q1; q++) {
         const long blk = b0 + q;
-        const int c = col[blk * 64 + l];
-        if (c < 0) continue;
+        const int cr = col[blk * 64 + l];
+        const int c = cr >= 0 ? cr : own ? a : 0;
         const double x0 = x[3L * c], x1 = x[3L * c + 1], x2 = x[3L * c + 2];
         const MT* v = val + blk * 576 + l;
-        y0 += (double)v[0] * x0 + (double)v[64] * x1 + (double)v[128] * x2;
-        y1 += (double)v[192] * x0 + (double)v[256] * x1 + (double)v[320] * x2;
-        y2 += (double)v[384] * x0 + (double)v[448] * x1 + (double)v[512] * x2;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            yi[i] += (double)v[192 * i] * x0 + (double)v[192 * i + 64] * x1 + (double)v[192 * i + 128] * x2;
     }
-    y[3L * a] = y0;
-    y[3L * a + 1] = y1;
-    y[3L * a + 2] = y2;
+#pragma unroll
+    for (int i = 0; i < 3; i++) red[wv][i][l] = yi[i];
+    __syncthreads();
+    if (wv > 0 || !own) return;
+    for (int j = 1; j < NW; j++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) yi[i] += red[j][i][l];
+#pragma unroll
+    for (int i = 0; i < 3; i++) y[3L * a + i] = m ? m[3L * a + i] * yi[i] : yi[i];
 }
 
 // z = M^-1 y for the point and block Jacobi preconditioners
@@ -163,10 +180,17 @@ static void gmres_t(tg_ctx* c, const MT* val, const double* b, double* x, double
     if (maxit <= 0) maxit = 3 * c->n_eq;
     const unsigned vb = nblocks(n3), nb = (unsigned)((nnd + GB - 1) / GB);
     const unsigned pb = (unsigned)std::min<long>(GNB, std::max<long>(1, (n3 + GB - 1) / GB));
-    auto spmv = [&](const double* in, double* out) {
+    auto spmv = [&](const double* in, const double* dinv, double* out) {
         TimedRegion tr(c, T_SPMV);
-        hipLaunchKernelGGL(k_gm_spmv<MT>, dim3(nb), dim3(GB), 0, c->stream, nnd, c->op.d_slice_base.p,
-                           c->op.d_slice_width.p, c->op.d_col.p, val, in, out);
+        const unsigned ns = (unsigned)((nnd + 63) / 64);
+        auto go = [&](auto kernel, int nw) {
+            hipLaunchKernelGGL(kernel, dim3(ns), dim3(64 * nw), 0, c->stream, nnd, c->op.d_slice_base.p,
+                               c->op.d_slice_width.p, c->op.d_col.p, val, dinv, in, out);
+        };
+        if (nnd <= 64 * 640)
+            go(k_gm_spmv<MT, 9>, 9);
+        else
+            go(k_gm_spmv<MT, 3>, 3);
     };
     auto precondition = [&](const double* in, double* out) {
         TimedRegion tr(c, c->precond == TG_PC_AMG ? T_PRECOND : T_VECTOR);
@@ -205,7 +229,7 @@ static void gmres_t(tg_ctx* c, const MT* val, const double* b, double* x, double
     double beta0 = -1.0, last = 0.0;
     while (!done && total < maxit) {
         // r = M^-1 (b - A x)
-        spmv(x, G.q.p);
+        spmv(x, nullptr, G.q.p);
         {
             TimedRegion tr(c, T_VECTOR);
             hipLaunchKernelGGL(k_gm_bminus, dim3(vb), dim3(GB), 0, c->stream, n3, b, G.q.p);
@@ -232,8 +256,9 @@ static void gmres_t(tg_ctx* c, const MT* val, const double* b, double* x, double
         for (int j = 0; j < m && total < maxit; j++, total++) {
             j_end = j;
             steps++;
-            spmv(G.V.p + (long)j * n3, G.q.p);
-            precondition(G.q.p, G.w.p);
+            const bool point = c->precond != TG_PC_AMG && c->precond != TG_PC_BLOCK_JACOBI;
+            spmv(G.V.p + (long)j * n3, point ? c->vdinv.p : nullptr, point ? G.w.p : G.q.p);
+            if (!point) precondition(G.q.p, G.w.p);
             // two classical Gram-Schmidt passes
             orthogonalise(j + 1, 0);
             orthogonalise(j + 1, m + 1);
