@@ -293,8 +293,13 @@ __global__ void __launch_bounds__(256) k_gather_rows(int nnd, int n_eq, int up_m
                         }
                 }
             }
-            // rows of nodes that no element uses
-            if (up.y == 0 && t < 3) dinv[3L * a + t] = 0.0;
+            // rows of nodes that no element uses: an empty diagonal (nothing
+            // clears the MSR values before this pass)
+            if (up.y == 0 && t < 3) {
+                const int e = eqn[3L * a + t];
+                if (e >= 0) val[e] = MT(0);
+                dinv[3L * a + t] = 0.0;
+            }
         }
     }
     __syncthreads();
