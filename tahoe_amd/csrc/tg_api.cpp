@@ -835,11 +835,12 @@ static void prepare_operator(tg_ctx* c)
     prepare_preconditioner(c);
 }
 
-// Newton's tangent in the inner solve's operator: straight into the block
-// operator (total-Lagrangian), or assembled into the MSR and expanded.
+// Newton's tangent in the inner solve's operator: by rows (MSR and operator
+// at once), or colour-ordered, straight into the block operator
+// (total-Lagrangian) or assembled into the MSR and expanded.
 static void newton_operator(tg_ctx* c)
 {
-    if (c->formulation == TG_TOTAL_LAGRANGIAN && c->newton_assembly == 1) {
+    if (c->formulation == TG_TOTAL_LAGRANGIAN && c->newton_assembly == 1 && !rows_assembly(c)) {
         launch_stiffness_operator(c, c->du.p);
         launch_operator_dinv(c);
         prepare_preconditioner(c);
