@@ -189,6 +189,15 @@ __global__ void __launch_bounds__(1024) k_fin_residual(const double* __restrict_
 constexpr int GR = 32;  // rows of a workgroup (half a slice), 8 lanes each
 constexpr int GQ = 2;   // elements whose loads are in flight
 
+// What a wave's lanes have written to LDS is there for its other lanes, and
+// nothing they read later is read before: an ordering for the compiler (one
+// wave's LDS operations stay in order), no instruction of its own.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Rows of half a slice: 8 lanes per row add the row's blocks of its elements,
 // in list order, into LDS, a block a lane (a row's lanes are in one wave, so
 // its sums need no barrier), and write the row's MSR values and 1/diag; then
@@ -227,6 +236,7 @@ __global__ void __launch_bounds__(256) k_gather_rows(int nnd, int n_eq, int up_m
             BT* my = acc + row * stride;
             const int2 up = upper[a];
             for (int x = t; x < 9 * up.y; x += 8) my[x] = BT(0);
+            wave_lds_fence();
             // lane t takes block t of a run
             const int p1 = ptr[a + 1];
             for (int p = ptr[a]; p < p1; p += GQ) {
@@ -248,9 +258,7 @@ __global__ void __launch_bounds__(256) k_gather_rows(int nnd, int n_eq, int up_m
                     if (slot[q] >= 0)
 #pragma unroll
                         for (int c = 0; c < 9; c++) my[9 * slot[q] + c] += v[q][c];
-                    // (lanes of a row read sums other lanes wrote: the wave's
-                    // LDS operations stay in this order)
-                    __builtin_amdgcn_wave_barrier();
+                    wave_lds_fence();  // lanes of a row read sums that other lanes wrote
                 }
             }
             // MSR values: row r[i] lists the node's own later dofs, then the
