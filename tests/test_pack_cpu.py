@@ -58,3 +58,8 @@ def test_arrays_of_another_size_are_refused():
     q.mesh = M.HexMesh(q.mesh.X, q.mesh.conn, q.mesh.mat[:1], q.mesh.nodesets, q.mesh.shape)
     with pytest.raises(ValueError):
         batch.pack([p, q])
+
+
+def test_no_problems_are_refused():
+    with pytest.raises(ValueError):
+        batch.pack([])
