@@ -47,7 +47,7 @@ def pack(problems: list) -> Packed:
     table.  Each array is written once, straight from the problems' own
     arrays: at a million nodes the pages of fresh arrays cost more than the
     copies, so there are no temporaries."""
-    if not problems:
+    if len(problems) == 0:
         raise ValueError("no problems to pack")
     mats, index, gids, gbeg = [], {}, [], [0]
     for p in problems:
