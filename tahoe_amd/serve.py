@@ -124,9 +124,9 @@ class RVEServer:
         # while another worker solves, a mini-batch that is not full waits up
         # to `linger` seconds for requests of its kind: a request joined costs
         # the batch little, on its own it costs a whole set-up and launch
-        # chain.  An idle server starts at once.
+        # chain.  With no worker solving it starts at once.
         self.linger = linger
-        self._solving = 0
+        self._solving = 0            # workers that solve (one that waits for requests is not among them)
         # each worker keeps one context per (formulation, size class,
         # preconditioner) alive between batches and sets it up again for the
         # next batch (batch.configure): no allocation once the kind's largest
@@ -168,14 +168,14 @@ class RVEServer:
             return None
         bid = self._next_batch
         self._next_batch += 1
-        self._solving += 1
         end = time.perf_counter() + self.linger
-        while len(picked) < self.max_batch and self._solving > 1 and not self._closed:
+        while len(picked) < self.max_batch and self._solving > 0 and not self._closed:
             left = end - time.perf_counter()
             if left <= 0:
                 break
             self._lock.wait(timeout=left)
             size += self._extend_batch(picked[0], picked)
+        self._solving += 1
         return bid, picked, size
 
     def _extend_batch(self, head, picked):
