@@ -32,19 +32,27 @@ from . import api, batch
 
 def footprint_bytes(req, precision=api.MIXED) -> int:
     """Device bytes of one request inside a batch context (upper bound for
-    a cube of L^3 hexes): per element the 300-entry MSR slot map, the 72-entry
-    operator slot map (either these two or the row assembly's slots, block and
-    force buffers, which are smaller together), connectivity, material and
-    element lists; per node the
-    upper MSR pattern and values (<= 123 entries), 27 operator blocks (column,
-    9 FP64 values, 9 FP32 values in mixed precision, 9-entry expansion map)
-    and about a dozen node-space vectors."""
+    a cube of L^3 hexes).  Per element: connectivity, material, node ranks
+    and the list of its nodes' elements; the row assembly's slots (64), force
+    buffer (24 FP64 values) and block buffer (324 values, FP32 for the
+    total-Lagrangian stiffness in mixed precision).  Per node: the upper MSR
+    pattern and values (<= 123 entries, FP64 and in that case FP32 too), 27
+    operator blocks (column, partner, row entry, 9 FP64 values, 9 FP32 values
+    in mixed precision), the node graph (27 neighbours, row lengths and
+    pointers), a dozen node-space vectors, the inverse diagonal block, the
+    equation numbers, three kinematic cards and the reductions' partials.
+    (The expansion's and the colour-ordered assembly's maps are built only for
+    that assembly, which a served context does not use.)"""
     nel = req.L ** 3
     nnd = (req.L + 1) ** 3 + 63          # padding to a 64-node boundary
-    per_el = 4 * (300 + 72 + 8 + 1 + 2)
-    val_b = 8 + (4 if precision == api.MIXED else 0)
-    per_node = 123 * (4 + val_b) + 27 * (4 + 9 * val_b + 9 * 4) + 12 * 3 * 8
-    return nel * per_el + nnd * per_node
+    mixed = precision == api.MIXED
+    fp32_stiffness = mixed and req.formulation == api.TOTAL_LAGRANGIAN
+    per_el = 4 * (8 + 1 + 1 + 8) + 64 + 24 * 8 + 324 * (4 if fp32_stiffness else 8)
+    msr = 123 * (4 + 8 + (4 if fp32_stiffness else 0))
+    operator = 27 * (4 + 4 + 2 + 9 * (8 + (4 if mixed else 0)))
+    graph = 27 * 4 + 2 * 4 + 2 * 8 + 2 * 3 * 8 + 8 + 4 + 1
+    nodal = 12 * 3 * 8 + 9 * 8 + 3 * 4 + 3 * (4 + 8) + 8
+    return nel * per_el + nnd * (msr + operator + graph + nodal)
 
 
 @dataclass
