@@ -305,8 +305,9 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
  *                      share a row's blocks up to 98,304 nodes and, in a
  *                      single problem, from 2^17 (FP64: up to 786,431). */
 /* TG_TUNE_AMG_DEGREE   multigrid: Chebyshev degree of each pre- and
- *                      post-smoothing pass, 2 (default) .. 4.  Until it is
- *                      set, levels of 393,216 and more dofs take one step. */
+ *                      post-smoothing pass, 2 .. 4, or -1 (default): 2, and
+ *                      one step on levels of 393,216 and more dofs.  Reads
+ *                      the fine level's degree, 1 for one step. */
 /* TG_TUNE_AMG_WEIGHT   multigrid: weight of the coarse-grid correction in
  *                      percent, 100 .. 190 (default 150: unsmoothed
  *                      aggregation under-corrects; any weight in (0, 2)

@@ -25,7 +25,7 @@ constexpr int AB = 256;          // threads per block of the vector/level kernel
 // to 1e-10): ratio 30 94 / 82 / 141, 16 87 / 78 / 132, 12 87 / 78 / 131, 8 91 /
 // 80 / 133, 4 101 / 87 / 148.
 constexpr double CHEB_RATIO = 14.0;
-// With one step (amg_level_degree) the interval is [lmax / 4, lmax], a damped
+// With one step (level_degree) the interval is [lmax / 4, lmax], a damped
 // Jacobi step with 1.6 / lmax: 128^3 mixed, fine and first coarse level so,
 // PCG iterations of a Newton step: ratio 4 109, 10 114; 96^3: 3 112, 4 112.
 constexpr double JACOBI_RATIO = 4.0;
@@ -509,7 +509,7 @@ static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const doub
 static int level_degree(const tg_ctx* c, int l)
 {
     const AmgLevel& A = *c->amg.lv[l];
-    return c->amg.degree_auto && (long)A.n * A.bs >= 3L << 17 ? 1 : c->amg.degree;
+    return amg_degree(c, (long)A.n * A.bs);
 }
 
 static double* level_dinv(tg_ctx* c, int l) { return l == 0 ? c->vdinv.p : c->amg.lv[l]->dinv; }

@@ -1221,9 +1221,10 @@ int tg_set_tuning(tg_ctx* c, int knob, long value)
             c->stiff_gather = (int)value;
             c->stiff_explicit = true;
         } else if (knob == TG_TUNE_AMG_DEGREE) {
-            if (value < 2 || value > 4) fail(TG_OUT_OF_RANGE, "multigrid smoother degree must be 2..4");
-            c->amg.degree = (int)value;
-            c->amg.degree_auto = false;
+            if (value != -1 && (value < 2 || value > 4))
+                fail(TG_OUT_OF_RANGE, "multigrid smoother degree must be 2..4, or -1 for the default");
+            c->amg.degree = value == -1 ? 2 : (int)value;
+            c->amg.degree_auto = value == -1;
             c->amg.gen++;
             c->amg.since = -1;
         } else if (knob == TG_TUNE_AMG_WEIGHT) {
@@ -1264,7 +1265,7 @@ int tg_get_tuning(tg_ctx* c, int knob, long* value)
         else if (knob == TG_TUNE_AMG_REUSE)
             *value = c->amg.reuse;
         else if (knob == TG_TUNE_AMG_DEGREE)
-            *value = c->amg.degree;
+            *value = amg_degree(c, 3L * c->nnd);
         else if (knob == TG_TUNE_AMG_WEIGHT)
             *value = c->amg.weight;
         else

@@ -228,7 +228,7 @@ struct AmgLevel {
 struct Amg {
     int gen = 0;                             // bumped on every rebuild or knob change (captured PCG graphs key on it)
     int degree = 2;                          // Chebyshev degree per smoothing pass
-    bool degree_auto = true;                 // not set by the caller: large levels take one step (k_amg.hip: level_degree)
+    bool degree_auto = true;                 // not set by the caller: large levels take one step (amg_degree)
     int weight = 150;                        // coarse-grid correction weight, percent
     int reuse = 6;                           // further tangents of one Newton solve served by one numeric set-up
                                              // of the coarse levels (a 128^3 Newton step: 1.4x faster, fewer PCG
@@ -467,6 +467,9 @@ inline int pcg_split(const tg_ctx* c)
     if (c->spmv_xcd >= 0 || !pcg_small(c)) return 0;
     return c->nnd <= 64 * 256 ? 9 : c->nnd <= 64 * 640 ? 5 : 3;
 }
+// Chebyshev degree of the smoothing passes of a multigrid level of that many
+// dofs (k_amg.hip: level_degree, whose comment has the times)
+inline int amg_degree(const tg_ctx* c, long dofs) { return c->amg.degree_auto && dofs >= 3L << 17 ? 1 : c->amg.degree; }
 // segments of at most this many slices run their whole PCG in one
 // persistent workgroup of 1024 threads, one node each (0: none).  Default
 // 12 slices (768 nodes, an 8^3-element cube): there it halves a PCG
