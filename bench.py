@@ -138,6 +138,18 @@ def spmv_kernel_name(mt, fused, variant, pc=0):
     return f"k_fused_spmv<{mt}, {pc}, {x}, {u}, {y}>" if fused else f"k_seg_spmv<{mt}, {x}, {u}, {y}>"
 
 
+def untuned_product(mt, fused, nnd, precond="jacobi"):
+    """The PCG product of a single problem that no SpMV variant was set for,
+    where several waves share a row (pcg_split and pcg_share of the library);
+    None where a lane takes a row and the variant that the knob reads runs."""
+    if nnd <= 64 * 1536:
+        waves = 9 if nnd <= 64 * 256 else 5 if nnd <= 64 * 640 else 3
+        return f"k_split_spmv<{mt}, {waves}>" if fused and precond != "amg" else None
+    if not fused and nnd >= 1 << 17 and not (mt == "double" and nnd >= 3 << 18):
+        return f"k_share_spmv<{mt}>"
+    return None
+
+
 def spmv_operator_bytes(n, nnd, vbytes, symmetric):
     """Algorithmic HBM bytes of the operator part of one SpMV on the
     structured n^3 cube: (3n+1)^3 node-neighbour blocks, nnd of them
@@ -346,6 +358,7 @@ def bench_cube(a):
         s.set_tuning(api.TUNE_SPMV_XCD, a.spmv_xcd)
     if a.pcg_fused is not None:
         s.set_tuning(api.TUNE_PCG_FUSED, a.pcg_fused)
+    untuned = (a.spmv_xcd if a.spmv_xcd is not None else tuned_spmv.get("xcd", -1)) == -1
     tuned_spmv.update(xcd=s.tuning(api.TUNE_SPMV_XCD), fused=s.tuning(api.TUNE_PCG_FUSED))
     s.set_tuning(api.TUNE_PCG_GRAPH, a.pcg_graph)
     log(f"PCG: SpMV variant {tuned_spmv['xcd']}, fused direction {tuned_spmv['fused']} "
@@ -394,14 +407,17 @@ def bench_cube(a):
     nblocks = (n + 1 + 2 * n) ** 3  # (3n+1)^3 node-neighbour blocks of the structured cube
     vbytes = 8 if a.precision == "fp64" else 4
     variant = s.tuning(api.TUNE_SPMV_XCD)
-    symmetric = bool(variant & 4)
-    fused = s.tuning(api.TUNE_PCG_FUSED) == 1 and a.precond != "block"
+    # (block Jacobi's iteration is fused while its totals are folded)
+    fused = s.tuning(api.TUNE_PCG_FUSED) == 1 and (a.precond != "block" or m.nnd <= 64 * 2048)
+    mt = "double" if a.precision == "fp64" else "float"
+    shared = untuned_product(mt, fused, m.nnd, a.precond) if untuned else None
+    symmetric = shared is None and bool(variant & 4)
     # operator values + columns once; node vectors once: x and y (FP64); the
     # fused iteration reads p_old and z's sources (r and 1/diag for Jacobi, z
-    # for the multigrid) instead of x, and writes the new p besides y
-    node_vectors = (5 if a.precond == "jacobi" else 4) if fused else 2
-    kname = spmv_kernel_name("double" if a.precision == "fp64" else "float", fused, variant,
-                             2 if a.precond == "amg" else 0)
+    # for the multigrid and where rows are shared) instead of x, and writes
+    # the new p besides y
+    node_vectors = (5 if a.precond == "jacobi" and not shared else 4) if fused else 2
+    kname = shared or spmv_kernel_name(mt, fused, variant, 2 if a.precond == "amg" else 0)
     profiled = n == 128 and a.precision == "fp64" and a.precond == "jacobi"
     # algorithmic bytes of the product on the full (both triangles) block
     # operator: every block's values and column, the node vectors once
@@ -440,7 +456,8 @@ def bench_cube(a):
                                        "operator" if tuned["assembly"] == 1 else "msr+expansion"),
                    "stiffness_shape_elements_per_workgroup": (None if tuned.get("rows") else
                                                               api.STIFF_SHAPE_EPB[tuned["shape"]]),
-                   "stiffness_chunk": tuned["chunk"], "spmv_variant": tuned_spmv["xcd"], "pcg_fused": bool(fused),
+                   "stiffness_chunk": tuned["chunk"], "spmv_variant": "rows shared" if shared else tuned_spmv["xcd"],
+                   "pcg_fused": bool(fused),
                    "precision": a.precision, "preconditioner": a.precond},
         "value_is": "elements / (residual pass + stiffness pass device time), HIP events on the solver stream",
         "roofline": {"bound": "hbm", "achieved": spmv_gbs, "peak": HBM_PEAK / 1e9, "unit": "GB/s",

@@ -99,10 +99,11 @@ def tune_stiffness(solid: api.Solid, shapes=None, chunks=None, reps: int = 2, ru
                    "rows": {} if t_rows is None else {1: t_rows}}}
 
 
-def tune_spmv_xcd(solid: api.Solid, run_pcg, fused=(1, 0), reps: int = 2, variants=range(8)) -> dict:
+def tune_spmv_xcd(solid: api.Solid, run_pcg, fused=(1, 0), reps: int = 2, variants=(*range(8), -1)) -> dict:
     """Time the PCG iteration over the SpMV variants (hardware or
     XCD-contiguous row order, plain or branch-free unrolled inner loop, lower
-    blocks read directly or as their upper partners' transposes), with
+    blocks read directly or as their upper partners' transposes; -1: the
+    untuned choice, whose rows several waves share at most sizes), with
     the direction formed inside the SpMV (fused) and as its own pass; run_pcg()
     must run a short PCG (e.g. one Newton correction with a small iteration
     cap) from a fixed state.  The figure compared is device time per
