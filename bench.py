@@ -340,12 +340,13 @@ def bench_cube(a):
     from tahoe_amd import autotune
     t_tune = time.perf_counter()
     if a.stiff_chunk is not None or a.stiff_shape is not None or a.assembly is not None or not a.autotune:
-        s.set_tuning(api.TUNE_STIFF_CHUNK, -1 if a.stiff_chunk is None else a.stiff_chunk)
-        if a.stiff_shape is not None:
-            s.set_tuning(api.TUNE_STIFF_SHAPE, a.stiff_shape)
-        s.set_tuning(api.TUNE_NEWTON_ASSEMBLY, 0 if a.assembly is None else a.assembly)
+        # (each of these knobs selects the colour-ordered assembly)
+        for knob, v in ((api.TUNE_STIFF_CHUNK, a.stiff_chunk), (api.TUNE_STIFF_SHAPE, a.stiff_shape),
+                        (api.TUNE_NEWTON_ASSEMBLY, a.assembly)):
+            if v is not None:
+                s.set_tuning(knob, v)
         tuned = {"assembly": s.tuning(api.TUNE_NEWTON_ASSEMBLY), "shape": s.tuning(api.TUNE_STIFF_SHAPE),
-                 "chunk": s.tuning(api.TUNE_STIFF_CHUNK), "ms": {}}
+                 "chunk": s.tuning(api.TUNE_STIFF_CHUNK), "rows": s.tuning(api.TUNE_STIFF_ROWS) == 1, "ms": {}}
     else:
         tuned = autotune.tune_stiffness(s, reps=1, run_correction=short_pcg)
     log(f"Newton assembly {'by rows, else ' if tuned.get('rows') else ''}{tuned['assembly']} stiffness shape "
