@@ -315,7 +315,7 @@ int tg_calib_copy(int device, long bytes, int reps, double* ms);
 /* TG_TUNE_PCG_FUSED    1: the direction update is formed inside the SpMV
  *                      (one kernel less per PCG iteration, no separate
  *                      direction pass), in any SpMV variant (block Jacobi:
- *                      only while no segment has more than 4,096 slices of
+ *                      only while no segment has more than 2,048 slices of
  *                      64 nodes); 0: the direction in its own pass; -1
  *                      (default): 0 for a problem or batch of more than
  *                      98,304 nodes, else 1. */

@@ -478,8 +478,13 @@ inline int amg_degree(const tg_ctx* c, long dofs) { return c->amg.degree_auto &&
 constexpr int PCG_PERSIST_MAX = 16;
 constexpr int PCG_PERSIST_DEFAULT = 12;
 // a segment of at most this many slices has its reductions formed inside the
-// kernels that need them (k_pcg.hip: wave_total)
-constexpr int PCG_FOLD_SLICES = 4096;
+// kernels that need them (k_pcg.hip: wave_total): every wave adds all partials,
+// which grows with the square of the slices, against two kernels an iteration.
+// us an iteration, Jacobi, kernels of their own / inside: mixed 1,614 slices
+// 32.1 / 31.3, 1,943 36.0 / 34.7, 2,461 43.1 / 43.5, 2,945 48.5 / 50.3, 3,547
+// 57.6 / 62.2, 4,094 74.5 / 80.1; FP64 46.3 / 45.8, 56.9 / 54.9, 71.0 / 71.8,
+// 82.0 / 84.8, 97.0 / 104.0, 112.2 / 119.2.
+constexpr int PCG_FOLD_SLICES = 2048;
 inline int pcg_persist(const tg_ctx* c) { return c->pcg_persist >= 0 ? c->pcg_persist : PCG_PERSIST_DEFAULT; }
 
 // TG_SETUP_TRACE=1 prints host-side set-up phases to stderr, each timed
