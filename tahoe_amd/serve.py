@@ -127,15 +127,12 @@ def solve_request(req, precision, opts, device=0, log=None, precond=None, one_st
 
 class RVEServer:
     def __init__(self, precision=api.MIXED, workers=6, max_batch=32, budget_bytes=64 << 30, lin_rtol=None,
-                 device=0, keep_u=True, on_batch=None, log=None, reuse_contexts=True, linger=0.0):
+                 device=0, keep_u=True, on_batch=None, log=None, reuse_contexts=True, linger=0.003):
         self.precision = precision
-        # linger > 0: while another worker solves, a mini-batch that is not
-        # full waits up to `linger` seconds for requests of its kind; with no
-        # worker solving it starts at once.  Off by default: a window of 3 ms
-        # takes more from a request than the larger batches give back (edges
-        # 4-32, six workers, medians of six runs, off / 3 ms: 30 requests/s
-        # p50 7.3 / 7.9 ms, 100/s 11.0 / 13.0, 200/s 41.6 / 43.0, 280/s 97 /
-        # 94 with p99 323 / 269, a burst 360 / 351 solves/s).
+        # while another worker solves, a mini-batch that is not full waits up
+        # to `linger` seconds for requests of its kind: a request joined costs
+        # the batch little, on its own it costs a whole set-up and launch
+        # chain.  With no worker solving it starts at once.
         self.linger = linger
         self._solving = 0            # workers that solve (one that waits for requests is not among them)
         # each worker keeps one context per (formulation, size class,

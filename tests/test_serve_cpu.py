@@ -94,13 +94,3 @@ def test_full_batch_does_not_wait():
     assert time.perf_counter() - t < 0.5 * LINGER
     assert [r.rid for r in reqs] == [1, 2] and [r.rid for r in s._queue] == [3]
     assert size == sum(serve.footprint_bytes(r, s.precision) for r in reqs) == s._in_use
-
-
-def test_no_window_by_default():
-    s = serve.RVEServer()
-    s._solving = 3
-    s._queue.append(request(1, 10))
-    t = time.perf_counter()
-    with s._lock:
-        _, reqs, _ = s._take_batch()
-    assert [r.rid for r in reqs] == [1] and s.linger == 0 and time.perf_counter() - t < 0.5
