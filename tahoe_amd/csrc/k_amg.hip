@@ -505,7 +505,11 @@ static void level_rows(tg_ctx* c, int l, const double* x, const E& e, const doub
 // / 1 at the first coarse level too: 128^3 440 (86) / 379 (99) / 341 (109), 96^3
 // 214 / 180 / 170, 80^3 127 / 110 / 108, 56^3 50.8 / 46.7 / 47.8, 48^3 27.4 /
 // 26.8 / 27.5, 32^3 16.8 / 17.2 / 17.9.  So from 3 * 2^17 dofs of a level: 2^17
-// nodes of the fine one, 2^16 of a coarse one.
+// nodes of the fine one, 2^16 of a coarse one.  The rule holds in FP64 (64^3 63
+// and 71 ms with degree 2 everywhere, 128^3 380 and 451) and for nearly
+// incompressible problems, one solve to 1e-3: Q1P0 nu 0.499 52^3 FP64 35 and 50
+// ms, 64^3 mixed 331 and 383, nu 0.49 82^3 25 and 40; total-Lagrangian nu 0.49
+// 96^3 40 and 148.
 static int level_degree(const tg_ctx* c, int l)
 {
     const AmgLevel& A = *c->amg.lv[l];

@@ -173,7 +173,8 @@ struct Bsell {
     DBuf<int4> d_srange;                   // [2 nslices] (e0, e1, r0, r1)
     long lds_values = 0;
     DBuf<int> d_tpos;                      // [nblocks_padded] for a lower block (column < row): value
-                                           // index of its transpose partner, else -1
+                                           // index of its transpose partner; for an upper one
+                                           // -index - 2 of its lower partner; else -1
     DBuf<double> d_val;                    // [nblocks_padded * 9]
     DBuf<float> d_val32;                   // FP32 copy for the mixed-precision inner solve
     DBuf<int> d_oslot;                     // [nel][36][2] element block (a<=b) -> value index of

@@ -1,6 +1,7 @@
-// Host-side setup of the equation system: element colouring and the node graph the multigrid's aggregation reads (the
-// operator's structure itself is built on the device, k_graph.hip).  Runs
-// once per mesh (the reference does the same work in
+// Host-side setup of the equation system: the element colouring (of the
+// colour-ordered assembly) and the node graph the multigrid's aggregation
+// reads (the operator's structure itself is built on the device,
+// k_graph.hip).  Runs once per mesh (the reference does the same work in
 // FEManagerT::SetEquationSystem, tahoe/src/main/FEManagerT.cpp:2248-2313).
 #include <algorithm>
 #include <cstring>

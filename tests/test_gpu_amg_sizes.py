@@ -1,6 +1,6 @@
 """Multigrid-preconditioned solves at the sizes where the V-cycle's products
-change form (9, 3 or 1 waves a row; lower blocks through their partners from
-2^17 nodes): the solution of the Jacobi-preconditioned solve, in far fewer
+change form (9 or 3 waves a row; a coarse level's lower blocks through their
+partners from 2^16 nodes): the solution of the Jacobi-preconditioned solve, in far fewer
 iterations."""
 import numpy as np
 import pytest

@@ -41,7 +41,7 @@ def state(m):
     return 0.01 / max(m.shape or (4,)) * np.random.default_rng(8).standard_normal((m.nnd, 3)) + 0.02 * m.X
 
 
-# one element; fewer and more than the 4, 10 and 12 elements of a workgroup;
+# one element; fewer and more than the 7 and 10 elements of a workgroup;
 # rows past a half slice
 @pytest.mark.parametrize("n", [(1, 1, 1), (3, 2, 2), (5, 3, 4), (7, 7, 7)])
 @pytest.mark.parametrize("form,model,precision", [(0, SIMO, 0), (0, SIMO, 1), (0, STVENANT, 0), (0, STVENANT, 1),

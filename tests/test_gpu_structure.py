@@ -1,6 +1,6 @@
 """The equation-system structure built on the device (node graph, MSR
 pattern) for connectivity outside the structured meshes of the other tests:
-nodes shared by more than 8 elements take the sorted-insertion path of the
+nodes shared by more than 8 elements hold eight passes of candidates in the
 neighbour kernel, an isolated node has no neighbours, and a node shared by
 more than 64 elements is refused.  Only the structure is checked (the hub
 elements' geometry is arbitrary), bit-exactly against the oracle's
